@@ -56,6 +56,9 @@ struct DevTables {
     const double *va = nullptr;    // the field's own values: depth, or u
     const double *vb = nullptr;    // v
     const SCell *scells = nullptr; // combined records with a current on shared cells
+    // a gridded field's own cell records, built on first use without shared cells
+    const DCell *dcells = nullptr;
+    const UCell *ucells = nullptr;
     ~DevTables()
     {
         for (void *p : allocs) (void)hipFree(p);
@@ -149,7 +152,7 @@ struct mr_field {
 struct mr_batch {
     int device = 0;
     int bk = 0, ck = 0;
-    bool shared_cells = true;           // every scene's depth and current share cells
+    int records = REC_SHARED;           // REC_*, the one mode every scene can run on
     int64_t n_rays = 0, max_ray_steps = 0;
     std::unique_ptr<DevTables> mem;     // descriptors, ray -> scene map, queue head
     SceneDesc *scenes = nullptr;
@@ -750,22 +753,21 @@ bool shared_cells(const mr_field *b, const mr_field *c)
     return true;
 }
 
-// The fast region of each cell along one axis (SCell): the f32 targets p in
-// [lo, hi] lie in cell i for the depth's f32 index rule (T32[i] <= p <
-// T32[i+1]), for every f64 coordinate that rounds to p lie in cell i for the
-// current's f64 index rule (T64[i] <= x < T64[i+1]), and are strictly
-// between the cell's node coordinates a[i] and a[i+1] (no corner).  If
-// RN32(x) >= lo > ceil32(T64[i]) then x > T64[i]; if RN32(x) <= hi <
-// floor32(T64[i+1]) then x < T64[i+1] (rounding is monotone).  The three
-// intervals need not meet (on axes whose spacing varies, the index rules,
-// which use the first spacing, can map a cell's targets outside its nodes):
-// an empty interval is stored as (-inf, -inf), the one form of an empty
-// region that the device's region test (med3(p, lo, hi) - p) reads as
-// empty; lo > hi would read as [hi, lo].
-std::vector<float2> fast_bounds(const std::vector<float> &a32, const std::vector<double> &a64)
+// The fast region of each cell along one axis (SCell, DCell, UCell): the f32
+// targets p in [lo, hi] lie in cell i for the depth's f32 index rule (T32[i]
+// <= p < T32[i+1]; t32 null: no depth on this axis), for every f64 coordinate
+// that rounds to p lie in cell i for the current's f64 index rule (T64[i] <=
+// x < T64[i+1]; t64 null: no current), and are strictly between the cell's
+// node coordinates a[i] and a[i+1] (no corner).  If RN32(x) >= lo >
+// ceil32(T64[i]) then x > T64[i]; if RN32(x) <= hi < floor32(T64[i+1]) then
+// x < T64[i+1] (rounding is monotone).  The intervals need not meet (on axes
+// whose spacing varies, the index rules, which use the first spacing, can map
+// a cell's targets outside its nodes): an empty interval is stored as
+// (-inf, -inf), the one form of an empty region that the device's region
+// test (med3(p, lo, hi) - p) reads as empty; lo > hi would read as [hi, lo].
+std::vector<float2> fast_bounds(const std::vector<float> &a, const std::vector<float> *t32,
+                                const std::vector<double> *t64)
 {
-    const std::vector<float> t32 = thresholds32(a32);
-    const std::vector<double> t64 = thresholds64(a64);
     auto up = [](float f) { return std::nextafter(f, INFINITY); };
     auto down = [](float f) { return std::nextafter(f, -INFINITY); };
     auto ceil32 = [&](double d) {
@@ -776,10 +778,17 @@ std::vector<float2> fast_bounds(const std::vector<float> &a32, const std::vector
         float f = (float)d;
         return (double)f > d ? down(f) : f;
     };
-    std::vector<float2> b(a32.size() - 1);
-    for (size_t i = 0; i + 1 < a32.size(); i++) {
-        const float lo = std::max({t32[i], up(a32[i]), up(ceil32(t64[i]))});
-        const float hi = std::min({down(t32[i + 1]), down(a32[i + 1]), down(floor32(t64[i + 1]))});
+    std::vector<float2> b(a.size() - 1);
+    for (size_t i = 0; i + 1 < a.size(); i++) {
+        float lo = up(a[i]), hi = down(a[i + 1]);
+        if (t32) {
+            lo = std::max(lo, (*t32)[i]);
+            hi = std::min(hi, down((*t32)[i + 1]));
+        }
+        if (t64) {
+            lo = std::max(lo, up(ceil32((*t64)[i])));
+            hi = std::min(hi, down(floor32((*t64)[i + 1])));
+        }
         b[i] = lo <= hi ? make_float2(lo, hi) : make_float2(-INFINITY, -INFINITY);
     }
     return b;
@@ -804,8 +813,12 @@ int shared_tables(const mr_field *cb, const mr_field *cc, int tl, const SCell **
         return MR_OK;
     }
     std::unique_ptr<DevTables> t(new DevTables);
-    std::vector<double> cx(cc->xd), cy(cc->yd);
-    std::vector<float2> fx = fast_bounds(b->xf, cx), fy = fast_bounds(b->yf, cy);
+    auto bounds = [](const std::vector<float> &a32, const std::vector<double> &a64) {
+        const std::vector<float> t32 = thresholds32(a32);
+        const std::vector<double> t64 = thresholds64(a64);
+        return fast_bounds(a32, &t32, &t64);
+    };
+    std::vector<float2> fx = bounds(b->xf, cc->xd), fy = bounds(b->yf, cc->yd);
     float2 *dfx, *dfy;
     if ((rc = dev_upload(*t, fx.data(), fx.size(), &dfx)) ||
         (rc = dev_upload(*t, fy.data(), fy.size(), &dfy)))
@@ -843,13 +856,93 @@ int shared_tables(const mr_field *cb, const mr_field *cc, int tl, const SCell **
     return MR_OK;
 }
 
-// shared cells whose combined records the kernels can index with 32-bit
-// byte offsets (grids up to about 5790 x 5790 cells)
-bool use_shared(const mr_field *b, const mr_field *c, int tl)
+// A gridded field's own cell records (DCell, UCell) on the current device,
+// built on first use and kept with its tables t.
+int own_records(const mr_field *cf, int tl, const DevTables *ct)
 {
-    return shared_cells(b, c) &&
-           (tiles_along(b->nx, tl) * tiles_along(b->ny, tl) << (2 * tl)) * (int64_t)sizeof(SCell) <
+    mr_field *f = const_cast<mr_field *>(cf);
+    DevTables &t = *const_cast<DevTables *>(ct);
+    const bool bathy = f->kind == MR_BATHY_GRID;
+    if (!bathy && f->kind != MR_CURRENT_GRID) return MR_OK;
+    std::lock_guard<std::mutex> lk(f->mu);
+    if (t.dcells || t.ucells) return MR_OK;
+    auto axis32 = [](const std::vector<double> &a) {
+        std::vector<float> r(a.size());
+        for (size_t i = 0; i < a.size(); i++) r[i] = (float)a[i];    // cartesian_current.rs:375-378
+        return r;
+    };
+    auto bounds = [&](const std::vector<float> &a32, const std::vector<double> &a64) {
+        std::vector<float> t32;
+        std::vector<double> t64;
+        if (bathy) t32 = thresholds32(a32);
+        else t64 = thresholds64(a64);
+        return fast_bounds(a32, bathy ? &t32 : nullptr, bathy ? nullptr : &t64);
+    };
+    const std::vector<float> x = bathy ? f->xf : axis32(f->xd), y = bathy ? f->yf : axis32(f->yd);
+    const std::vector<float2> xp = axis_pairs(x), yp = axis_pairs(y);
+    const std::vector<float2> fx = bounds(x, f->xd), fy = bounds(y, f->yd);
+    // (the axis arrays are needed by the build alone)
+    DevTables tmp;
+    float2 *dxp, *dyp, *dfx, *dfy;
+    int rc = dev_upload(tmp, xp.data(), xp.size(), &dxp);
+    if (!rc) rc = dev_upload(tmp, yp.data(), yp.size(), &dyp);
+    if (!rc) rc = dev_upload(tmp, fx.data(), fx.size(), &dfx);
+    if (!rc) rc = dev_upload(tmp, fy.data(), fy.size(), &dfy);
+    if (rc) return rc;
+    const int64_t ntx = tiles_along(f->nx, tl), nty = tiles_along(f->ny, tl);
+    const size_t n = (size_t)((ntx * nty) << (2 * tl));
+    RecBuildArgs a;
+    a.nx = f->nx; a.ny = f->ny;
+    a.xp = dxp; a.yp = dyp; a.fx = dfx; a.fy = dfy;
+    a.oob_from = first_oob_cell(f->nx, f->ny, (int64_t)f->a.size());
+    if (!bathy) a.oob_from = std::min(a.oob_from, first_oob_cell(f->nx, f->ny, (int64_t)f->b.size()));
+    a.ntx = (int)(ntx << 4 | tl);
+    DCell *dc = nullptr;
+    UCell *uc = nullptr;
+    if (bathy) {
+        if ((rc = dev_alloc(t, n, &dc))) return rc;
+        MR_HIP_TRY(launch_build_depth_rec(a, t.bp.cells, dc, 0));
+    } else {
+        if ((rc = dev_alloc(t, n, &uc))) return rc;
+        MR_HIP_TRY(launch_build_current_rec(a, t.cp.cells, t.cp.mtab, uc, 0));
+    }
+    MR_HIP_TRY(hipDeviceSynchronize());
+    t.dcells = dc;
+    t.ucells = uc;
+    return MR_OK;
+}
+
+// Which cell records a pair of fields runs on (REC_*): the combined ones
+// where they share cells, each gridded field's own otherwise, provided the
+// kernels can index them with 32-bit byte offsets: grids up to about
+// 5790 x 5790 cells for the 128-byte records (SCell, UCell), 8190 x 8190 for
+// DCell.  A larger grid's records would need a 64-bit address per load, about
+// six more vector instructions in every step; such a pair runs on the plain
+// records (REC_NONE) instead.
+int record_mode(const mr_field *b, const mr_field *c, int tl)
+{
+    auto fits = [tl](const mr_field *f, size_t rec) {
+        return (tiles_along(f->nx, tl) * tiles_along(f->ny, tl) << (2 * tl)) * (int64_t)rec <
                (int64_t(1) << 32);
+    };
+    if (shared_cells(b, c) && fits(b, sizeof(SCell))) return REC_SHARED;
+    if (b->kind == MR_BATHY_GRID && !fits(b, sizeof(DCell))) return REC_NONE;
+    if (c->kind == MR_CURRENT_GRID && !fits(c, sizeof(UCell))) return REC_NONE;
+    return REC_OWN;
+}
+
+// the records of a mode, built on first use (bt, ct: the fields' tables)
+int record_tables(const mr_field *b, const mr_field *c, int tl, int mode, const DevTables *bt,
+                  const DevTables *ct, RecPtrs *out)
+{
+    *out = RecPtrs{nullptr, nullptr, nullptr};
+    if (mode == REC_NONE) return MR_OK;
+    if (mode == REC_SHARED) return shared_tables(b, c, tl, &out->scells);
+    int rc = own_records(b, tl, bt);
+    if (!rc) rc = own_records(c, tl, ct);
+    out->dcells = bt->dcells;
+    out->ucells = ct->ucells;
+    return rc;
 }
 
 // the trace itself, all pointers device pointers, enqueued on stream
@@ -885,10 +978,8 @@ int trace_device(const mr_field *bathy, const mr_field *current, int64_t n_rays,
     a.len_out = len_out;
     a.end_out = end_out;
     a.solout = o.solout;
-    a.shared_cells = use_shared(bathy, current, o.record_tile) ? 1 : 0;
-    a.scells = nullptr;
-    if (a.shared_cells && (rc = shared_tables(bathy, current, o.record_tile, &a.scells)))
-        return rc;
+    a.records = record_mode(bathy, current, o.record_tile);
+    if ((rc = record_tables(bathy, current, o.record_tile, a.records, bt, ct, &a.rec))) return rc;
     const int block = o.block_size ? o.block_size : tuned_block(n_rays);
     if ((n_rays + block - 1) / block >= (int64_t)INT32_MAX)
         return fail(MR_ERR_UNSUPPORTED, "too many rays for one launch");
@@ -1398,7 +1489,12 @@ int mr_batch_create(int32_t n_scenes, const mr_scene *scenes, const mr_options *
         if (i == 0) { b->bk = bk; b->ck = ck; }
         else if (bk != b->bk || ck != b->ck)
             return fail(MR_ERR_INVALID_ARGUMENT, "scenes of one batch must share field kinds");
-        b->shared_cells = b->shared_cells && use_shared(sc.bathy, sc.current, o.record_tile);
+        // one mode for every scene: combined records where all share cells,
+        // plain records where any scene needs them, the fields' own otherwise
+        const int mode = record_mode(sc.bathy, sc.current, o.record_tile);
+        if (i == 0 || b->records == mode) b->records = mode;
+        else if (mode == REC_NONE || b->records == REC_NONE) b->records = REC_NONE;
+        else b->records = REC_OWN;
         if (sc.n_rays < 0) return fail(MR_ERR_INVALID_ARGUMENT, "negative ray count");
         if (sc.n_rays > 0 && (!sc.x0 || !sc.y0 || !sc.kx0 || !sc.ky0 || !sc.len_out || !sc.end_out))
             return fail(MR_ERR_INVALID_ARGUMENT, "null scene arrays");
@@ -1415,17 +1511,19 @@ int mr_batch_create(int32_t n_scenes, const mr_scene *scenes, const mr_options *
         d.ray0 = b->n_rays;
         d.x0 = sc.x0; d.y0 = sc.y0; d.kx0 = sc.kx0; d.ky0 = sc.ky0;
         d.len_out = sc.len_out; d.end_out = sc.end_out;
-        d.scells = nullptr;
         b->n_rays += sc.n_rays;
         b->max_ray_steps += sc.n_rays * n;
         ray_scene.insert(ray_scene.end(), (size_t)sc.n_rays, i);
     }
     if (b->n_rays >= (int64_t(1) << 31)) return fail(MR_ERR_UNSUPPORTED, "too many rays");
-    if (b->shared_cells)
-        for (int32_t i = 0; i < n_scenes; i++)
-            if ((rc = shared_tables(scenes[i].bathy, scenes[i].current, o.record_tile,
-                                    &desc[(size_t)i].scells)))
-                return rc;
+    for (int32_t i = 0; i < n_scenes; i++) {
+        const mr_field *sb = scenes[i].bathy, *sc = scenes[i].current;
+        const DevTables *bt, *ct;
+        if ((rc = field_tables(sb, o.record_tile, &bt)) ||
+            (rc = field_tables(sc, o.record_tile, &ct)) ||
+            (rc = record_tables(sb, sc, o.record_tile, b->records, bt, ct, &desc[(size_t)i].rec)))
+            return rc;
+    }
     if ((rc = dev_upload(*b->mem, desc.data(), desc.size(), &b->scenes)) ||
         (rc = dev_upload(*b->mem, ray_scene.data(), ray_scene.size(), &b->ray_scene)) ||
         (rc = dev_alloc(*b->mem, 1, &b->next)))
@@ -1464,7 +1562,7 @@ int mr_batch_run(mr_batch *b, const mr_options *opt)
     a.n_rays = b->n_rays;
     a.next = b->next;
     a.solout = o.solout;
-    a.shared_cells = b->shared_cells ? 1 : 0;
+    a.records = b->records;
     MR_HIP_TRY(launch_clear_counter(b->next, stream));
     MR_HIP_TRY(launch_batch(a, b->bk, b->ck, o.math, block, blocks, stream));
     return MR_OK;

@@ -77,6 +77,33 @@ struct SCell {                    // 128 B
     double ux, uy, vx, vy;        // current slopes (f64), cartesian_current.rs:515-536
 };
 
+// One cell of a gridded depth on its own, and of a gridded current on its
+// own: SCell's pieces of that field, with a fast region that stands for that
+// field's index rule alone.  Used where the two fields do not share cells or
+// only one of them is gridded.
+struct DCell {                    // 64 B
+    float lo_x, hi_x, lo_y, hi_y;
+    float x0, y0, m01, m10;
+    float a00, a10, a01, a11;
+    double hx, hy;
+};
+
+struct alignas(128) UCell {       // 96 B used, one 128-byte line per record
+    float lo_x, hi_x, lo_y, hi_y;
+    float x0, y0, m01, m10;
+    float ua00, ua10, ua01, ua11;
+    float va00, va10, va01, va11;
+    double ux, uy, vx, vy;
+};
+
+// The records a trace reads: scells for shared cells, otherwise dcells and
+// ucells for whichever field is gridded.
+struct RecPtrs {
+    const SCell *scells;
+    const DCell *dcells;
+    const UCell *ucells;
+};
+
 struct BathyView {
     int kind;
     float h;                              // ConstantDepth
@@ -652,13 +679,17 @@ __device__ __forceinline__ bool current_fast(const CurrentSlot &cs, double x, do
 }
 
 // ---------------------------------------------------------------------------
-// Shared-cell records (SCell) in registers: eight 16-byte pieces, held as
-// f64 pairs so that copies between slots move 64 bits per instruction.
-
-struct SharedSlot {
-    // a slot never loaded has the empty region (four -inf bounds)
-    mr_d2 q[8] = {{MR_EMPTY_REGION, MR_EMPTY_REGION}, {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0},
-                  {0.0, 0.0},                         {0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}};
+// Cell records (SCell, DCell, UCell) in registers, as 16-byte pieces held as
+// f64 pairs.  A record starts with its fast region (piece 0) and its origin
+// and change of basis (piece 1).  SH: one SCell serves both fields;
+// otherwise each gridded field has a record of its own, and an analytic
+// field none.
+template <int BK, int CK, bool SH>
+struct RecSlot {
+    static constexpr int ND = SH ? 8 : BK == BK_GRID ? 4 : 0;
+    static constexpr int NC = !SH && CK == CK_GRID ? 6 : 0;
+    mr_d2 d[ND ? ND : 1];              // the shared record, or the depth's
+    mr_d2 c[NC ? NC : 1];              // the current's
 };
 
 // the four f32 values of a 16-byte record piece.  The whole piece is bit-cast
@@ -669,52 +700,67 @@ __device__ __forceinline__ mr_f4 f4of(mr_d2 d)
     return __builtin_bit_cast(mr_f4, d);
 }
 
-__device__ __forceinline__ void shared_load(const SCell *cells, SharedSlot &s, uint32_t cell)
+template <int N, class Rec>
+__device__ __forceinline__ void rec_load(const Rec *cells, mr_d2 (&q)[N], uint32_t cell)
 {
-    const MR_GLOBAL mr_d2 *p = (const MR_GLOBAL mr_d2 *)((const MR_GLOBAL char *)cells + cell * 128u);
+    static_assert(N * 16 <= (int)sizeof(Rec), "pieces of one record");
+    const MR_GLOBAL mr_d2 *p =
+        (const MR_GLOBAL mr_d2 *)((const MR_GLOBAL char *)cells + cell * (uint32_t)sizeof(Rec));
 #pragma unroll
-    for (int k = 0; k < 8; ++k) s.q[k] = p[k];
+    for (int k = 0; k < N; ++k) q[k] = p[k];
 }
 
-// (px, py) in the slot's fast region; a NaN target is in none
-__device__ __forceinline__ bool shared_in_region(const SharedSlot &s, float px, float py)
+// How far (px, py) lies outside a record's fast region: zero exactly when
+// it is in the region.  lo <= p <= hi exactly when med3(p, lo, hi) - p is
+// zero (med3 returns one of its operands, and with f32 denormals kept a
+// difference of two finite floats is zero only when they are equal), so a
+// sum of the axes' (and the fields') distances tests all of them with one
+// compare, in vector ALU operations.  A NaN or infinite p gives NaN or
+// infinity, so it is in no region; the empty region, lo = hi = -inf, holds
+// no target.
+__device__ __forceinline__ float off_region(mr_d2 piece0, float px, float py)
 {
-    // lo <= p <= hi exactly when med3(p, lo, hi) - p is zero (med3 returns
-    // one of its operands, and with f32 denormals kept a difference of two
-    // finite floats is zero only when they are equal); the two axes'
-    // differences are tested at once, in vector ALU operations with one mask
-    // at the end.  A NaN or infinite p makes a difference NaN or infinite, so
-    // it is in no region; the empty region, lo = hi = -inf, holds no target.
-    const mr_f4 b = f4of(s.q[0]);              // (lo_x, hi_x, lo_y, hi_y)
+    const mr_f4 b = f4of(piece0);              // (lo_x, hi_x, lo_y, hi_y)
     const float dx = __builtin_amdgcn_fmed3f(px, b.x, b.y) - px;
     const float dy = __builtin_amdgcn_fmed3f(py, b.z, b.w) - py;
-    return __builtin_fabsf(dx) + __builtin_fabsf(dy) == 0.0f;
+    return __builtin_fabsf(dx) + __builtin_fabsf(dy);
 }
 
-// Both fields at (x, y) from the slot's record, for a target in its fast
-// region: the operations bathy_query and current_query take there
-// (interpolator.rs:39-84 with u = m01 tty, w = m10 ttx; the u and v pieces
-// at the same (u, w)), and slow set where the target is outside the region.
-__device__ __forceinline__ void shared_fast(const SharedSlot &s, double x, double y, double &h,
-                                            double &hx, double &hy, double &u, double &v,
-                                            double &ux, double &uy, double &vx, double &vy,
-                                            bool &slow)
+// The values of the gridded fields at (x, y) from the slot's records, for a
+// target in their fast regions: the operations bathy_query and current_query
+// take there (interpolator.rs:39-84 with u = m01 tty, w = m10 ttx).  Returns
+// how far the target is from the regions (0: inside).
+template <int BK, int CK, bool SH>
+__device__ __forceinline__ float rec_fast(const RecSlot<BK, CK, SH> &s, double x, double y,
+                                          double &h, double &hx, double &hy, double &u, double &v,
+                                          double &ux, double &uy, double &vx, double &vy)
 {
     const float px = (float)x, py = (float)y;
-    slow = !shared_in_region(s, px, py);
-    const mr_f4 om = f4of(s.q[1]);             // (x0, y0, m01, m10)
-    const float tx = px - om.x, ty = py - om.y;
-    const float uu = om.z * ty, ww = om.w * tx;
-    const mr_f4 d = f4of(s.q[2]), uc = f4of(s.q[4]), vc = f4of(s.q[5]);
-    const float hv = bilin_eval(d.x, d.y, d.z, d.w, uu, ww);
-    const float uf = bilin_eval(uc.x, uc.y, uc.z, uc.w, uu, ww);
-    const float vf = bilin_eval(vc.x, vc.y, vc.z, vc.w, uu, ww);
-    h = (double)hv;
-    hx = s.q[3].x;
-    hy = s.q[3].y;
-    u = (double)uf;
-    v = (double)vf;
-    ux = s.q[6].x; uy = s.q[6].y; vx = s.q[7].x; vy = s.q[7].y;
+    float off = 0.0f;
+    if constexpr (BK == BK_GRID) {
+        off = off_region(s.d[0], px, py);
+        const mr_f4 om = f4of(s.d[1]), d = f4of(s.d[2]);   // (x0, y0, m01, m10)
+        const float uu = om.z * (py - om.y), ww = om.w * (px - om.x);
+        h = (double)bilin_eval(d.x, d.y, d.z, d.w, uu, ww);
+        hx = s.d[3].x;
+        hy = s.d[3].y;
+        if constexpr (SH) {
+            const mr_f4 uc = f4of(s.d[4]), vc = f4of(s.d[5]);
+            u = (double)bilin_eval(uc.x, uc.y, uc.z, uc.w, uu, ww);
+            v = (double)bilin_eval(vc.x, vc.y, vc.z, vc.w, uu, ww);
+            ux = s.d[6].x; uy = s.d[6].y; vx = s.d[7].x; vy = s.d[7].y;
+        }
+    }
+    if constexpr (!SH && CK == CK_GRID) {
+        const float offc = off_region(s.c[0], px, py);
+        off = BK == BK_GRID ? off + offc : offc;
+        const mr_f4 om = f4of(s.c[1]), uc = f4of(s.c[2]), vc = f4of(s.c[3]);
+        const float uu = om.z * (py - om.y), ww = om.w * (px - om.x);
+        u = (double)bilin_eval(uc.x, uc.y, uc.z, uc.w, uu, ww);
+        v = (double)bilin_eval(vc.x, vc.y, vc.z, vc.w, uu, ww);
+        ux = s.c[4].x; uy = s.c[4].y; vx = s.c[5].x; vy = s.c[5].y;
+    }
+    return off;
 }
 
 // Whether any lane of the wave has c, as a wave-uniform value the compiler
@@ -731,29 +777,35 @@ __device__ __forceinline__ bool wave_any(bool c)
     return m != 0;
 }
 
-// WaveRayPath::system for gridded depth and current on shared cells: every
-// lane evaluates from the record in hand; lanes outside its fast region
-// evaluate again through the full queries (bathy_query, current_query),
-// which find and load their cells' records and handle nodes and errors.
-template <int MATH>
-__device__ __forceinline__ void rhs_shared(const BathyView &B, const BathyPtrs &BP,
-                                           const CurrentView &C, const CurrentPtrs &CP,
-                                           const SharedSlot &ss, const FastConsts &K, double x,
-                                           double y, double kx, double ky, double &dx,
-                                           double &dy, double &dkx, double &dky)
+// WaveRayPath::system (wave_ray_path.rs:220-234) around odes (:118-150) with
+// the cell records in hand: every lane evaluates from them in one block of
+// straight-line code; lanes outside a record's fast region evaluate again
+// through the full queries (bathy_query, current_query), which find and load
+// their cells and handle nodes and errors.  An analytic field is evaluated
+// in place.
+template <int BK, int CK, bool SH, int MATH>
+__device__ __forceinline__ void rhs_rec(const BathyView &B, const BathyPtrs &BP,
+                                        const CurrentView &C, const CurrentPtrs &CP,
+                                        const RecSlot<BK, CK, SH> &ss, const FastConsts &K,
+                                        double x, double y, double kx, double ky, double &dx,
+                                        double &dy, double &dkx, double &dky)
 {
     double h, hx, hy, u, v, ux, uy, vx, vy;
-    bool slow;
-    shared_fast(ss, x, y, h, hx, hy, u, v, ux, uy, vx, vy, slow);
+    BathySlot bs;
+    CurrentSlot cs;
+    const float off = rec_fast<BK, CK, SH>(ss, x, y, h, hx, hy, u, v, ux, uy, vx, vy);
+    if (BK != BK_GRID) h = bathy_query<BK>(B, BP, bs, x, y, hx, hy);
+    if (CK != CK_GRID) current_query<CK>(C, CP, cs, x, y, u, v, ux, uy, vx, vy);
     odes<MATH>(K, h, hx, hy, true, u, v, ux, uy, vx, vy, kx, ky, dx, dy, dkx, dky);
-    if (__builtin_expect(wave_any(slow), 0)) {
-        __asm__ volatile("");
-        if (slow) {
-            BathySlot bs;
-            CurrentSlot cs;
-            const double h2 = bathy_query<BK_GRID>(B, BP, bs, x, y, hx, hy);
-            const bool okc = current_query<CK_GRID>(C, CP, cs, x, y, u, v, ux, uy, vx, vy);
-            odes<MATH>(K, h2, hx, hy, okc, u, v, ux, uy, vx, vy, kx, ky, dx, dy, dkx, dky);
+    if (BK == BK_GRID || CK == CK_GRID) {
+        const bool slow = !(off == 0.0f);
+        if (__builtin_expect(wave_any(slow), 0)) {
+            __asm__ volatile("");
+            if (slow) {
+                const double h2 = bathy_query<BK>(B, BP, bs, x, y, hx, hy);
+                const bool okc = current_query<CK>(C, CP, cs, x, y, u, v, ux, uy, vx, vy);
+                odes<MATH>(K, h2, hx, hy, okc, u, v, ux, uy, vx, vy, kx, ky, dx, dy, dkx, dky);
+            }
         }
     }
 }

@@ -5,6 +5,12 @@
 
 namespace mr {
 
+// Which cell records a trace or batch runs on: one combined record per cell
+// for a gridded depth and current on the same cells; each gridded field's
+// own (analytic fields have none); or none, for grids whose records the
+// kernels could not index with 32-bit byte offsets.
+enum RecMode : int { REC_NONE = 0, REC_SHARED = 1, REC_OWN = 2 };
+
 // The numeric field views live in device memory and are copied into
 // per-lane registers at kernel start (see load_view); the field pointers
 // travel as kernel arguments.
@@ -22,8 +28,8 @@ struct TraceArgs {
     int32_t *len_out;                  // may be null
     double *end_out;                   // 4 per ray, may be null
     int solout;                        // 0 state, 1 next derivative
-    int shared_cells;                  // gridded depth and current on one set of cells
-    const SCell *scells;               // their combined records (with shared_cells)
+    int records;                       // REC_*
+    RecPtrs rec;                       // the cell records it names
 };
 
 // One scene of a batched trace, in device memory.
@@ -37,7 +43,7 @@ struct SceneDesc {
     const double *x0, *y0, *kx0, *ky0; // the scene's initial conditions
     int32_t *len_out;                  // the scene's outputs
     double *end_out;
-    const SCell *scells;               // combined records (batches with shared_cells)
+    RecPtrs rec;                       // the scene's cell records
 };
 
 // A persistent batched trace: rays of every scene taken from one queue.
@@ -47,7 +53,7 @@ struct BatchArgs {
     int64_t n_rays;                    // over all scenes
     unsigned long long *next;          // queue head, cleared before the launch
     int solout;
-    int shared_cells;                  // as in TraceArgs, for every scene
+    int records;                       // REC_*, for every scene
 };
 
 struct RhsArgs {
@@ -81,6 +87,15 @@ struct SharedBuildArgs {
     double cxspace, cyspace;           // x[1] - x[0] of the f64 axes (current slopes)
     int ntx;                           // as in BathyBuildArgs
     SCell *cells;
+};
+
+// a field's own records (DCell, UCell), from its plain ones
+struct RecBuildArgs {
+    int64_t nx, ny;
+    const float2 *xp, *yp;             // the f32 axis pairs (a[i], a[i+1])
+    const float2 *fx, *fy;             // per axis cell: the fast region's (lo, hi)
+    int64_t oob_from;                  // cells from here on have a corner past some array
+    int ntx;                           // as in BathyBuildArgs
 };
 
 struct CurrentBuildArgs {
@@ -156,6 +171,10 @@ hipError_t launch_batch(const BatchArgs &a, int bk, int ck, int math, int block,
 hipError_t launch_clear_counter(unsigned long long *p, hipStream_t stream);
 hipError_t launch_build_bathy(const BathyBuildArgs &a, hipStream_t stream);
 hipError_t launch_build_current(const CurrentBuildArgs &a, hipStream_t stream);
+hipError_t launch_build_depth_rec(const RecBuildArgs &a, const BCell *plain, DCell *cells,
+                                  hipStream_t stream);
+hipError_t launch_build_current_rec(const RecBuildArgs &a, const CCell *plain, const float2 *mtab,
+                                    UCell *cells, hipStream_t stream);
 hipError_t launch_build_shared(const SharedBuildArgs &a, hipStream_t stream);
 hipError_t launch_trace64(const Trace64Args &a, int bk, int ck, int math, int block,
                           hipStream_t stream);

@@ -24,7 +24,9 @@ namespace mr {
 //   y <- y + (((k1 + k2 2) + k3 2) + k4) (dt/6)
 // with the stop test of WaveRayPath::solout (wave_ray_path.rs:236-246).
 //
-// Stages 1 and 3 start the loads of the cell records that the following
+// rk4_step runs on the plain records (BCell, CCell), for the grids whose
+// cell records rk4_step_rec cannot index (record_mode in mr_capi.cpp).
+// Stages 1 and 3 start the loads of the plain records that the following
 // stages will most likely use (their points guessed from the latest
 // derivative) when those are not the cells already held, so a record is in
 // registers one evaluation after it was asked for and a ray crossing into a
@@ -99,18 +101,17 @@ __device__ __forceinline__ void rk4_step(const BathyView &B, const BathyPtrs &BP
     o[2] = kx + akx * sixth; o[3] = ky + aky * sixth;
 }
 
-// rk4_step for gridded depth and current on shared cells: one combined
-// record (SCell) per cell serves both fields, from two slots with fixed
-// roles.  In the stage loop below (st = 0..3), sa serves st 0 and st 3 (the
-// step's start y and y + k3 dt, nearly the next step's start), sb serves
-// st 1 and st 2 (y + k1 dt/2 and y + k2 dt/2).  Each slot is refilled while
-// the other one serves, two evaluations before its next use: sa at st 1 for
-// the point guessed at x + k1 dt, sb at st 3 for the next step's pair,
-// guessed at x + k3 (3 dt / 2).  A lane loads only when the guess lies
-// outside the fast region of the record its slot holds, and otherwise keeps
-// that record, the right one; so no slot is ever copied.  A guess is only a
-// guess: rhs_shared tests the region of the record it uses, and lanes
-// outside it take the full queries.  g1, g3: dt and 3 dt / 2 in f32.
+// rk4_step on cell records (RecSlot): two slots with fixed roles.  In the
+// stage loop below (st = 0..3), sa serves st 0 and st 3 (the step's start y
+// and y + k3 dt, nearly the next step's start), sb serves st 1 and st 2
+// (y + k1 dt/2 and y + k2 dt/2).  Each slot is refilled while the other one
+// serves, two evaluations before its next use: sa at st 1 for the point
+// guessed at x + k1 dt, sb at st 3 for the next step's pair, guessed at
+// x + k3 (3 dt / 2).  A lane loads a record only when the guess lies outside
+// the fast region of the one its slot holds, and otherwise keeps that
+// record, the right one; so no slot is ever copied.  A guess is only a
+// guess: rhs_rec tests the regions of the records it uses, and lanes
+// outside them take the full queries.  g1, g3: dt and 3 dt / 2 in f32.
 //
 // Before each refill the step waits for the vector memory operations issued
 // up to then but the last NST (the caller's row stores of the step before,
@@ -122,15 +123,57 @@ __device__ __forceinline__ void rk4_step(const BathyView &B, const BathyPtrs &BP
 // DY: dt and dt/2 are powers of two, so k * hs is exact (for every k whose
 // product is not subnormal) and the stage state y + k * hs of Rk4::step is
 // one rounding: fma(k, hs, y) gives it bitwise in one instruction.
-template <int MATH, bool DY, int NST, class OnStop>
-__device__ __forceinline__ void rk4_step_shared(const BathyView &B, const BathyPtrs &BP,
-                                                const CurrentView &C, const CurrentPtrs &CP,
-                                                const SCell *cells, SharedSlot &sa,
-                                                SharedSlot &sb, const FastConsts &K, double &px,
-                                                double &py, double dt, double half,
-                                                double sixth, float g1, float g3, int solout,
-                                                double x, double y, double kx, double ky,
-                                                double o[4], bool &stop_before, OnStop &&on_stop)
+//
+// What bounds it: one wave's instruction issue (a wave holds a SIMD alone up
+// to 65,536 rays, and a dependent f64 operation issues every 4 cycles, so
+// every instruction of the step counts and latency hidden by another wave
+// does not exist).  On own records it replaced rk4_step, whose slots are
+// copied at every other stage and whose reloads the compiler waits for at
+// once: 30,011 rays x 2000 steps of 0.7 s on a 1201 x 907 depth and a 444 x
+// 335 current with trajectories 3.60 -> 2.65 ms, 20,000 rays x 1500 steps on
+// a 1024 x 768 depth under a constant current 1.90 -> 1.44 ms.
+
+// The refill of one slot for the point (gx, gy).  The records' offsets are
+// formed before the tests, in every step: some lane of the wave refills in
+// most steps anyway, and these vector operations then stand between a test's
+// compare and the scalar EXEC update that reads it, which otherwise waits
+// for the compare's result (the empty asm keeps them out of the conditional
+// blocks).
+template <int BK, int CK, bool SH>
+__device__ __forceinline__ void rec_refill(const BathyView &B, const CurrentView &C,
+                                           const RecPtrs &R, RecSlot<BK, CK, SH> &s, float gx,
+                                           float gy)
+{
+    uint32_t bcell = 0, ccell = 0;
+    if (BK == BK_GRID) {
+        bcell = tiled_cell(guess_cell(gx, B.ax0, B.pinv_sx, B.pmax_x),
+                           guess_cell(gy, B.ay0, B.pinv_sy, B.pmax_y), B.ntx);
+        __asm__ volatile("" : "+v"(bcell));
+    }
+    if (!SH && CK == CK_GRID) {
+        ccell = tiled_cell(guess_cell(gx, C.px0, C.pinv_sx, C.pmax_x),
+                           guess_cell(gy, C.py0, C.pinv_sy, C.pmax_y), C.ntx);
+        __asm__ volatile("" : "+v"(ccell));
+    }
+    if constexpr (SH) {
+        if (!(off_region(s.d[0], gx, gy) == 0.0f)) rec_load(R.scells, s.d, bcell);
+    } else {
+        if constexpr (BK == BK_GRID)
+            if (!(off_region(s.d[0], gx, gy) == 0.0f)) rec_load(R.dcells, s.d, bcell);
+        if constexpr (CK == CK_GRID)
+            if (!(off_region(s.c[0], gx, gy) == 0.0f)) rec_load(R.ucells, s.c, ccell);
+    }
+}
+
+template <int BK, int CK, bool SH, int MATH, bool DY, int NST, class OnStop>
+__device__ __forceinline__ void rk4_step_rec(const BathyView &B, const BathyPtrs &BP,
+                                             const CurrentView &C, const CurrentPtrs &CP,
+                                             const RecPtrs &R, RecSlot<BK, CK, SH> &sa,
+                                             RecSlot<BK, CK, SH> &sb, const FastConsts &K,
+                                             double &px, double &py, double dt, double half,
+                                             double sixth, float g1, float g3, int solout,
+                                             double x, double y, double kx, double ky,
+                                             double o[4], bool &stop_before, OnStop &&on_stop)
 {
     double sx = x, sy = y, skx = kx, sky = ky;   // stage state
     double ax = 0.0, ay = 0.0, akx = 0.0, aky = 0.0;
@@ -138,28 +181,18 @@ __device__ __forceinline__ void rk4_step_shared(const BathyView &B, const BathyP
 #pragma unroll
     for (int st = 0; st < 4; ++st) {
         const double hs = st < 2 ? half : dt;
-        if (st == 1 || st == 3) {
+        if ((BK == BK_GRID || CK == CK_GRID) && (st == 1 || st == 3)) {
             if (st == 1) vm_wait<NST>();
             else vm_wait<0>();
             // the guessed point in f32: it only chooses which record to load
-            SharedSlot &refill = st == 1 ? sa : sb;
             const float g = st == 1 ? g1 : g3;
-            const float gx = __builtin_fmaf((float)px, g, (float)x);
-            const float gy = __builtin_fmaf((float)py, g, (float)y);
-            // The record's offset is formed before the test, in every step:
-            // some lane of the wave refills in most steps anyway, and these
-            // vector operations then stand between the test's compare and
-            // the scalar EXEC update that reads it, which otherwise waits for
-            // the compare's result (the empty asm keeps them out of the
-            // conditional block).
-            uint32_t cell = tiled_cell(guess_cell(gx, B.ax0, B.pinv_sx, B.pmax_x),
-                                       guess_cell(gy, B.ay0, B.pinv_sy, B.pmax_y), B.ntx);
-            __asm__ volatile("" : "+v"(cell));
-            if (!shared_in_region(refill, gx, gy)) shared_load(cells, refill, cell);
+            rec_refill<BK, CK, SH>(B, C, R, st == 1 ? sa : sb,
+                                   __builtin_fmaf((float)px, g, (float)x),
+                                   __builtin_fmaf((float)py, g, (float)y));
         }
         double dx, dy, dkx, dky;
-        rhs_shared<MATH>(B, BP, C, CP, (st == 0 || st == 3) ? sa : sb, K, sx, sy, skx, sky, dx,
-                         dy, dkx, dky);
+        rhs_rec<BK, CK, SH, MATH>(B, BP, C, CP, (st == 0 || st == 3) ? sa : sb, K, sx, sy, skx,
+                                  sky, dx, dy, dkx, dky);
         px = dx; py = dy;
         if (st == 0) {
             // the MR_SOLOUT_NEXT_DERIV test, as in rk4_step
@@ -186,16 +219,31 @@ __device__ __forceinline__ void rk4_step_shared(const BathyView &B, const BathyP
     o[2] = kx + akx * sixth; o[3] = ky + aky * sixth;
 }
 
-// the first records of a lane: both slots hold the cell its start most
+// the first records of a lane: both slots hold the cells its start most
 // likely lies in
-__device__ __forceinline__ void shared_prefetch(const BathyView &B, const SCell *cells,
-                                                SharedSlot &sa, SharedSlot &sb, double x,
-                                                double y)
+template <int BK, int CK, bool SH>
+__device__ __forceinline__ void rec_prefetch(const BathyView &B, const CurrentView &C,
+                                             const RecPtrs &R, RecSlot<BK, CK, SH> &sa,
+                                             RecSlot<BK, CK, SH> &sb, double x, double y)
 {
-    const int i1 = guess_cell((float)x, B.ax0, B.pinv_sx, B.pmax_x);
-    const int j1 = guess_cell((float)y, B.ay0, B.pinv_sy, B.pmax_y);
-    shared_load(cells, sa, tiled_cell(i1, j1, B.ntx));
-    shared_load(cells, sb, tiled_cell(i1, j1, B.ntx));
+    const float fx = (float)x, fy = (float)y;
+    if constexpr (BK == BK_GRID) {
+        const uint32_t cell = tiled_cell(guess_cell(fx, B.ax0, B.pinv_sx, B.pmax_x),
+                                         guess_cell(fy, B.ay0, B.pinv_sy, B.pmax_y), B.ntx);
+        if constexpr (SH) {
+            rec_load(R.scells, sa.d, cell);
+            rec_load(R.scells, sb.d, cell);
+        } else {
+            rec_load(R.dcells, sa.d, cell);
+            rec_load(R.dcells, sb.d, cell);
+        }
+    }
+    if constexpr (!SH && CK == CK_GRID) {
+        const uint32_t cell = tiled_cell(guess_cell(fx, C.px0, C.pinv_sx, C.pmax_x),
+                                         guess_cell(fy, C.py0, C.pinv_sy, C.pmax_y), C.ntx);
+        rec_load(R.ucells, sa.c, cell);
+        rec_load(R.ucells, sb.c, cell);
+    }
 }
 
 // A buffer descriptor over the rows from p on (raw: no stride, no swizzle;
@@ -222,14 +270,14 @@ __device__ __forceinline__ void store_row_nt(__amdgpu_buffer_rsrc_t d, uint32_t 
 // their stores write the same bytes to the same addresses): every lane
 // stores every row, with no branch around the stores.  OUT: 0 no
 // trajectories, 1 all four components, 2 any subset.
-// SC: 0 separate records per field; 1 the shared-cell records (SCell) of a
-// depth and current on the same cells (rk4_step_shared); 2 the same with dt
-// a power of two (its DY).
-template <int BK, int CK, int MATH, int OUT, int SC = 0>
+// REC: REC_NONE (rk4_step, no cell records), REC_SHARED or REC_OWN
+// (rk4_step_rec on the shared-cell records, or on each gridded field's own);
+// DYAD: dt a power of two (rk4_step_rec's DY).
+template <int BK, int CK, int MATH, int OUT, int REC, bool DYAD>
 __global__ void __launch_bounds__(256) trace_kernel(TraceArgs a)
 {
     constexpr bool PF_B = BK == BK_GRID, PF_C = CK == CK_GRID;
-    constexpr bool DYAD = SC == 2;
+    constexpr bool SH = REC == REC_SHARED;
     constexpr int NST = OUT == 1 ? 4 : 0;   // row stores issued per step
     if ((int)blockIdx.x == a.ray_blocks) {
         // the time column: t_s = t_{s-1} + dt (ode_solvers accumulates), a
@@ -261,12 +309,12 @@ __global__ void __launch_bounds__(256) trace_kernel(TraceArgs a)
     settle(K);
     BathySlot bn;                      // records prefetched for the next evaluation
     CurrentSlot cn;
-    SharedSlot sa, sb;                 // the two record slots, for shared cells
+    RecSlot<BK, CK, SH> sa, sb;        // the two record slots
     const float g1 = (float)dt, g3 = (float)(dt + half);
-    if (SC) {
-        shared_prefetch(B, a.scells, sa, sb, x, y);
-        settle(sa);                    // likewise for the first records
-        settle(sb);
+    if (REC != REC_NONE) {
+        rec_prefetch<BK, CK, SH>(B, C, a.rec, sa, sb, x, y);
+        if (PF_B) { settle(sa.d); settle(sb.d); }    // likewise for the first records
+        if (PF_C && !SH) { settle(sa.c); settle(sb.c); }
     } else {
         if (PF_B) bathy_prefetch(B, a.bp, bn, x, y);
         if (PF_C) current_prefetch(C, a.cp, cn, x, y);
@@ -337,10 +385,10 @@ __global__ void __launch_bounds__(256) trace_kernel(TraceArgs a)
                     }
                     len = -(len + 1);
                 };
-                if constexpr (SC != 0)
-                    rk4_step_shared<MATH, DYAD, NST>(B, a.bp, C, a.cp, a.scells, sa, sb, K, px,
-                                                     py, dt, half, sixth, g1, g3, so, x, y, kx,
-                                                     ky, o, stop_before, on_stop);
+                if constexpr (REC != REC_NONE)
+                    rk4_step_rec<BK, CK, SH, MATH, DYAD, NST>(
+                        B, a.bp, C, a.cp, a.rec, sa, sb, K, px, py, dt, half, sixth, g1, g3, so,
+                        x, y, kx, ky, o, stop_before, on_stop);
                 else
                     rk4_step<BK, CK, MATH>(B, a.bp, bn, C, a.cp, cn, K, px, py, dt, half,
                                            sixth, so, x, y, kx, ky, o, stop_before, on_stop);
@@ -394,10 +442,11 @@ done:
 // atomic add per wave.  Each lane holds its scene's field views, pointers and
 // step in registers, and its record slots are emptied when it changes rays.
 // Outputs: each ray's row count and last row, as trace_kernel writes them.
-template <int BK, int CK, int MATH, bool SC = false>
+template <int BK, int CK, int MATH, int REC>
 __global__ void __launch_bounds__(256) batch_kernel(BatchArgs a)
 {
     constexpr bool PF_B = BK == BK_GRID, PF_C = CK == CK_GRID;
+    constexpr bool SH = REC == REC_SHARED;
     const FastConsts K = load_view<FastConsts>(mr_fast_consts);
     settle(K);                         // as in trace_kernel
     const int lane = (int)(threadIdx.x & 63);
@@ -407,8 +456,8 @@ __global__ void __launch_bounds__(256) batch_kernel(BatchArgs a)
     CurrentPtrs cp{};
     BathySlot bn;
     CurrentSlot cn;
-    SharedSlot sa, sb;
-    const SCell *scells = nullptr;
+    RecSlot<BK, CK, SH> sa, sb;
+    RecPtrs rec{};
     double x = 0.0, y = 0.0, kx = 0.0, ky = 0.0, px = 0.0, py = 0.0;
     double dt = 0.0, half = 0.0, sixth = 0.0;
     int64_t local = 0, n_steps = 0, step = 0, len = 1;
@@ -441,9 +490,9 @@ __global__ void __launch_bounds__(256) batch_kernel(BatchArgs a)
                     end_out = S->end_out;
                     x = S->x0[local]; y = S->y0[local]; kx = S->kx0[local]; ky = S->ky0[local];
                     step = 0; len = 1; px = 0.0; py = 0.0;
-                    if (SC) {
-                        scells = S->scells;
-                        shared_prefetch(B, scells, sa, sb, x, y);
+                    if (REC != REC_NONE) {
+                        rec = S->rec;
+                        rec_prefetch<BK, CK, SH>(B, C, rec, sa, sb, x, y);
                     } else {
                         bn = BathySlot{};
                         cn = CurrentSlot{};
@@ -462,10 +511,10 @@ __global__ void __launch_bounds__(256) batch_kernel(BatchArgs a)
             if (!finished) {
                 double o[4];
                 bool stop_before;
-                if constexpr (SC)
-                    rk4_step_shared<MATH, false, 0>(B, bp, C, cp, scells, sa, sb, K, px, py, dt,
-                                                 half, sixth, (float)dt, (float)(dt + half),
-                                                 a.solout, x, y, kx, ky, o, stop_before, [] {});
+                if constexpr (REC != REC_NONE)
+                    rk4_step_rec<BK, CK, SH, MATH, false, 0>(
+                        B, bp, C, cp, rec, sa, sb, K, px, py, dt, half, sixth, (float)dt,
+                        (float)(dt + half), a.solout, x, y, kx, ky, o, stop_before, [] {});
                 else
                     rk4_step<BK, CK, MATH>(B, bp, bn, C, cp, cn, K, px, py, dt, half, sixth,
                                            a.solout, x, y, kx, ky, o, stop_before, [] {});
@@ -594,6 +643,21 @@ __global__ void build_current_kernel(CurrentBuildArgs a)
     a.mtab[t] = cell_basis(a.xp, a.yp, i, j);
 }
 
+// The fast region of a cell's record from the per-axis bounds.  An empty
+// region is lo = hi = -inf, which holds no target under the region test
+// (off_region): a target in a cell where the reference errs always takes the
+// full queries.
+template <class Args, class Rec>
+__device__ __forceinline__ void region_of(const Args &a, int64_t i, int64_t j, bool err, Rec &r)
+{
+    const float2 bx = a.fx[i], by = a.fy[j];
+    const float ninf = -__builtin_inff();
+    r.lo_x = err ? ninf : bx.x;
+    r.hi_x = err ? ninf : bx.y;
+    r.lo_y = err ? ninf : by.x;
+    r.hi_y = err ? ninf : by.y;
+}
+
 // Combined records of a depth and a current on shared cells (SCell): the
 // depth's coefficients and slopes as build_bathy_kernel makes them, the
 // current's as build_current_kernel does, the change of basis of the shared
@@ -637,16 +701,45 @@ __global__ void build_shared_kernel(SharedBuildArgs a)
         r.vx = (a.v[iD] - a.v[iA]) / a.cxspace;
         r.vy = (a.v[iB] - a.v[iA]) / a.cyspace;
     }
-    // An empty region is lo = hi = -inf, which holds no target under the
-    // region test (shared_in_region): a target in a cell where the reference
-    // errs always takes the full queries.
-    const float2 bx = a.fx[i], by = a.fy[j];
-    const float ninf = -__builtin_inff();
-    r.lo_x = err ? ninf : bx.x;
-    r.hi_x = err ? ninf : bx.y;
-    r.lo_y = err ? ninf : by.x;
-    r.hi_y = err ? ninf : by.y;
+    region_of(a, i, j, err, r);
     a.cells[tiled_cell((int)i, (int)j, a.ntx)] = r;
+}
+
+// A field's own records (DCell, UCell), from its plain records: the same
+// values with the cell's origin and fast region beside them.
+__global__ void build_depth_rec_kernel(RecBuildArgs a, const BCell *plain, DCell *cells)
+{
+    const int64_t ncx = a.nx - 1;
+    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= ncx * (a.ny - 1)) return;
+    const int64_t i = c % ncx, j = c / ncx;
+    const uint32_t t = tiled_cell((int)i, (int)j, a.ntx);
+    const BCell p = plain[t];
+    DCell r;
+    r.x0 = a.xp[i].x; r.y0 = a.yp[j].x; r.m01 = p.m01; r.m10 = p.m10;
+    r.a00 = p.a00; r.a10 = p.a10; r.a01 = p.a01; r.a11 = p.a11;
+    r.hx = (double)p.hx; r.hy = (double)p.hy;
+    region_of(a, i, j, c >= a.oob_from || __builtin_isnan(p.m01), r);
+    cells[t] = r;
+}
+
+__global__ void build_current_rec_kernel(RecBuildArgs a, const CCell *plain, const float2 *mtab,
+                                         UCell *cells)
+{
+    const int64_t ncx = a.nx - 1;
+    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= ncx * (a.ny - 1)) return;
+    const int64_t i = c % ncx, j = c / ncx;
+    const uint32_t t = tiled_cell((int)i, (int)j, a.ntx);
+    const CCell p = plain[t];
+    const float2 m = mtab[t];
+    UCell r;
+    r.x0 = a.xp[i].x; r.y0 = a.yp[j].x; r.m01 = m.x; r.m10 = m.y;
+    r.ua00 = p.ua00; r.ua10 = p.ua10; r.ua01 = p.ua01; r.ua11 = p.ua11;
+    r.va00 = p.va00; r.va10 = p.va10; r.va01 = p.va01; r.va11 = p.va11;
+    r.ux = p.ux; r.uy = p.uy; r.vx = p.vx; r.vy = p.vy;
+    region_of(a, i, j, c >= a.oob_from || __builtin_isnan(m.x), r);
+    cells[t] = r;
 }
 
 // ---------------------------------------------------------------------------
@@ -663,41 +756,38 @@ hipError_t launch_trace(const TraceArgs &a, int bk, int ck, int math, int block,
     // takes any subset (OUT 2)
     int nout = (a.xo != nullptr) + (a.yo != nullptr) + (a.kxo != nullptr) + (a.kyo != nullptr);
     if (nout == 4 && a.n_rays >= (int64_t(1) << 27)) nout = 5;
-    if (a.shared_cells && bk == BK_GRID && ck == CK_GRID) {
-        // a power-of-two step: dt/2 and dt scale exactly
-        int e2 = 0;
-        const bool dy = std::fabs(std::frexp(a.dt, &e2)) == 0.5 && std::isnormal(a.half);
-        auto go = [&](auto m, auto sc) {
-            constexpr int M = decltype(m)::value, S = decltype(sc)::value;
-            if (nout == 0)
-                hipLaunchKernelGGL((trace_kernel<BK_GRID, CK_GRID, M, 0, S>), grid, dim3(block),
-                                   0, stream, a);
-            else if (nout == 4)
-                hipLaunchKernelGGL((trace_kernel<BK_GRID, CK_GRID, M, 1, S>), grid, dim3(block),
-                                   0, stream, a);
-            else
-                hipLaunchKernelGGL((trace_kernel<BK_GRID, CK_GRID, M, 2, S>), grid, dim3(block),
-                                   0, stream, a);
-        };
-        auto by_sc = [&](auto m) {
-            if (dy) go(m, std::integral_constant<int, 2>{});
-            else go(m, std::integral_constant<int, 1>{});
-        };
-        if (math == MATH_FAST) by_sc(std::integral_constant<int, MATH_FAST>{});
-        else by_sc(std::integral_constant<int, MATH_LITERAL>{});
-        return hipGetLastError();
-    }
+    // a power-of-two step: dt/2 and dt scale exactly
+    int e2 = 0;
+    const bool dyad = std::fabs(std::frexp(a.dt, &e2)) == 0.5 && std::isnormal(a.half);
+    auto launch = [&](auto k, auto rc, auto dy) {
+        using K = decltype(k);
+        constexpr int REC = decltype(rc)::value;
+        constexpr bool DY = decltype(dy)::value;
+        if (REC != REC_NONE && nout == 0)
+            hipLaunchKernelGGL((trace_kernel<K::bk, K::ck, K::math, 0, REC, DY>), grid,
+                               dim3(block), 0, stream, a);
+        else if (REC != REC_NONE && nout == 4)
+            hipLaunchKernelGGL((trace_kernel<K::bk, K::ck, K::math, 1, REC, DY>), grid,
+                               dim3(block), 0, stream, a);
+        else
+            hipLaunchKernelGGL((trace_kernel<K::bk, K::ck, K::math, 2, REC, DY>), grid,
+                               dim3(block), 0, stream, a);
+    };
+    auto by_step = [&](auto k, auto rc) {
+        if (dyad) launch(k, rc, std::true_type{});
+        else launch(k, rc, std::false_type{});
+    };
     dispatch_kinds(bk, ck, math, [&](auto k) {
         using K = decltype(k);
-        if (nout == 0)
-            hipLaunchKernelGGL((trace_kernel<K::bk, K::ck, K::math, 0>), grid, dim3(block), 0,
-                               stream, a);
-        else if (nout == 4)
-            hipLaunchKernelGGL((trace_kernel<K::bk, K::ck, K::math, 1>), grid, dim3(block), 0,
-                               stream, a);
-        else
-            hipLaunchKernelGGL((trace_kernel<K::bk, K::ck, K::math, 2>), grid, dim3(block), 0,
-                               stream, a);
+        constexpr bool both = K::bk == BK_GRID && K::ck == CK_GRID;
+        constexpr bool any = K::bk == BK_GRID || K::ck == CK_GRID;
+        if constexpr (both)
+            if (a.records == REC_SHARED)
+                return by_step(k, std::integral_constant<int, REC_SHARED>{});
+        if constexpr (any)
+            if (a.records == REC_NONE)
+                return launch(k, std::integral_constant<int, REC_NONE>{}, std::false_type{});
+        by_step(k, std::integral_constant<int, REC_OWN>{});
     });
     return hipGetLastError();
 }
@@ -707,19 +797,20 @@ hipError_t launch_batch(const BatchArgs &a, int bk, int ck, int math, int block,
 {
     if (a.n_rays <= 0) return hipSuccess;
     if (block < 64 || block > 256 || block % 64 || blocks < 1) return hipErrorInvalidValue;
-    if (a.shared_cells && bk == BK_GRID && ck == CK_GRID) {
-        if (math == MATH_FAST)
-            hipLaunchKernelGGL((batch_kernel<BK_GRID, CK_GRID, MATH_FAST, true>),
-                               dim3((unsigned)blocks), dim3(block), 0, stream, a);
-        else
-            hipLaunchKernelGGL((batch_kernel<BK_GRID, CK_GRID, MATH_LITERAL, true>),
-                               dim3((unsigned)blocks), dim3(block), 0, stream, a);
-        return hipGetLastError();
-    }
     dispatch_kinds(bk, ck, math, [&](auto k) {
-        using KK = decltype(k);
-        hipLaunchKernelGGL((batch_kernel<KK::bk, KK::ck, KK::math>), dim3((unsigned)blocks),
-                           dim3(block), 0, stream, a);
+        using K = decltype(k);
+        constexpr bool both = K::bk == BK_GRID && K::ck == CK_GRID;
+        constexpr bool any = K::bk == BK_GRID || K::ck == CK_GRID;
+        auto launch = [&](auto rc) {
+            hipLaunchKernelGGL((batch_kernel<K::bk, K::ck, K::math, decltype(rc)::value>),
+                               dim3((unsigned)blocks), dim3(block), 0, stream, a);
+        };
+        if constexpr (both)
+            if (a.records == REC_SHARED)
+                return launch(std::integral_constant<int, REC_SHARED>{});
+        if constexpr (any)
+            if (a.records == REC_NONE) return launch(std::integral_constant<int, REC_NONE>{});
+        launch(std::integral_constant<int, REC_OWN>{});
     });
     return hipGetLastError();
 }
@@ -755,6 +846,26 @@ hipError_t launch_build_bathy(const BathyBuildArgs &a, hipStream_t stream)
     const int block = 256;
     hipLaunchKernelGGL(build_bathy_kernel, dim3((unsigned)((ncell + block - 1) / block)),
                        dim3(block), 0, stream, a);
+    return hipGetLastError();
+}
+
+hipError_t launch_build_depth_rec(const RecBuildArgs &a, const BCell *plain, DCell *cells,
+                                  hipStream_t stream)
+{
+    const int64_t ncell = (a.nx - 1) * (a.ny - 1);
+    if (ncell <= 0) return hipSuccess;
+    hipLaunchKernelGGL(build_depth_rec_kernel, dim3((unsigned)((ncell + 255) / 256)), dim3(256),
+                       0, stream, a, plain, cells);
+    return hipGetLastError();
+}
+
+hipError_t launch_build_current_rec(const RecBuildArgs &a, const CCell *plain, const float2 *mtab,
+                                    UCell *cells, hipStream_t stream)
+{
+    const int64_t ncell = (a.nx - 1) * (a.ny - 1);
+    if (ncell <= 0) return hipSuccess;
+    hipLaunchKernelGGL(build_current_rec_kernel, dim3((unsigned)((ncell + 255) / 256)),
+                       dim3(256), 0, stream, a, plain, mtab, cells);
     return hipGetLastError();
 }
 
