@@ -63,7 +63,7 @@ extern "C" {
 
 /* mr_options.math */
 #define MR_MATH_FAST    0       /* dispersion terms in closed form from one exp */
-#define MR_MATH_LITERAL 1       /* atan2/cos/sin/tanh/cosh/sinh as written */
+#define MR_MATH_LITERAL 1       /* the reference's formulas to its libm's accuracy */
 
 /* mr_options.solout: what stops a ray (src/wave_ray_path.rs:236-246) */
 #define MR_SOLOUT_STATE      0  /* the new state is all-NaN */

@@ -524,13 +524,25 @@ __device__ __forceinline__ double rsq_nr(double x)
     return __builtin_fma(0.5 * y, e, y);
 }
 
-// The f64 constants of the fast dispersion evaluation.  Kernels copy them
+// 1/sqrt(x) to about an ulp: the same estimate and residual e = 1 - x y^2,
+// with the next term of the series, y (1 + e/2 + 3/8 e^2), whose own error is
+// of order e^3 (1e-21).
+__device__ __forceinline__ double rsq_full(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    const double t = x * y;
+    const double e = __builtin_fma(-t, y, 1.0);
+    return __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
+}
+
+// The f64 constants of the dispersion evaluations.  Kernels copy them
 // into per-lane registers at start (load_view), so that the loop does not
 // rebuild each one in a scalar register pair at every use.
 struct FastConsts {
     double inv_ln2, ln2_hi, ln2_lo;   // 1/ln 2; ln 2 split in two parts
     double clamp;                     // |argument| limit of exp_pair
     double expc[10];                  // expm1(f)/f ~ sum c_j f^j, c_9 first (Horner order)
+    double expl[10];                  // (expm1(f) - f)/f^2, likewise
     double g, half_g, m2g;            // g, g/2 and -2g
     double nan;                       // a quiet NaN
 };
@@ -559,6 +571,26 @@ __device__ __forceinline__ void exp_pair(double r, double &e, double &em, const 
     em = __builtin_fma(-s, p, 1.0 - s);
 }
 
+// exp_pair to about an ulp: expm1(f) = f + f^2 Q(f) with Q of degree 9
+// interpolating (expm1(f) - f)/f^2 at the Chebyshev nodes of [-ln2/2, ln2/2]
+// (3.7e-17 of expm1(f)), so that only the last addition rounds at the size
+// of the result.
+__device__ __forceinline__ void exp_pair_full(double r, double &e, double &em,
+                                              const FastConsts &K)
+{
+    r = __builtin_fmax(__builtin_fmin(r, K.clamp), -K.clamp);
+    const double m = __builtin_rint(r * K.inv_ln2);
+    double f = __builtin_fma(-m, K.ln2_hi, r);
+    f = __builtin_fma(-m, K.ln2_lo, f);
+    double Q = K.expl[0];
+#pragma unroll
+    for (int j = 1; j < 10; ++j) Q = __builtin_fma(Q, f, K.expl[j]);
+    const double p = __builtin_fma(f * f, Q, f);        // expm1(f)
+    const double s = __builtin_ldexp(1.0, (int)m);
+    e = __builtin_fma(s, p, s);
+    em = __builtin_fma(-s, p, 1.0 - s);
+}
+
 // ---------------------------------------------------------------------------
 // WaveRayPath::odes (wave_ray_path.rs:118-150) from the field values at the
 // point: depth h (NaN where the bathymetry errs), its gradient, the current
@@ -571,30 +603,46 @@ __device__ __forceinline__ void odes(const FastConsts &K, double h, double hx, d
                                      double &dy, double &dkx, double &dky)
 {
     if (MATH == MATH_LITERAL) {
-        // A NaN depth (a provider error, or a NaN target or datum) makes
-        // every derivative NaN through group_velocity and dkdt_bathy, as an
-        // error does, except when k <= 0 errs first; both end all-NaN.
-        bool ok = okc;
-        const double k = sqrt(kx * kx + ky * ky);           // :133-134
-        const double theta = atan2(ky, kx);
-        // group_velocity :177-188: h <= 0 -> NaN (Ok); k <= 0 -> Err
-        if (!(h <= 0.0) && k <= 0.0) ok = false;
-        double cg;
-        if (h <= 0.0) {
-            cg = MR_NAN;
-        } else {
-            const double ch = cosh(k * h);
-            cg = (G / 2.0) * ((tanh(k * h) + (k * h) / (ch * ch)) / sqrt(k * G * tanh(k * h)));
-        }
-        const double cgx = cg * cos(theta) + u;             // :138-139
-        const double cgy = cg * sin(theta) + v;
-        // dkdt_bathy :207-216
-        const double c = (-0.5) * k / sinh(k * h) / cosh(k * h) * sqrt(G * k * tanh(k * h));
-        const double dkxb = c * hx, dkyb = c * hy;
-        dx = ok ? cgx : MR_NAN;
-        dy = ok ? cgy : MR_NAN;
-        dkx = ok ? (dkxb - kx * ux) - ky * vx : MR_NAN;      // :146-147
-        dky = ok ? (dkyb - kx * uy) - ky * vy : MR_NAN;
+        // The reference's formulas to the accuracy of its libm calls, from
+        // one exponential and two reciprocal square roots refined to full
+        // precision.  With e = exp(-2kh), em = 1 - e and
+        // W = 1/sqrt(g k em (1 + e)):
+        //   cos theta = kx/k, sin theta = ky/k                (:133-139)
+        //   tanh kh = em/(1+e), kh/cosh^2 kh = 4kh e/(1+e)^2   (:177-188)
+        //   sinh kh cosh kh = em (1+e)/(4e)                   (:207-216)
+        // so cg = (g/2) W (em + 4kh e/(1+e)) and c = -2 g k^2 (e/(1+e)) W,
+        // as in the fast form below, whose account of errors and NaNs holds
+        // here too.  Against 128-bit arithmetic, over k of 0.002 to 1 rad/m
+        // and depths of 0.5 to 3000 m, cg cos(theta) is off by 0.9-1.0e-16 of
+        // cg (rms) where the libm calls (tanh, cosh, sinh, atan2, cos, sin)
+        // were off by 1.1-1.2e-16, and c by no more than they were (1.4e-16
+        // at 0.5 m; in deep water both lose kh 2^-53 to the rounding of
+        // kh).  Those calls were nine tenths of the step, which this form
+        // leaves bound by the issue of its own instructions, as the fast
+        // form is: 16,384 rays x 500 steps on shared cells with trajectories
+        // 4.33 -> 0.57 ms.
+        h = okc ? h : MR_NAN;
+        const double k2 = __builtin_fma(kx, kx, ky * ky);
+        const double rk = rsq_full(k2);                     // 1/k
+        const double k1 = k2 * rk;
+        const double k = __builtin_fma(__builtin_fma(-k1, k1, k2), 0.5 * rk, k1);
+        const double kh = k * h;
+        double e, em;
+        exp_pair_full(-2.0 * kh, e, em, K);
+        const double gke = (K.g * k) * em;
+        const double W = rsq_full(__builtin_fma(gke, e, gke));
+        // e/(1+e): from 1/(1+e) to a few ulps, corrected by the residual
+        // e - (1+e) q, formed without rounding 1+e (e - q is exact)
+        const double i0 = gke * (W * W);
+        const double q = e * i0;
+        const double ei = __builtin_fma(i0, __builtin_fma(-e, q, e - q), q);
+        const double cgr = ((K.half_g * rk) * W) * __builtin_fma(kh, 4.0 * ei, em);
+        // (k twice, not k^2: its rounding then partly cancels that of e's k)
+        const double c = (K.m2g * k) * (k * (ei * W));
+        dx = __builtin_fma(cgr, kx, u);
+        dy = __builtin_fma(cgr, ky, v);
+        dkx = __builtin_fma(-ky, vx, __builtin_fma(-kx, ux, c * hx));    // :146-147
+        dky = __builtin_fma(-ky, vy, __builtin_fma(-kx, uy, c * hy));
     } else {
         // Every provider error, h <= 0 (or NaN), k <= 0 (or NaN) and a
         // non-finite k*h give all-NaN derivatives in the reference (an

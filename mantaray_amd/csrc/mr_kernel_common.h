@@ -78,6 +78,17 @@ static __device__ double mr_fast_consts[sizeof(FastConsts) / sizeof(double)] = {
     1.6666666666615648e-01,
     5.000000000000001e-01,
     1.0000000000000013,
+    // (expm1(f) - f)/f^2, interpolated likewise, c_9 .. c_0
+    2.5100375832561234e-08,
+    2.7620075879983367e-07,
+    2.7557268480310024e-06,
+    2.4801521322368692e-05,
+    1.9841269863040545e-04,
+    1.3888888917196719e-03,
+    8.333333333330065e-03,
+    4.1666666666624164e-02,
+    1.6666666666666669e-01,
+    5.000000000000001e-01,
     G,
     0.5 * G,
     -2.0 * G,
