@@ -171,6 +171,11 @@ int mr_trace_many(const mr_field *bathy, const mr_field *current, int64_t n_rays
                   double *t_out, double *x_out, double *y_out, double *kx_out,
                   double *ky_out, int32_t *len_out, double *end_out);
 
+/* The time of every row of every ray, as mantaray.core.ray_tracing lays it
+ * out (python/mantaray/core.py:114-125): out[s * n_rays + r] = t[s] for
+ * s < len[r], NaN past a ray's last row.  Host arrays. */
+int mr_time_rows(int64_t n_rows, int64_t n_rays, const double *t, const int32_t *len, double *out);
+
 /* SingleRay::trace_individual (src/ray.rs:198-213) as called by
  * _mantaray.single_ray (src/ffi.rs:25-49).  rows_out holds (n+1) rows of
  * (t, x, y, kx, ky); *n_rows receives the rows produced. */

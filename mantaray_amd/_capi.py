@@ -37,7 +37,7 @@ EXPORTS = (
     "mr_current_from_arrays", "mr_bathy_constant", "mr_bathy_slope", "mr_bathy_array",
     "mr_current_constant", "mr_field_free", "mr_field_kind", "mr_field_grid_shape",
     "mr_field_copy_grid", "mr_field_upload", "mr_num_steps", "mr_trace_many",
-    "mr_single_ray", "mr_rhs_many", "mr_checkpoint_count", "mr_adjoint_workspace_size",
+    "mr_single_ray", "mr_time_rows", "mr_rhs_many", "mr_checkpoint_count", "mr_adjoint_workspace_size",
     "mr_trace_fp64", "mr_adjoint_many", "mr_adjoint_many_noalloc", "mr_ray_result_json",
     "mr_ray_result_append_tsv",
     "mr_batch_create", "mr_batch_run", "mr_batch_info", "mr_batch_free",
@@ -114,6 +114,7 @@ _SIGS = {
                                      _vp, _vp]),
     "mr_single_ray": (ctypes.c_int, [_fieldp, _fieldp, _f64, _f64, _f64, _f64, _f64, _f64,
                                      _f64, ctypes.POINTER(Options), _vp, _i64p]),
+    "mr_time_rows": (ctypes.c_int, [_i64, _i64, _vp, _vp, _vp]),
     "mr_rhs_many": (ctypes.c_int, [_fieldp, _fieldp, _i64, _vp, _vp, ctypes.POINTER(Options)]),
     "mr_checkpoint_count": (ctypes.c_int, [_f64, _f64, _f64, ctypes.c_int32, _i64p]),
     "mr_adjoint_workspace_size": (ctypes.c_int, [_i64, ctypes.c_int32, _i64p]),

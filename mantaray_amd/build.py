@@ -39,7 +39,8 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libmantaray_hip.so")
-SOURCES = ["mr_kernels.hip", "mr_adjoint.hip", "mr_capi.cpp", "mr_netcdf3.cpp", "mr_results.cpp"]
+SOURCES = ["mr_kernels.hip", "mr_adjoint.hip", "mr_capi.cpp", "mr_hostio.cpp",
+           "mr_netcdf3.cpp", "mr_results.cpp"]
 ARCH = os.environ.get("MANTARAY_OFFLOAD_ARCH", "gfx950")
 # packed FP32 arithmetic the device code must not contain
 BANNED = re.compile(r"\bv_pk_(add|mul|fma)_f32\b")

@@ -196,22 +196,27 @@ def ray_tracing(x0: Sequence[float], y0: Sequence[float], kx0: Sequence[float],
     ray, as core.py:114-125 pads the per-ray lists.
     """
     b, c = _fields(bathymetry, current)
-    return rays_dataset(trace_many(b, c, x0, y0, kx0, ky0, 0.0, duration, step_size, **kw))
+    return rays_dataset(trace_many(b, c, x0, y0, kx0, ky0, 0.0, duration, step_size, **kw),
+                        copy=False)
 
 
-def rays_dataset(r: dict):
+def rays_dataset(r: dict, copy: bool = True):
     """The ray_tracing Dataset (core.py:104-132) of a trace_many result: each
-    ray's rows, then all-NaN rows (time too) up to the longest ray."""
+    ray's rows, then all-NaN rows (time too) up to the longest ray.  With
+    copy=False the Dataset takes the result's arrays over where it keeps all
+    their rows."""
     ln = r["len"]
     nr = ln.size
     if nr == 0:
         raise ValueError("max() arg is an empty sequence")   # core.py:111 on no rays
     longest = int(ln.max())
-    valid = np.arange(longest)[:, None] < ln[None, :]
-    time = np.where(valid, r["t"][:longest, None], np.nan)
+    t = np.ascontiguousarray(r["t"], dtype=np.float64)
+    lens = np.ascontiguousarray(ln, dtype=np.int32)
+    time = np.empty((longest, nr))
+    C.check(C.lib().mr_time_rows(longest, nr, t.ctypes.data, lens.ctypes.data, time.ctypes.data))
     data = {"time": time}
     for k in ("x", "y", "kx", "ky"):
-        data[k] = r[k][:longest].copy()
+        data[k] = r[k][:longest].copy() if copy or longest < len(r[k]) else r[k]
     ds = _Dataset({name: (["time_step", "ray"], v) for name, v in data.items()})
     ds = ds.set_coords(["time", "x", "y"])
     ds["time_step"] = range(longest)

@@ -18,6 +18,7 @@
 #include <string>
 #include <vector>
 
+#include "mr_hostio.h"
 #include "mr_kernels.h"
 #include "mr_netcdf3.h"
 
@@ -147,7 +148,16 @@ struct mr_field {
     // a bathymetry's combined records with a current on shared cells, per
     // (device * 16 + record tile, current uid)
     std::map<std::pair<int, uint64_t>, std::unique_ptr<DevTables>> shared;
+
+    mr_field() { ++live; }
+    ~mr_field()
+    {
+        if (--live == 0) drop_idle_stages();
+    }
+    static std::atomic<int64_t> live;   // handles of the process
 };
+
+std::atomic<int64_t> mr_field::live{0};
 
 struct mr_batch {
     int device = 0;
@@ -989,6 +999,59 @@ int trace_device(const mr_field *bathy, const mr_field *current, int64_t n_rays,
     return MR_OK;
 }
 
+// the trace with host arrays, synchronous: through a stage's device buffer
+int trace_host(const mr_field *bathy, const mr_field *current, int64_t n_rays, const double *x0,
+               const double *y0, const double *kx0, const double *ky0, double t0, int64_t n,
+               double dt, const mr_options &o, double *t_out, double *x_out, double *y_out,
+               double *kx_out, double *ky_out, int32_t *len_out, double *end_out)
+{
+    // t += dt as ode_solvers accumulates it
+    if (t_out) {
+        double t = t0;
+        t_out[0] = t;
+        for (int64_t s = 1; s <= n; s++) t_out[s] = t = t + dt;
+    }
+    const size_t nr = (size_t)n_rays, rows = (size_t)n + 1;
+    if (nr && rows > (SIZE_MAX / 64) / nr)
+        return fail(MR_ERR_OUT_OF_MEMORY, "trajectories do not fit in memory");
+    size_t used = 0;
+    std::vector<HostPiece> in, out;
+    // the pieces' device addresses are 256-byte aligned, as an allocation's are
+    auto piece = [&](std::vector<HostPiece> &list, const void *host, size_t bytes) {
+        if (host && bytes)
+            list.push_back({static_cast<char *>(const_cast<void *>(host)), used, bytes});
+        const size_t at = used;
+        if (host) used += (bytes + 255) & ~size_t(255);
+        return at;
+    };
+    size_t ic[4], row[4];
+    const double *h_ic[4] = {x0, y0, kx0, ky0};
+    double *h_row[4] = {x_out, y_out, kx_out, ky_out};
+    for (int q = 0; q < 4; q++) ic[q] = piece(in, h_ic[q], nr * sizeof(double));
+    const size_t len_at = piece(out, len_out, nr * sizeof(int32_t));
+    const size_t end_at = piece(out, end_out, 4 * nr * sizeof(double));
+    for (int q = 0; q < 4; q++) row[q] = piece(out, h_row[q], rows * nr * sizeof(double));
+    hipError_t e = hipSuccess;
+    const StagePtr st = acquire_stage(used, &e);
+    MR_HIP_TRY(e);
+    MR_HIP_TRY(copy_in(*st, in));
+    char *dev = stage_device(*st);
+    auto at = [&](const void *host, size_t off) {
+        return host ? reinterpret_cast<double *>(dev + off) : nullptr;
+    };
+    const int rc = trace_device(bathy, current, n_rays, at(x0, ic[0]), at(y0, ic[1]),
+                                at(kx0, ic[2]), at(ky0, ic[3]), t0, n, dt, o, stage_stream(*st),
+                                nullptr, at(x_out, row[0]), at(y_out, row[1]), at(kx_out, row[2]),
+                                at(ky_out, row[3]),
+                                reinterpret_cast<int32_t *>(at(len_out, len_at)),
+                                at(end_out, end_at));
+    // wait also when the launch failed: the stage goes back to the pool
+    e = rc ? hipStreamSynchronize(stage_stream(*st)) : copy_out(*st, out);
+    if (rc) return rc;
+    MR_HIP_TRY(e);
+    return MR_OK;
+}
+
 // mr_adjoint_many and mr_adjoint_many_noalloc: with no_alloc the work buffer
 // is this device's scratch array and no field table is built
 int adjoint_run(const mr_field *bathy, const mr_field *current, const double *depth,
@@ -1353,37 +1416,24 @@ int mr_trace_many(const mr_field *bathy, const mr_field *current, int64_t n_rays
                             (hipStream_t)o.stream, t_out, x_out, y_out, kx_out, ky_out,
                             len_out, end_out);
     }
-    // host memory: stage through device buffers, synchronous
-    DevTables tmp;
-    const size_t nr = (size_t)n_rays, rows = (size_t)n + 1;
-    double *d_ic = nullptr, *d_t = nullptr, *d_end = nullptr;
-    double *d_out[4] = {nullptr, nullptr, nullptr, nullptr};
-    int32_t *d_len = nullptr;
-    double *h_out[4] = {x_out, y_out, kx_out, ky_out};
-    if ((rc = dev_alloc(tmp, 4 * nr, &d_ic))) return rc;
-    const double *h_ic[4] = {x0, y0, kx0, ky0};
-    for (int q = 0; q < 4; q++)
-        if (nr) MR_HIP_TRY(hipMemcpy(d_ic + q * nr, h_ic[q], nr * sizeof(double),
-                                     hipMemcpyHostToDevice));
-    if (t_out && (rc = dev_alloc(tmp, rows, &d_t))) return rc;
-    for (int q = 0; q < 4; q++)
-        if (h_out[q] && (rc = dev_alloc(tmp, rows * nr, &d_out[q]))) return rc;
-    if (len_out && (rc = dev_alloc(tmp, nr, &d_len))) return rc;
-    if (end_out && (rc = dev_alloc(tmp, 4 * nr, &d_end))) return rc;
-    rc = trace_device(bathy, current, n_rays, d_ic, d_ic + nr, d_ic + 2 * nr, d_ic + 3 * nr,
-                      t0, n, dt, o, 0, d_t, d_out[0], d_out[1], d_out[2], d_out[3], d_len,
-                      d_end);
-    if (rc) return rc;
-    MR_HIP_TRY(hipDeviceSynchronize());
-    if (t_out) MR_HIP_TRY(hipMemcpy(t_out, d_t, rows * sizeof(double), hipMemcpyDeviceToHost));
-    for (int q = 0; q < 4; q++)
-        if (h_out[q] && nr)
-            MR_HIP_TRY(hipMemcpy(h_out[q], d_out[q], rows * nr * sizeof(double),
-                                 hipMemcpyDeviceToHost));
-    if (len_out && nr)
-        MR_HIP_TRY(hipMemcpy(len_out, d_len, nr * sizeof(int32_t), hipMemcpyDeviceToHost));
-    if (end_out && nr)
-        MR_HIP_TRY(hipMemcpy(end_out, d_end, 4 * nr * sizeof(double), hipMemcpyDeviceToHost));
+    return trace_host(bathy, current, n_rays, x0, y0, kx0, ky0, t0, n, dt, o, t_out, x_out, y_out,
+                      kx_out, ky_out, len_out, end_out);
+    MR_GUARD_END
+}
+
+int mr_time_rows(int64_t n_rows, int64_t n_rays, const double *t, const int32_t *len, double *out)
+{
+    MR_GUARD_BEGIN
+    if (n_rows < 0 || n_rays < 0 || (n_rows && !t) || (n_rays && !len) ||
+        (n_rows && n_rays && !out))
+        return fail(MR_ERR_INVALID_ARGUMENT, "invalid arrays");
+    const int64_t per = std::max<int64_t>(1, (int64_t(1) << 19) / std::max<int64_t>(1, n_rays));
+    parallel_for((n_rows + per - 1) / per, copy_threads((size_t)(n_rows * n_rays) * 8),
+                 [&](int64_t c) {
+        for (int64_t s = c * per; s < std::min(n_rows, (c + 1) * per); s++)
+            for (int64_t r = 0; r < n_rays; r++)
+                out[s * n_rays + r] = s < len[r] ? t[s] : (double)NAN;
+    });
     return MR_OK;
     MR_GUARD_END
 }
