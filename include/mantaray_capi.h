@@ -85,12 +85,14 @@ typedef struct mr_options {
     int32_t block_size;    /* threads per block, multiple of 64; 0 = tuned */
     int32_t blocks_per_cu; /* mr_batch_run: resident workgroups per CU; 0 = tuned */
     void   *stream;        /* hipStream_t for MR_MEM_DEVICE; NULL = null stream */
-    int32_t record_tile;   /* gridded fields, reference precision: cell records
-                              are stored in square tiles of 2^record_tile cells
-                              a side (0 = row-major ... 5 = 32 x 32); -1 =
-                              default (3, 8 x 8).  Results do not depend on it.
-                              A field keeps the tables of each tile shape it
-                              was used with until it is freed. */
+    int32_t record_tile;   /* gridded fields, reference precision: the records
+                              that full queries read (and grids too large for
+                              cell records run on) are stored in square tiles
+                              of 2^record_tile cells a side (0 = row-major ...
+                              5 = 32 x 32); -1 = default (3, 8 x 8).  Results
+                              do not depend on it.  A field keeps the tables
+                              of each tile shape it was used with until it is
+                              freed. */
 } mr_options;
 
 /* Defaults: reference precision, fast math, MR_SOLOUT_STATE, host memory,

@@ -191,7 +191,7 @@ __global__ void __launch_bounds__(256) trace64_kernel(Trace64Args a)
     }
     const Grid64View B = load_view<Grid64View>(a.B);
     const Grid64View C = load_view<Grid64View>(a.C);
-    const FastConsts K = load_view<FastConsts>(mr_fast_consts);
+    const FastConsts K = load_consts();
     const double half = a.half, dt = a.dt, sixth = a.sixth;
     Slots64 sa, sb;                    // the step's two cell slots
     load_guess64<BK, CK>(B, a.bp, C, a.cp, a.f, sa, s[0], s[1]);
@@ -200,7 +200,6 @@ __global__ void __launch_bounds__(256) trace64_kernel(Trace64Args a)
     // nothing pending to wait for (as in trace_kernel)
     settle(B);
     settle(C);
-    settle(K);
     settle(sa);
     settle(sb);
     bool alive = true;
@@ -363,7 +362,7 @@ __global__ void __launch_bounds__(ADJ_BLOCK) adjoint_kernel(AdjointArgs a)
     const int64_t r = active ? rr : nr - 1;
     const Grid64View B = load_view<Grid64View>(a.B);
     const Grid64View C = load_view<Grid64View>(a.C);
-    const FastConsts K = load_view<FastConsts>(mr_fast_consts);
+    const FastConsts K = load_consts();
     const double dt = a.dt, half = a.half, sixth = a.sixth;
     const int stride = a.stride;
     const int64_t ld = a.work_ld;
@@ -477,7 +476,7 @@ __global__ void __launch_bounds__(64) adjoint_seq_kernel(AdjointArgs a)
     const int64_t r = active ? rr : nr - 1;
     const Grid64View B = load_view<Grid64View>(a.B);
     const Grid64View C = load_view<Grid64View>(a.C);
-    const FastConsts K = load_view<FastConsts>(mr_fast_consts);
+    const FastConsts K = load_consts();
     const double dt = a.dt, half = a.half, sixth = a.sixth;
     const int stride = a.stride;
     const int64_t ld = a.work_ld;
@@ -605,7 +604,7 @@ __global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs 
     const int64_t r = active ? rr : nr - 1;
     const Grid64View B = load_view<Grid64View>(a.B);
     const Grid64View C = load_view<Grid64View>(a.C);
-    const FastConsts K = load_view<FastConsts>(mr_fast_consts);
+    const FastConsts K = load_consts();
     const double dt = a.dt, half = a.half, sixth = a.sixth;
     const int stride = a.stride;
     const int64_t ld = a.work_ld;
@@ -868,7 +867,7 @@ __global__ void __launch_bounds__(256) rhs64_kernel(Rhs64Args a)
     if (i >= a.n) return;
     const Grid64View B = load_view<Grid64View>(a.B);
     const Grid64View C = load_view<Grid64View>(a.C);
-    const FastConsts K = load_view<FastConsts>(mr_fast_consts);
+    const FastConsts K = load_consts();
     double dx, dy, dkx, dky;
     Slots64 sl;                        // empty: the query loads the cell
     rhs64<BK, CK, MATH>(B, a.bp, C, a.cp, a.f, sl, K, a.s[4 * i], a.s[4 * i + 1], a.s[4 * i + 2],

@@ -146,7 +146,7 @@ struct mr_field {
     std::mutex mu;
     std::map<int, std::unique_ptr<DevTables>> dev;
     // a bathymetry's combined records with a current on shared cells, per
-    // (device * 16 + record tile, current uid)
+    // (device, current uid)
     std::map<std::pair<int, uint64_t>, std::unique_ptr<DevTables>> shared;
 
     mr_field() { ++live; }
@@ -815,7 +815,7 @@ int shared_tables(const mr_field *cb, const mr_field *cc, int tl, const SCell **
     mr_field *b = const_cast<mr_field *>(cb);
     int dev = 0;
     MR_HIP_TRY(hipGetDevice(&dev));
-    const std::pair<int, uint64_t> key(dev * 16 + tl, cc->uid);
+    const std::pair<int, uint64_t> key(dev, cc->uid);
     std::lock_guard<std::mutex> lk(b->mu);
     auto it = b->shared.find(key);
     if (it != b->shared.end()) {
@@ -833,11 +833,8 @@ int shared_tables(const mr_field *cb, const mr_field *cc, int tl, const SCell **
     if ((rc = dev_upload(*t, fx.data(), fx.size(), &dfx)) ||
         (rc = dev_upload(*t, fy.data(), fy.size(), &dfy)))
         return rc;
-    const int64_t ntx = tiles_along(b->nx, tl), nty = tiles_along(b->ny, tl);
     SCell *cells;
-    if ((rc = validate_grid(b->nx, b->ny, (int64_t)sizeof(SCell), tl)) ||
-        (rc = dev_alloc(*t, (size_t)((ntx * nty) << (2 * tl)), &cells)))
-        return rc;
+    if ((rc = dev_alloc(*t, (size_t)((b->nx - 1) * (b->ny - 1)), &cells))) return rc;
     SharedBuildArgs a;
     a.nx = b->nx; a.ny = b->ny;
     // the depth's axis pairs and raw values, and the current's raw values,
@@ -856,7 +853,6 @@ int shared_tables(const mr_field *cb, const mr_field *cc, int tl, const SCell **
     a.byspace = (double)b->yf[1] - (double)b->yf[0];
     a.cxspace = cc->xd[1] - cc->xd[0];                      // cartesian_current.rs:512-513
     a.cyspace = cc->yd[1] - cc->yd[0];
-    a.ntx = (int)(ntx << 4 | tl);
     a.cells = cells;
     MR_HIP_TRY(launch_build_shared(a, 0));
     MR_HIP_TRY(hipDeviceSynchronize());
@@ -899,14 +895,13 @@ int own_records(const mr_field *cf, int tl, const DevTables *ct)
     if (!rc) rc = dev_upload(tmp, fx.data(), fx.size(), &dfx);
     if (!rc) rc = dev_upload(tmp, fy.data(), fy.size(), &dfy);
     if (rc) return rc;
-    const int64_t ntx = tiles_along(f->nx, tl), nty = tiles_along(f->ny, tl);
-    const size_t n = (size_t)((ntx * nty) << (2 * tl));
+    const size_t n = (size_t)((f->nx - 1) * (f->ny - 1));
     RecBuildArgs a;
     a.nx = f->nx; a.ny = f->ny;
     a.xp = dxp; a.yp = dyp; a.fx = dfx; a.fy = dfy;
     a.oob_from = first_oob_cell(f->nx, f->ny, (int64_t)f->a.size());
     if (!bathy) a.oob_from = std::min(a.oob_from, first_oob_cell(f->nx, f->ny, (int64_t)f->b.size()));
-    a.ntx = (int)(ntx << 4 | tl);
+    a.ntx = (int)(tiles_along(f->nx, tl) << 4 | tl);
     DCell *dc = nullptr;
     UCell *uc = nullptr;
     if (bathy) {
@@ -929,11 +924,10 @@ int own_records(const mr_field *cf, int tl, const DevTables *ct)
 // DCell.  A larger grid's records would need a 64-bit address per load, about
 // six more vector instructions in every step; such a pair runs on the plain
 // records (REC_NONE) instead.
-int record_mode(const mr_field *b, const mr_field *c, int tl)
+int record_mode(const mr_field *b, const mr_field *c)
 {
-    auto fits = [tl](const mr_field *f, size_t rec) {
-        return (tiles_along(f->nx, tl) * tiles_along(f->ny, tl) << (2 * tl)) * (int64_t)rec <
-               (int64_t(1) << 32);
+    auto fits = [](const mr_field *f, size_t rec) {
+        return (f->nx - 1) * (f->ny - 1) * (int64_t)rec < (int64_t(1) << 32);
     };
     if (shared_cells(b, c) && fits(b, sizeof(SCell))) return REC_SHARED;
     if (b->kind == MR_BATHY_GRID && !fits(b, sizeof(DCell))) return REC_NONE;
@@ -988,7 +982,7 @@ int trace_device(const mr_field *bathy, const mr_field *current, int64_t n_rays,
     a.len_out = len_out;
     a.end_out = end_out;
     a.solout = o.solout;
-    a.records = record_mode(bathy, current, o.record_tile);
+    a.records = record_mode(bathy, current);
     if ((rc = record_tables(bathy, current, o.record_tile, a.records, bt, ct, &a.rec))) return rc;
     const int block = o.block_size ? o.block_size : tuned_block(n_rays);
     if ((n_rays + block - 1) / block >= (int64_t)INT32_MAX)
@@ -1541,7 +1535,7 @@ int mr_batch_create(int32_t n_scenes, const mr_scene *scenes, const mr_options *
             return fail(MR_ERR_INVALID_ARGUMENT, "scenes of one batch must share field kinds");
         // one mode for every scene: combined records where all share cells,
         // plain records where any scene needs them, the fields' own otherwise
-        const int mode = record_mode(sc.bathy, sc.current, o.record_tile);
+        const int mode = record_mode(sc.bathy, sc.current);
         if (i == 0 || b->records == mode) b->records = mode;
         else if (mode == REC_NONE || b->records == REC_NONE) b->records = REC_NONE;
         else b->records = REC_OWN;

@@ -524,6 +524,15 @@ __device__ __forceinline__ double rsq_nr(double x)
     return __builtin_fma(0.5 * y, e, y);
 }
 
+// 2 rsq_nr(x), exactly
+__device__ __forceinline__ double rsq2_nr(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    const double t = x * y;
+    const double e = __builtin_fma(-t, y, 1.0);
+    return __builtin_fma(y, e, y + y);
+}
+
 // 1/sqrt(x) to about an ulp: the same estimate and residual e = 1 - x y^2,
 // with the next term of the series, y (1 + e/2 + 3/8 e^2), whose own error is
 // of order e^3 (1e-21).
@@ -535,60 +544,72 @@ __device__ __forceinline__ double rsq_full(double x)
     return __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
 }
 
-// The f64 constants of the dispersion evaluations.  Kernels copy them
-// into per-lane registers at start (load_view), so that the loop does not
+// The f64 constants of the dispersion evaluations.  Kernels copy them into
+// per-lane registers at start (load_consts), so that the loop does not
 // rebuild each one in a scalar register pair at every use.
 struct FastConsts {
-    double inv_ln2, ln2_hi, ln2_lo;   // 1/ln 2; ln 2 split in two parts
+    double m2_ln2;                    // -2/ln 2
+    double round;                     // 1.5 * 2^52: x + round rounds x to an integer
+    double hln2_hi, hln2_lo;          // (ln 2)/2 split in two parts
     double clamp;                     // |argument| limit of exp_pair
-    double expc[10];                  // expm1(f)/f ~ sum c_j f^j, c_9 first (Horner order)
-    double expl[10];                  // (expm1(f) - f)/f^2, likewise
-    double g, half_g, m2g;            // g, g/2 and -2g
-    double nan;                       // a quiet NaN
+    double expc[10];                  // 2^(j+1) c_j of expm1(f)/f ~ sum c_j f^j, j = 9 first
+    double expl[10];                  // 2^(j+1) c_j of (expm1(f) - f)/f^2, likewise
+    double g, half_g, qg;             // g, g/2, g/4
 };
 
-// e = exp(r) and em = 1 - exp(r) (r <= 0 in use: r = -2kh), each with small
-// relative error, from one reduced-argument evaluation: r = m ln2 + f,
-// |f| <= ln2/2, expm1(f) = f P(f) with P the degree-9 polynomial
-// interpolating expm1(f)/f at the Chebyshev nodes of [-ln2/2, ln2/2] (within
-// 1.8e-15 relative, evaluated in f64), e = 2^m (1 + p), em = (1 - 2^m) -
-// 2^m p, which has no cancellation for m <= -1 and is exactly -p for m = 0.
-// r is clamped to [-1400, 1400], beyond which exp(r) is 0 or overflows in
-// f64 either way; fmin first, so that a NaN r gives exp(+1400) = inf, which
-// makes the callers' results NaN.
-__device__ __forceinline__ void exp_pair(double r, double &e, double &em, const FastConsts &K)
+// The argument reduction of exp(-2q), q in [-700, 700] (beyond, exp is 0 or
+// overflows in f64 either way): -2q = m ln 2 + 2f, |f| <= (ln 2)/4.  The
+// polynomials below are in f with their coefficients scaled by powers of
+// two, which keeps the arithmetic that of exp's own argument without the
+// multiplication by -2.  m is rounded by adding 1.5 * 2^52, whose sum holds
+// it as an integer in its low word.  The lower bound first, so that a NaN q
+// gives exp(1400) = inf, which makes the callers' results NaN.  Returns 2^m.
+__device__ __forceinline__ double exp_reduce(double q, double &f, const FastConsts &K)
 {
-    r = __builtin_fmax(__builtin_fmin(r, K.clamp), -K.clamp);
-    const double m = __builtin_rint(r * K.inv_ln2);
-    double f = __builtin_fma(-m, K.ln2_hi, r);
-    f = __builtin_fma(-m, K.ln2_lo, f);
+    // max(q, -clamp) as -min(-q, clamp): a negated constant would be quieted
+    // again at every use
+    q = __builtin_fmin(-__builtin_fmin(-q, K.clamp), K.clamp);
+    const double t = __builtin_fma(q, K.m2_ln2, K.round);
+    const double m = t - K.round;
+    f = __builtin_fma(-m, K.hln2_hi, -q);
+    f = __builtin_fma(-m, K.hln2_lo, f);
+    return __builtin_ldexp(1.0, (int)(uint32_t)__builtin_bit_cast(uint64_t, t));
+}
+
+// e = exp(-2q) and em = 1 - exp(-2q) (q >= 0 in use: q = kh), each with
+// small relative error, from one reduced-argument evaluation: with F = 2f,
+// expm1(F) = F P(F), P the degree-9 polynomial interpolating expm1(F)/F at
+// the Chebyshev nodes of [-ln2/2, ln2/2] (within 1.8e-15 relative, evaluated
+// in f64), e = 2^m (1 + p), em = (1 - 2^m) - 2^m p, which has no
+// cancellation for m <= -1 and is exactly -p for m = 0.
+__device__ __forceinline__ void exp_pair(double q, double &e, double &em, const FastConsts &K)
+{
+    double f;
+    const double s = exp_reduce(q, f, K);
     double P = K.expc[0];
 #pragma unroll
     for (int j = 1; j < 10; ++j) P = __builtin_fma(P, f, K.expc[j]);
-    const double p = f * P;                             // expm1(f)
-    const double s = __builtin_ldexp(1.0, (int)m);
+    const double p = f * P;                             // expm1(2f)
     e = __builtin_fma(s, p, s);
     em = __builtin_fma(-s, p, 1.0 - s);
 }
 
-// exp_pair to about an ulp: expm1(f) = f + f^2 Q(f) with Q of degree 9
-// interpolating (expm1(f) - f)/f^2 at the Chebyshev nodes of [-ln2/2, ln2/2]
-// (3.7e-17 of expm1(f)), so that only the last addition rounds at the size
-// of the result.
-__device__ __forceinline__ void exp_pair_full(double r, double &e, double &em,
+// exp_pair to about an ulp: expm1(F) = F + F^2 Q(F) with Q of degree 9
+// interpolating (expm1(F) - F)/F^2 at the Chebyshev nodes (3.7e-17 of
+// expm1(F)), so that only the last addition rounds at the size of the
+// result.  p is half of expm1(F).
+__device__ __forceinline__ void exp_pair_full(double q, double &e, double &em,
                                               const FastConsts &K)
 {
-    r = __builtin_fmax(__builtin_fmin(r, K.clamp), -K.clamp);
-    const double m = __builtin_rint(r * K.inv_ln2);
-    double f = __builtin_fma(-m, K.ln2_hi, r);
-    f = __builtin_fma(-m, K.ln2_lo, f);
+    double f;
+    const double s = exp_reduce(q, f, K);
     double Q = K.expl[0];
 #pragma unroll
     for (int j = 1; j < 10; ++j) Q = __builtin_fma(Q, f, K.expl[j]);
-    const double p = __builtin_fma(f * f, Q, f);        // expm1(f)
-    const double s = __builtin_ldexp(1.0, (int)m);
-    e = __builtin_fma(s, p, s);
-    em = __builtin_fma(-s, p, 1.0 - s);
+    const double p = __builtin_fma(f * f, Q, f);
+    const double s2 = s + s;
+    e = __builtin_fma(s2, p, s);
+    em = __builtin_fma(-s2, p, 1.0 - s);
 }
 
 // ---------------------------------------------------------------------------
@@ -628,7 +649,7 @@ __device__ __forceinline__ void odes(const FastConsts &K, double h, double hx, d
         const double k = __builtin_fma(__builtin_fma(-k1, k1, k2), 0.5 * rk, k1);
         const double kh = k * h;
         double e, em;
-        exp_pair_full(-2.0 * kh, e, em, K);
+        exp_pair_full(kh, e, em, K);
         const double gke = (K.g * k) * em;
         const double W = rsq_full(__builtin_fma(gke, e, gke));
         // e/(1+e): from 1/(1+e) to a few ulps, corrected by the residual
@@ -638,7 +659,7 @@ __device__ __forceinline__ void odes(const FastConsts &K, double h, double hx, d
         const double ei = __builtin_fma(i0, __builtin_fma(-e, q, e - q), q);
         const double cgr = ((K.half_g * rk) * W) * __builtin_fma(kh, 4.0 * ei, em);
         // (k twice, not k^2: its rounding then partly cancels that of e's k)
-        const double c = (K.m2g * k) * (k * (ei * W));
+        const double c = (K.g * k) * (k * (-2.0 * (ei * W)));
         dx = __builtin_fma(cgr, kx, u);
         dy = __builtin_fma(cgr, ky, v);
         dkx = __builtin_fma(-ky, vx, __builtin_fma(-kx, ux, c * hx));    // :146-147
@@ -667,15 +688,17 @@ __device__ __forceinline__ void odes(const FastConsts &K, double h, double hx, d
         const double k = k2 * rk;
         const double kh = k * h;
         double e, em;
-        exp_pair(-2.0 * kh, e, em, K);                      // e = exp(-2kh), em = 1 - e
+        exp_pair(kh, e, em, K);                             // e = exp(-2kh), em = 1 - e
         const double ope = 1.0 + e;
         const double gke = (K.g * k) * em;
-        const double W = rsq_nr(gke * ope);
-        const double iope = gke * (W * W);                  // 1/(1+e)
-        const double ei = e * iope;
-        // cg cos(theta)/kx = cg/k, with (g/2)/k formed beside the chain
-        const double cgr = ((K.half_g * rk) * W) * __builtin_fma(4.0 * kh, ei, em);
-        const double c = (K.m2g * k2) * (ei * W);
+        // 2W and 4/(1+e) in the places of W and 1/(1+e), which take the
+        // factors 2 and 4 of the formulas into the constants
+        const double W2 = rsq2_nr(gke * ope);
+        const double iope4 = gke * (W2 * W2);               // 4/(1+e)
+        const double ei4 = e * iope4;
+        // cg cos(theta)/kx = cg/k, with (g/4)/k formed beside the chain
+        const double cgr = ((K.qg * rk) * W2) * __builtin_fma(kh, ei4, em);
+        const double c = (-K.qg * k2) * (ei4 * W2);
         dx = __builtin_fma(cgr, kx, u);                     // cg cos(atan2(ky, kx)) + u
         dy = __builtin_fma(cgr, ky, v);
         // (c hx - kx ux) - ky vx with one rounding per term
@@ -746,6 +769,18 @@ struct RecSlot {
 __device__ __forceinline__ mr_f4 f4of(mr_d2 d)
 {
     return __builtin_bit_cast(mr_f4, d);
+}
+
+// Cell records are stored row-major: their order makes no difference to the
+// loads (a wave's lanes sit in unrelated cells; tiles of 1 x 1 to 32 x 32
+// cells all ran within 1 % on 1023 x 1023 and 1200 x 906 cells), and this
+// index is one instruction of a refill that runs twice in every step (a
+// tiled one ten, a full 32-bit multiply among them).  j and ncx are below
+// 2^24 (the axes' limit), where the 24-bit multiply is exact, and the index
+// fits 32 bits (record_mode).
+__device__ __forceinline__ uint32_t rec_index(int i, int j, int ncx)
+{
+    return __umul24((uint32_t)j, (uint32_t)ncx) + (uint32_t)i;
 }
 
 template <int N, class Rec>
@@ -846,10 +881,9 @@ __device__ __forceinline__ void rhs_rec(const BathyView &B, const BathyPtrs &BP,
     if (CK != CK_GRID) current_query<CK>(C, CP, cs, x, y, u, v, ux, uy, vx, vy);
     odes<MATH>(K, h, hx, hy, true, u, v, ux, uy, vx, vy, kx, ky, dx, dy, dkx, dky);
     if (BK == BK_GRID || CK == CK_GRID) {
-        const bool slow = !(off == 0.0f);
-        if (__builtin_expect(wave_any(slow), 0)) {
+        if (__builtin_expect(__builtin_amdgcn_fcmpf(off, 0.0f, 14) != 0, 0)) {
             __asm__ volatile("");
-            if (slow) {
+            if (!(off == 0.0f)) {
                 const double h2 = bathy_query<BK>(B, BP, bs, x, y, hx, hy);
                 const bool okc = current_query<CK>(C, CP, cs, x, y, u, v, ux, uy, vx, vy);
                 odes<MATH>(K, h2, hx, hy, okc, u, v, ux, uy, vx, vy, kx, ky, dx, dy, dkx, dky);

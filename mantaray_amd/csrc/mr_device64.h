@@ -528,7 +528,7 @@ __device__ __forceinline__ void lin_record(const FastConsts &K, const Val64 &h, 
     const double ex = kx * rk, ey = ky * rk;
     const double q = k * hh;
     double e, em;
-    exp_pair(-2.0 * q, e, em, K);
+    exp_pair(q, e, em, K);
     const double ope = 1.0 + e;
     // one reciprocal square root, W = 1/sqrt(g k (1-e)(1+e)), gives the
     // reciprocal D = 1/((1-e)(1+e)) = g k W^2 and 1/sigma = W (1+e), as
@@ -715,7 +715,7 @@ __device__ __forceinline__ void rhs64_vjp(const Grid64View &B, const Grid64Ptrs 
     const double ex = kx * rk, ey = ky * rk;
     const double q = k * hh;
     double e, em;
-    exp_pair(-2.0 * q, e, em, K);                        // e = exp(-2q), em = 1 - e
+    exp_pair(q, e, em, K);                               // e = exp(-2q), em = 1 - e
     const double ope = 1.0 + e;
     const double D = rcp_nr(em * ope);
     const double iope = em * D;

@@ -62,38 +62,50 @@ __device__ __forceinline__ void settle(const View &v)
 }
 
 static __device__ double mr_fast_consts[sizeof(FastConsts) / sizeof(double)] = {
-    1.4426950408889634,                    // 1/ln 2
-    6.93147180369123816490e-01,            // ln 2 split, upper part
-    1.90821492927058770002e-10,            // ln 2 - upper part
-    1400.0,
-    // expm1(f)/f interpolated at the 10 Chebyshev nodes of [-ln2/2, ln2/2]
-    // (computed in 50-digit arithmetic and rounded), c_9 .. c_0
-    2.7620075879983367e-07,
-    2.7632640675430236e-06,
-    2.4801521322368692e-05,
-    1.984119064754424e-04,
-    1.3888888917196719e-03,
-    8.333333367311603e-03,
-    4.1666666666624164e-02,
-    1.6666666666615648e-01,
-    5.000000000000001e-01,
-    1.0000000000000013,
-    // (expm1(f) - f)/f^2, interpolated likewise, c_9 .. c_0
-    2.5100375832561234e-08,
-    2.7620075879983367e-07,
-    2.7557268480310024e-06,
-    2.4801521322368692e-05,
-    1.9841269863040545e-04,
-    1.3888888917196719e-03,
-    8.333333333330065e-03,
-    4.1666666666624164e-02,
-    1.6666666666666669e-01,
-    5.000000000000001e-01,
+    -2.0 * 1.4426950408889634,             // -2/ln 2
+    0x1.8p52,
+    0.5 * 6.93147180369123816490e-01,      // (ln 2)/2 split, upper part
+    0.5 * 1.90821492927058770002e-10,      // (ln 2)/2 - upper part
+    700.0,
+    // expm1(F)/F interpolated at the 10 Chebyshev nodes of [-ln2/2, ln2/2]
+    // (computed in 50-digit arithmetic and rounded), c_9 .. c_0, each times
+    // 2^(j+1) (exact) for the argument f = F/2
+    2.7620075879983367e-07 * 0x1p10,
+    2.7632640675430236e-06 * 0x1p9,
+    2.4801521322368692e-05 * 0x1p8,
+    0.0001984119064754424 * 0x1p7,
+    0.0013888888917196719 * 0x1p6,
+    0.008333333367311603 * 0x1p5,
+    0.041666666666624164 * 0x1p4,
+    0.16666666666615648 * 0x1p3,
+    0.5000000000000001 * 0x1p2,
+    1.0000000000000013 * 0x1p1,
+    // (expm1(F) - F)/F^2, interpolated likewise
+    2.5100375832561234e-08 * 0x1p10,
+    2.7620075879983367e-07 * 0x1p9,
+    2.7557268480310024e-06 * 0x1p8,
+    2.4801521322368692e-05 * 0x1p7,
+    0.00019841269863040545 * 0x1p6,
+    0.0013888888917196719 * 0x1p5,
+    0.008333333333330065 * 0x1p4,
+    0.041666666666624164 * 0x1p3,
+    0.16666666666666669 * 0x1p2,
+    0.5000000000000001 * 0x1p1,
     G,
     0.5 * G,
-    -2.0 * G,
-    __builtin_nan(""),
+    0.25 * G,
 };
+
+// The constants in per-lane registers, in place before the code that
+// follows.  The clamp goes through an addition, whose result is known to be no
+// signalling NaN: the compiler would quiet a loaded value again in every step.
+__device__ __forceinline__ FastConsts load_consts()
+{
+    FastConsts K = load_view<FastConsts>(mr_fast_consts);
+    settle(K);
+    K.clamp = K.clamp + 0.0;
+    return K;
+}
 
 // t[0] = t0, t[s] = t[s-1] + dt for s <= n
 __device__ __forceinline__ void time_column(double t0, double dt, int64_t n, double *t)

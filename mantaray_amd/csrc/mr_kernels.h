@@ -85,7 +85,6 @@ struct SharedBuildArgs {
     int64_t oob_from;                  // cells from here on have a corner past some array
     double bxspace, byspace;           // (f64)x[1] - (f64)x[0] of the f32 axes (depth slopes)
     double cxspace, cyspace;           // x[1] - x[0] of the f64 axes (current slopes)
-    int ntx;                           // as in BathyBuildArgs
     SCell *cells;
 };
 
@@ -95,7 +94,7 @@ struct RecBuildArgs {
     const float2 *xp, *yp;             // the f32 axis pairs (a[i], a[i+1])
     const float2 *fx, *fy;             // per axis cell: the fast region's (lo, hi)
     int64_t oob_from;                  // cells from here on have a corner past some array
-    int ntx;                           // as in BathyBuildArgs
+    int ntx;                           // the plain records' tiling, as in BathyBuildArgs
 };
 
 struct CurrentBuildArgs {

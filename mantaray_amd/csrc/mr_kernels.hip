@@ -131,7 +131,12 @@ __device__ __forceinline__ void rk4_step(const BathyView &B, const BathyPtrs &BP
 // copied at every other stage and whose reloads the compiler waits for at
 // once: 30,011 rays x 2000 steps of 0.7 s on a 1201 x 907 depth and a 444 x
 // 335 current with trajectories 3.60 -> 2.65 ms, 20,000 rays x 1500 steps on
-// a 1024 x 768 depth under a constant current 1.90 -> 1.44 ms.
+// a 1024 x 768 depth under a constant current 1.90 -> 1.44 ms.  Taking
+// instructions out of the common path (row-major records, the factors 2 and
+// 4 of the dispersion in its constants, the slow test on one compare and
+// branch, the row offset as the step count) then gave 2.55 and 1.36 ms, and
+// 5.60 -> 5.42 ms on 65,536 rays x 5000 steps on shared cells (there the
+// clock drops as the lanes idle less: the load is near the power limit).
 
 // The refill of one slot for the point (gx, gy).  The records' offsets are
 // formed before the tests, in every step: some lane of the wave refills in
@@ -146,13 +151,13 @@ __device__ __forceinline__ void rec_refill(const BathyView &B, const CurrentView
 {
     uint32_t bcell = 0, ccell = 0;
     if (BK == BK_GRID) {
-        bcell = tiled_cell(guess_cell(gx, B.ax0, B.pinv_sx, B.pmax_x),
-                           guess_cell(gy, B.ay0, B.pinv_sy, B.pmax_y), B.ntx);
+        bcell = rec_index(guess_cell(gx, B.ax0, B.pinv_sx, B.pmax_x),
+                          guess_cell(gy, B.ay0, B.pinv_sy, B.pmax_y), B.ncx);
         __asm__ volatile("" : "+v"(bcell));
     }
     if (!SH && CK == CK_GRID) {
-        ccell = tiled_cell(guess_cell(gx, C.px0, C.pinv_sx, C.pmax_x),
-                           guess_cell(gy, C.py0, C.pinv_sy, C.pmax_y), C.ntx);
+        ccell = rec_index(guess_cell(gx, C.px0, C.pinv_sx, C.pmax_x),
+                          guess_cell(gy, C.py0, C.pinv_sy, C.pmax_y), C.ncx);
         __asm__ volatile("" : "+v"(ccell));
     }
     if constexpr (SH) {
@@ -228,8 +233,8 @@ __device__ __forceinline__ void rec_prefetch(const BathyView &B, const CurrentVi
 {
     const float fx = (float)x, fy = (float)y;
     if constexpr (BK == BK_GRID) {
-        const uint32_t cell = tiled_cell(guess_cell(fx, B.ax0, B.pinv_sx, B.pmax_x),
-                                         guess_cell(fy, B.ay0, B.pinv_sy, B.pmax_y), B.ntx);
+        const uint32_t cell = rec_index(guess_cell(fx, B.ax0, B.pinv_sx, B.pmax_x),
+                                        guess_cell(fy, B.ay0, B.pinv_sy, B.pmax_y), B.ncx);
         if constexpr (SH) {
             rec_load(R.scells, sa.d, cell);
             rec_load(R.scells, sb.d, cell);
@@ -239,8 +244,8 @@ __device__ __forceinline__ void rec_prefetch(const BathyView &B, const CurrentVi
         }
     }
     if constexpr (!SH && CK == CK_GRID) {
-        const uint32_t cell = tiled_cell(guess_cell(fx, C.px0, C.pinv_sx, C.pmax_x),
-                                         guess_cell(fy, C.py0, C.pinv_sy, C.pmax_y), C.ntx);
+        const uint32_t cell = rec_index(guess_cell(fx, C.px0, C.pinv_sx, C.pmax_x),
+                                        guess_cell(fy, C.py0, C.pinv_sy, C.pmax_y), C.ncx);
         rec_load(R.ucells, sa.c, cell);
         rec_load(R.ucells, sb.c, cell);
     }
@@ -299,14 +304,13 @@ __global__ void __launch_bounds__(256) trace_kernel(TraceArgs a)
     }
     const BathyView B = load_view<BathyView>(a.B);
     const CurrentView C = load_view<CurrentView>(a.C);
-    const FastConsts K = load_view<FastConsts>(mr_fast_consts);
+    const FastConsts K = load_consts();
     const double half = a.half, dt = a.dt, sixth = a.sixth;
     // the views and constants arrive before the loop: otherwise they count
     // as pending at the loop head, and each step waits for every load and
     // store in flight where it first reads them
     settle(B);
     settle(C);
-    settle(K);
     BathySlot bn;                      // records prefetched for the next evaluation
     CurrentSlot cn;
     RecSlot<BK, CK, SH> sa, sb;        // the two record slots
@@ -365,14 +369,16 @@ __global__ void __launch_bounds__(256) trace_kernel(TraceArgs a)
         const __amdgpu_buffer_rsrc_t bx = row_rsrc(a.xo + row0, 0), by = row_rsrc(a.yo + row0, 1),
                                      bkx = row_rsrc(a.kxo + row0, 2),
                                      bky = row_rsrc(a.kyo + row0, 3);
+        // The block's steps are counted by the row offset itself, in 32 bits:
+        // a count of its own the compiler keeps in a vector register, whose
+        // carry the scalar unit then waits for, and a 64-bit bound it can
+        // test only through a vector compare.  The loops are left by goto
+        // when every lane's ray has ended: a flag tested by the block loop
+        // would keep, in the compiler's view, a path from that exit back into
+        // the step loop.
         uint32_t soff = 0;
-        // the block's steps counted down in 32 bits: the scalar unit tests a
-        // 32-bit count in one instruction, a 64-bit signed bound only through
-        // a vector compare.  The loops are left by goto when every lane's ray
-        // has ended: a flag tested by the block loop would keep, in the
-        // compiler's view, a path from that exit back into the step loop.
-        for (uint32_t left = (uint32_t)(s_end - s + 1); left != 0u;
-             --left, ++s, soff += row_bytes) {
+        const uint32_t soff_end = (uint32_t)(s_end - s + 1) * row_bytes;
+        do {
             const bool live = !__builtin_isnan(m);
             if (__builtin_amdgcn_ballot_w64(live) == 0) goto done;
             if (live) {
@@ -412,7 +418,9 @@ __global__ void __launch_bounds__(256) trace_kernel(TraceArgs a)
                 if (a.kyo) a.kyo[o] = ky;
             }
             so = a.solout;
-        }
+            ++s;
+            soff += row_bytes;
+        } while (soff != soff_end);
     }
 done:
     // rows past the wave's last live step
@@ -447,8 +455,7 @@ __global__ void __launch_bounds__(256) batch_kernel(BatchArgs a)
 {
     constexpr bool PF_B = BK == BK_GRID, PF_C = CK == CK_GRID;
     constexpr bool SH = REC == REC_SHARED;
-    const FastConsts K = load_view<FastConsts>(mr_fast_consts);
-    settle(K);                         // as in trace_kernel
+    const FastConsts K = load_consts();
     const int lane = (int)(threadIdx.x & 63);
     BathyView B{};
     CurrentView C{};
@@ -554,7 +561,7 @@ __global__ void __launch_bounds__(256) rhs_kernel(RhsArgs a)
     double dx, dy, dkx, dky;
     const BathyView B = load_view<BathyView>(a.B);
     const CurrentView C = load_view<CurrentView>(a.C);
-    const FastConsts K = load_view<FastConsts>(mr_fast_consts);
+    const FastConsts K = load_consts();
     BathySlot bs;
     CurrentSlot cs;
     rhs<BK, CK, MATH>(B, a.bp, bs, C, a.cp, cs, K, a.s[4 * i], a.s[4 * i + 1], a.s[4 * i + 2],
@@ -702,7 +709,7 @@ __global__ void build_shared_kernel(SharedBuildArgs a)
         r.vy = (a.v[iB] - a.v[iA]) / a.cyspace;
     }
     region_of(a, i, j, err, r);
-    a.cells[tiled_cell((int)i, (int)j, a.ntx)] = r;
+    a.cells[c] = r;
 }
 
 // A field's own records (DCell, UCell), from its plain records: the same
@@ -720,7 +727,7 @@ __global__ void build_depth_rec_kernel(RecBuildArgs a, const BCell *plain, DCell
     r.a00 = p.a00; r.a10 = p.a10; r.a01 = p.a01; r.a11 = p.a11;
     r.hx = (double)p.hx; r.hy = (double)p.hy;
     region_of(a, i, j, c >= a.oob_from || __builtin_isnan(p.m01), r);
-    cells[t] = r;
+    cells[c] = r;
 }
 
 __global__ void build_current_rec_kernel(RecBuildArgs a, const CCell *plain, const float2 *mtab,
@@ -739,7 +746,7 @@ __global__ void build_current_rec_kernel(RecBuildArgs a, const CCell *plain, con
     r.va00 = p.va00; r.va10 = p.va10; r.va01 = p.va01; r.va11 = p.va11;
     r.ux = p.ux; r.uy = p.uy; r.vx = p.vx; r.vy = p.vy;
     region_of(a, i, j, c >= a.oob_from || __builtin_isnan(m.x), r);
-    cells[t] = r;
+    cells[c] = r;
 }
 
 // ---------------------------------------------------------------------------
