@@ -9,8 +9,6 @@
 //                    respect to the initial states and to the gridded depth,
 //                    u and v values.
 //   rhs64_kernel     WaveRayPath::system in fp64 mode at a batch of states.
-//   build_m64        per-cell change of basis (m01, m10) of interpolator.rs
-//                    :59-72 in f64.
 //   fill             constant fill (gradient grids start at zero).
 //
 // The adjoint is that of the discrete map the forward computes (ode_solvers
@@ -81,11 +79,12 @@ hipError_t adjoint_scratch(void **ptr)
 // old, have landed by then.  Without that wait the compiler waits at the
 // serving slot's first use, after the refill, and as the refill is
 // conditional it cannot count it: it waits for the refill's loads as well.
-template <int BK, int CK, int MATH, int NST>
+template <int BK, int CK, bool SH, int MATH, int NST>
 __device__ __forceinline__ void rk4_step64(const Grid64View &B, const Grid64Ptrs &BP,
                                            const Grid64View &C, const Grid64Ptrs &CP,
-                                           const Fields64 &F, const FastConsts &K, Slots64 &sa,
-                                           Slots64 &sb, double dt, double half, double sixth,
+                                           const Fields64 &F, const FastConsts &K,
+                                           Slots64<BK, CK, SH> &sa, Slots64<BK, CK, SH> &sb,
+                                           double dt, double half, double sixth,
                                            const double s[4], double k[3][4],
                                            double ys[3][4], double o[4])
 {
@@ -98,12 +97,13 @@ __device__ __forceinline__ void rk4_step64(const Grid64View &B, const Grid64Ptrs
         if (st == 1 || st == 3) {
             if (st == 1) vm_wait_upto<NST>();
             else vm_wait_upto<0>();
-            Slots64 &refill = st == 1 ? sa : sb;
+            Slots64<BK, CK, SH> &refill = st == 1 ? sa : sb;
             const double g = st == 1 ? dt : 1.5 * dt;
-            prefetch64<BK, CK>(B, BP, C, CP, F, refill, refill, s[0] + px * g, s[1] + py * g);
+            prefetch64<BK, CK, SH>(B, BP, C, CP, F, refill, refill, __builtin_fma(px, g, s[0]),
+                                   __builtin_fma(py, g, s[1]));
         }
         double dx, dy, dkx, dky;
-        rhs64<BK, CK, MATH>(B, BP, C, CP, F, (st == 0 || st == 3) ? sa : sb, K, sx, sy, skx,
+        rhs64<BK, CK, SH, MATH>(B, BP, C, CP, F, (st == 0 || st == 3) ? sa : sb, K, sx, sy, skx,
                             sky, dx, dy, dkx, dky);
         px = dx; py = dy;
         if (st < 3) {
@@ -117,14 +117,15 @@ __device__ __forceinline__ void rk4_step64(const Grid64View &B, const Grid64Ptrs
         } else {
             ax = ax + dx; ay = ay + dy; akx = akx + dkx; aky = aky + dky;
         }
-        sx = s[0] + dx * hs; sy = s[1] + dy * hs;
-        skx = s[2] + dkx * hs; sky = s[3] + dky * hs;
+        // (one rounding where the reference's f64 step takes two)
+        sx = __builtin_fma(dx, hs, s[0]); sy = __builtin_fma(dy, hs, s[1]);
+        skx = __builtin_fma(dkx, hs, s[2]); sky = __builtin_fma(dky, hs, s[3]);
         if (st < 3) {
             ys[st][0] = sx; ys[st][1] = sy; ys[st][2] = skx; ys[st][3] = sky;
         }
     }
-    o[0] = s[0] + ax * sixth; o[1] = s[1] + ay * sixth;
-    o[2] = s[2] + akx * sixth; o[3] = s[3] + aky * sixth;
+    o[0] = __builtin_fma(ax, sixth, s[0]); o[1] = __builtin_fma(ay, sixth, s[1]);
+    o[2] = __builtin_fma(akx, sixth, s[2]); o[3] = __builtin_fma(aky, sixth, s[3]);
 }
 
 // The work buffer: two halves of [stride][8][work_ld] pairs of doubles.
@@ -170,7 +171,7 @@ constexpr int RECOMPUTE_STORES = 8;
 // holds the state at row c * stride, stored when the step from that row
 // starts; a ray's checkpoints up to its last live step are always written.
 
-template <int BK, int CK, int MATH, int OUT>
+template <int BK, int CK, bool SH, int MATH, int OUT>
 __global__ void __launch_bounds__(256) trace64_kernel(Trace64Args a)
 {
     if ((int)blockIdx.x == a.ray_blocks) {
@@ -193,9 +194,9 @@ __global__ void __launch_bounds__(256) trace64_kernel(Trace64Args a)
     const Grid64View C = load_view<Grid64View>(a.C);
     const FastConsts K = load_consts();
     const double half = a.half, dt = a.dt, sixth = a.sixth;
-    Slots64 sa, sb;                    // the step's two cell slots
-    load_guess64<BK, CK>(B, a.bp, C, a.cp, a.f, sa, s[0], s[1]);
-    load_guess64<BK, CK>(B, a.bp, C, a.cp, a.f, sb, s[0], s[1]);
+    Slots64<BK, CK, SH> sa, sb;                    // the step's two cell slots
+    load_guess64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sa, s[0], s[1]);
+    load_guess64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sb, s[0], s[1]);
     // all of it in registers before the loop, so that the loop head has
     // nothing pending to wait for (as in trace_kernel)
     settle(B);
@@ -222,7 +223,7 @@ __global__ void __launch_bounds__(256) trace64_kernel(Trace64Args a)
             double k[3][4], ys[3][4], n[4];
             // the row stores of the step before are the last operations
             // issued before this step's first refill
-            rk4_step64<BK, CK, MATH, OUT == 1 ? 4 : 0>(B, a.bp, C, a.cp, a.f, K, sa, sb, dt,
+            rk4_step64<BK, CK, SH, MATH, OUT == 1 ? 4 : 0>(B, a.bp, C, a.cp, a.f, K, sa, sb, dt,
                                                        half, sixth, s, k, ys, n);
             // the MR_SOLOUT_NEXT_DERIV test applies from the second step on
             // (solout is asked only after a step)
@@ -275,10 +276,10 @@ __global__ void __launch_bounds__(256) trace64_kernel(Trace64Args a)
 //   z1 = J(Y1)^T kb1
 //   lam <- lam + z1 + z2 + z3 + z4
 // and the field-value cotangents of the four products go to the grids.
-template <int BK, int CK>
+template <int BK, int CK, bool SH>
 __device__ __forceinline__ void rk4_step_adjoint(const Grid64View &B, const Grid64Ptrs &BP,
                                                  const Grid64View &C, const Grid64Ptrs &CP,
-                                                 const Fields64 &F, Slots64 &sn,
+                                                 const Fields64 &F, Slots64<BK, CK, SH> &sn,
                                                  const Grads64 &Gr, Accs64 &acc,
                                                  const FastConsts &K, double dt, double half,
                                                  double sixth, const double s[4],
@@ -298,7 +299,7 @@ __device__ __forceinline__ void rk4_step_adjoint(const Grid64View &B, const Grid
         Y[st][0] = ys[st - 1][0];
         Y[st][1] = ys[st - 1][1];
     }
-    Slots64 sq = sn;
+    Slots64<BK, CK, SH> sq = sn;
 #pragma unroll
     for (int st = 3; st >= 0; --st) {
         double Yk[2];
@@ -315,9 +316,9 @@ __device__ __forceinline__ void rk4_step_adjoint(const Grid64View &B, const Grid
         if (st == 2 || st == 0)
             sq = sn;
         else
-            prefetch64<BK, CK>(B, BP, C, CP, F, sq, sn, Y[st - 1][0], Y[st - 1][1]);
+            prefetch64<BK, CK, SH>(B, BP, C, CP, F, sq, sn, Y[st - 1][0], Y[st - 1][1]);
         double z[4] = {0.0, 0.0, 0.0, 0.0};
-        rhs64_vjp<BK, CK>(B, BP, C, CP, F, sq, Gr, acc, K, Y[st][0], Y[st][1], Yk[0], Yk[1],
+        rhs64_vjp<BK, CK, SH>(B, BP, C, CP, F, sq, Gr, acc, K, Y[st][0], Y[st][1], Yk[0], Yk[1],
                           kb[st][0], kb[st][1], kb[st][2], kb[st][3], z[0], z[1], z[2], z[3]);
         if (st == 0) sn = sq;          // the cells in hand, for the previous step's Y3
         if (st > 0) {
@@ -352,7 +353,7 @@ __device__ __forceinline__ int wave_max(int v)
     return v;
 }
 
-template <int BK, int CK, int MATH>
+template <int BK, int CK, bool SH, int MATH>
 __global__ void __launch_bounds__(ADJ_BLOCK) adjoint_kernel(AdjointArgs a)
 {
     const int64_t nr = a.n_rays;
@@ -374,7 +375,7 @@ __global__ void __launch_bounds__(ADJ_BLOCK) adjoint_kernel(AdjointArgs a)
     const int cmax_r = (active && m >= 1) ? (int)((m - 1) / stride) : -1;
     const int cmax = wave_max(cmax_r);
     if (wave == 0) {
-        Slots64 sa, sb;                                // the step's two cell slots
+        Slots64<BK, CK, SH> sa, sb;                                // the step's two cell slots
         for (int t = 0; t <= cmax + 1; ++t) {
             const int c = cmax - t;
             if (c >= 0 && c <= cmax_r) {
@@ -383,11 +384,11 @@ __global__ void __launch_bounds__(ADJ_BLOCK) adjoint_kernel(AdjointArgs a)
                 double *wk = a.work + (t & 1) * half_work;
                 const double *cp = a.ckpt + ((int64_t)c * 4) * nr + r;
                 double s[4] = {cp[0], cp[nr], cp[2 * nr], cp[3 * nr]};
-                load_guess64<BK, CK>(B, a.bp, C, a.cp, a.f, sa, s[0], s[1]);
-                load_guess64<BK, CK>(B, a.bp, C, a.cp, a.f, sb, s[0], s[1]);
+                load_guess64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sa, s[0], s[1]);
+                load_guess64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sb, s[0], s[1]);
                 for (int j = 0; j < nseg; ++j) {
                     double k[3][4], ys[3][4], n[4];
-                    rk4_step64<BK, CK, MATH, RECOMPUTE_STORES>(B, a.bp, C, a.cp, a.f, K, sa, sb,
+                    rk4_step64<BK, CK, SH, MATH, RECOMPUTE_STORES>(B, a.bp, C, a.cp, a.f, K, sa, sb,
                                                                dt, half, sixth, s, k, ys, n);
                     work_put(wk, ld, r, j, s, ys);
 #pragma unroll
@@ -410,7 +411,7 @@ __global__ void __launch_bounds__(ADJ_BLOCK) adjoint_kernel(AdjointArgs a)
         if (a.g_kx) lam[2] += a.g_kx[o];
         if (a.g_ky) lam[3] += a.g_ky[o];
     }
-    Slots64 sn;                                        // cells for the next evaluation
+    Slots64<BK, CK, SH> sn;                                        // cells for the next evaluation
     Accs64 acc;
     for (int t = 0; t <= cmax + 1; ++t) {
         const int c = cmax - t + 1;
@@ -435,8 +436,8 @@ __global__ void __launch_bounds__(ADJ_BLOCK) adjoint_kernel(AdjointArgs a)
                     work_get(wk, ld, r, j - 1, nxt, [](int) { return true; });
                 }
                 if (j == nseg - 1)     // the sweep starts at the segment's last stage point
-                    prefetch64<BK, CK>(B, a.bp, C, a.cp, a.f, sn, sn, ys[2][0], ys[2][1]);
-                rk4_step_adjoint<BK, CK>(B, a.bp, C, a.cp, a.f, sn, a.grads, acc, K, dt, half,
+                    prefetch64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sn, sn, ys[2][0], ys[2][1]);
+                rk4_step_adjoint<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sn, a.grads, acc, K, dt, half,
                                          sixth, y, ys, lam);
                 const int64_t o = (i0 + j) * nr + r;
                 if (a.g_x) lam[0] += a.g_x[o];
@@ -467,7 +468,7 @@ __global__ void __launch_bounds__(ADJ_BLOCK) adjoint_kernel(AdjointArgs a)
 // step costs about twice a forward step, and each holds a SIMD of its own;
 // once the launch has waves enough to fill every SIMD several times over,
 // one wave doing both takes about a quarter less SIMD time.
-template <int BK, int CK, int MATH>
+template <int BK, int CK, bool SH, int MATH>
 __global__ void __launch_bounds__(64) adjoint_seq_kernel(AdjointArgs a)
 {
     const int64_t nr = a.n_rays;
@@ -499,7 +500,7 @@ __global__ void __launch_bounds__(64) adjoint_seq_kernel(AdjointArgs a)
     }
     // the recomputation's two cell slots; the sweep then uses sa (both are
     // loaded whole at each segment's start)
-    Slots64 sa, sb;
+    Slots64<BK, CK, SH> sa, sb;
     Accs64 acc;
     double *wk = a.work;                               // the first half of the buffer
     for (int c = cmax; c >= 0; --c) {
@@ -509,11 +510,11 @@ __global__ void __launch_bounds__(64) adjoint_seq_kernel(AdjointArgs a)
             // recompute the segment from its checkpoint
             const double *cp = a.ckpt + ((int64_t)c * 4) * nr + r;
             double s[4] = {cp[0], cp[nr], cp[2 * nr], cp[3 * nr]};
-            load_guess64<BK, CK>(B, a.bp, C, a.cp, a.f, sa, s[0], s[1]);
-            load_guess64<BK, CK>(B, a.bp, C, a.cp, a.f, sb, s[0], s[1]);
+            load_guess64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sa, s[0], s[1]);
+            load_guess64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sb, s[0], s[1]);
             for (int j = 0; j < nseg; ++j) {
                 double k[3][4], ys[3][4], n[4];
-                rk4_step64<BK, CK, MATH, RECOMPUTE_STORES>(B, a.bp, C, a.cp, a.f, K, sa, sb, dt,
+                rk4_step64<BK, CK, SH, MATH, RECOMPUTE_STORES>(B, a.bp, C, a.cp, a.f, K, sa, sb, dt,
                                                            half, sixth, s, k, ys, n);
                 work_put(wk, ld, r, j, s, ys);
 #pragma unroll
@@ -535,8 +536,8 @@ __global__ void __launch_bounds__(64) adjoint_seq_kernel(AdjointArgs a)
                     work_get(wk, ld, r, j - 1, nxt, [](int) { return true; });
                 }
                 if (j == nseg - 1)     // the sweep starts at the segment's last stage point
-                    prefetch64<BK, CK>(B, a.bp, C, a.cp, a.f, sa, sa, ys[2][0], ys[2][1]);
-                rk4_step_adjoint<BK, CK>(B, a.bp, C, a.cp, a.f, sa, a.grads, acc, K, dt, half,
+                    prefetch64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sa, sa, ys[2][0], ys[2][1]);
+                rk4_step_adjoint<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sa, a.grads, acc, K, dt, half,
                                          sixth, y, ys, lam);
                 const int64_t o = (i0 + j) * nr + r;
                 if (a.g_x) lam[0] += a.g_x[o];
@@ -591,7 +592,7 @@ __device__ constexpr bool lin_uses(int f)
     return true;
 }
 
-template <int BK, int CK, int MATH, int NL>
+template <int BK, int CK, bool SH, int MATH, int NL>
 __global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs a)
 {
     constexpr int SPW = 4 / NL;                        // stages per linearising wave
@@ -620,7 +621,7 @@ __global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs 
     // per round: the state of one role is then not live across another's
     // code, and registers go to the largest role, not to all of them.
     if (wave == 0) {
-        Slots64 sa, sb;                                // the step's two cell slots
+        Slots64<BK, CK, SH> sa, sb;                                // the step's two cell slots
         double s[4] = {0.0, 0.0, 0.0, 0.0};            // the state being advanced
         for (int rho = 0; rho < rounds; ++rho) {
             const int c = cmax - rho / stride, j = rho % stride;
@@ -630,11 +631,11 @@ __global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs 
                     if (j == 0) {
                         const double *cp = a.ckpt + ((int64_t)c * 4) * nr + r;
                         s[0] = cp[0]; s[1] = cp[nr]; s[2] = cp[2 * nr]; s[3] = cp[3 * nr];
-                        load_guess64<BK, CK>(B, a.bp, C, a.cp, a.f, sa, s[0], s[1]);
-                        load_guess64<BK, CK>(B, a.bp, C, a.cp, a.f, sb, s[0], s[1]);
+                        load_guess64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sa, s[0], s[1]);
+                        load_guess64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sb, s[0], s[1]);
                     }
                     double k[3][4], ys[3][4], n[4];
-                    rk4_step64<BK, CK, MATH, RECOMPUTE_STORES>(B, a.bp, C, a.cp, a.f, K, sa,
+                    rk4_step64<BK, CK, SH, MATH, RECOMPUTE_STORES>(B, a.bp, C, a.cp, a.f, K, sa,
                                                                sb, dt, half, sixth, s, k, ys, n);
                     work_put(a.work + (c & 1) * half_work, ld, r, j, s, ys);
 #pragma unroll
@@ -649,7 +650,7 @@ __global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs 
         // use; 0 for the general case
         auto lin_role = [&](auto wc) {
             constexpr int W = decltype(wc)::value;
-            Slots64 sn;
+            Slots64<BK, CK, SH> sn;
             double nxt[16];                                // the next step's data
             bool pre = false;
             for (int rho = 0; rho < rounds; ++rho) {
@@ -689,14 +690,14 @@ __global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs 
                     // k1 dt = 2 (P[1] - y) (only a guess of where to load)
                     const double bx = W == 2 ? 0.0 : 2.0 * (d[0] - P[1][0]);
                     const double by = W == 2 ? 0.0 : 2.0 * (d[1] - P[1][1]);
-                    Slots64 sq = sn;
+                    Slots64<BK, CK, SH> sq = sn;
                     if (NL == 2) {
                         // the cells of this wave's next point, into sn (see below)
                         if constexpr (W == 1)
-                            prefetch64<BK, CK>(B, a.bp, C, a.cp, a.f, sq, sn, P[1][0] + bx,
+                            prefetch64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, sn, P[1][0] + bx,
                                                P[1][1] + by);
                         else
-                            prefetch64<BK, CK>(B, a.bp, C, a.cp, a.f, sq, sn, P[0][0], P[0][1]);
+                            prefetch64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, sn, P[0][0], P[0][1]);
                     }
                     // start loading the next round's step (same segment)
                     pre = j >= 1;
@@ -714,27 +715,27 @@ __global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs 
                         // not prefetch hold the same cells in both).
                         double R[LIN_N];
                         if constexpr (W == 1) {
-                            rhs64_lin<BK, CK>(B, a.bp, C, a.cp, a.f, sq, K, P[2][0], P[2][1],
+                            rhs64_lin<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, K, P[2][0], P[2][1],
                                               P[2][2], P[2][3], R);
 #pragma unroll
                             for (int f = 0; f < LIN_N; ++f)
-                                if (lin_field_used<BK, CK>(f)) ring[rho & 1][2][f][lane] = R[f];
-                            rhs64_lin<BK, CK>(B, a.bp, C, a.cp, a.f, sq, K, P[1][0], P[1][1],
+                                if (lin_field_used<BK, CK, SH>(f)) ring[rho & 1][2][f][lane] = R[f];
+                            rhs64_lin<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, K, P[1][0], P[1][1],
                                               P[1][2], P[1][3], R);
 #pragma unroll
                             for (int f = 0; f < LIN_N; ++f)
-                                if (lin_field_used<BK, CK>(f)) ring[rho & 1][1][f][lane] = R[f];
+                                if (lin_field_used<BK, CK, SH>(f)) ring[rho & 1][1][f][lane] = R[f];
                         } else {
-                            rhs64_lin<BK, CK>(B, a.bp, C, a.cp, a.f, sq, K, P[3][0], P[3][1],
+                            rhs64_lin<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, K, P[3][0], P[3][1],
                                               P[3][2], P[3][3], R);
 #pragma unroll
                             for (int f = 0; f < LIN_N; ++f)
-                                if (lin_field_used<BK, CK>(f)) ring[rho & 1][3][f][lane] = R[f];
-                            rhs64_lin<BK, CK>(B, a.bp, C, a.cp, a.f, sn, K, P[0][0], P[0][1],
+                                if (lin_field_used<BK, CK, SH>(f)) ring[rho & 1][3][f][lane] = R[f];
+                            rhs64_lin<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sn, K, P[0][0], P[0][1],
                                               P[0][2], P[0][3], R);
 #pragma unroll
                             for (int f = 0; f < LIN_N; ++f)
-                                if (lin_field_used<BK, CK>(f)) ring[rho & 1][0][f][lane] = R[f];
+                                if (lin_field_used<BK, CK, SH>(f)) ring[rho & 1][0][f][lane] = R[f];
                         }
                     } else {
                         // this wave's stages, latest first (the wave selects values,
@@ -750,7 +751,7 @@ __global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs 
                                        : st == 2 ? P[2][q]
                                        : st == 1 ? P[1][q]
                                                  : P[0][q];
-                            Slots64 sq = sn;
+                            Slots64<BK, CK, SH> sq = sn;
                             // the next point: this wave's next stage, or, after its
                             // last, its first stage one step earlier (guessed one
                             // step back along k1)
@@ -767,12 +768,12 @@ __global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs 
                                 gx = fx + bx;
                                 gy = fy + by;
                             }
-                            prefetch64<BK, CK>(B, a.bp, C, a.cp, a.f, sq, sn, gx, gy);
+                            prefetch64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, sn, gx, gy);
                             double R[LIN_N];
-                            rhs64_lin<BK, CK>(B, a.bp, C, a.cp, a.f, sq, K, Y[0], Y[1], Y[2], Y[3], R);
+                            rhs64_lin<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, K, Y[0], Y[1], Y[2], Y[3], R);
 #pragma unroll
                             for (int f = 0; f < LIN_N; ++f)
-                                if (lin_field_used<BK, CK>(f)) ring[rho & 1][st][f][lane] = R[f];
+                                if (lin_field_used<BK, CK, SH>(f)) ring[rho & 1][st][f][lane] = R[f];
                         }
                     }
                 } else {
@@ -815,7 +816,7 @@ __global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs 
                     double Rn[LIN_N];
 #pragma unroll
                     for (int f = 0; f < LIN_N; ++f)
-                        Rn[f] = lin_field_used<BK, CK>(f) ? ring[(rho - 1) & 1][3][f][lane] : 0.0;
+                        Rn[f] = lin_field_used<BK, CK, SH>(f) ? ring[(rho - 1) & 1][3][f][lane] : 0.0;
 #pragma unroll
                     for (int st = 3; st >= 0; --st) {
                         double R[LIN_N];
@@ -824,11 +825,11 @@ __global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs 
                         if (st > 0) {
 #pragma unroll
                             for (int f = 0; f < LIN_N; ++f)
-                                Rn[f] = lin_field_used<BK, CK>(f)
+                                Rn[f] = lin_field_used<BK, CK, SH>(f)
                                             ? ring[(rho - 1) & 1][st - 1][f][lane] : 0.0;
                         }
                         double z[4];
-                        lin_apply<BK, CK>(R, B, C, a.grads, acc, kb[st], z);
+                        lin_apply<BK, CK, SH>(R, B, C, a.grads, acc, kb[st], z);
                         if (st > 0) {
                             const double hs = st < 3 ? half : dt;
 #pragma unroll
@@ -869,26 +870,10 @@ __global__ void __launch_bounds__(256) rhs64_kernel(Rhs64Args a)
     const Grid64View C = load_view<Grid64View>(a.C);
     const FastConsts K = load_consts();
     double dx, dy, dkx, dky;
-    Slots64 sl;                        // empty: the query loads the cell
-    rhs64<BK, CK, MATH>(B, a.bp, C, a.cp, a.f, sl, K, a.s[4 * i], a.s[4 * i + 1], a.s[4 * i + 2],
+    Slots64<BK, CK, false> sl;                        // empty: the query loads the cell
+    rhs64<BK, CK, false, MATH>(B, a.bp, C, a.cp, a.f, sl, K, a.s[4 * i], a.s[4 * i + 1], a.s[4 * i + 2],
                         a.s[4 * i + 3], dx, dy, dkx, dky);
     a.ds[4 * i] = dx; a.ds[4 * i + 1] = dy; a.ds[4 * i + 2] = dkx; a.ds[4 * i + 3] = dky;
-}
-
-// per-cell (m01, m10) of interpolator.rs:59-72 in f64, on the corners
-// A = (x_i, y_j), B = (x_i, y_j+1), D = (x_i+1, y_j); NaN marks det == 0
-__global__ void build_m64_kernel(M64BuildArgs a)
-{
-    const int64_t ncx = a.nx - 1;
-    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ncx * (a.ny - 1)) return;
-    const int64_t i = c % ncx, j = c / ncx;
-    const double Ax = a.ax[i], Ay = a.ay[j];
-    const double btx = Ax - Ax, bty = a.ay[j + 1] - Ay;
-    const double dtx = a.ax[i + 1] - Ax, dty = Ay - Ay;
-    const double det = (btx * dty) - (dtx * bty);
-    a.m[c] = det == 0.0 ? make_double2(MR_NAN, MR_NAN)
-                        : make_double2(-(dtx / det), -(bty / det));
 }
 
 __global__ void fill_kernel(double *p, int64_t n, double v)
@@ -901,6 +886,19 @@ __global__ void fill_kernel(double *p, int64_t n, double v)
 // ---------------------------------------------------------------------------
 // launchers
 
+// dispatch_kinds with f(kinds, shared): shared (a compile-time flag) when
+// depth and current are both gridded and on the same axes
+template <class F>
+static void dispatch_kinds64(int bk, int ck, int math, bool shared, F &&f)
+{
+    dispatch_kinds(bk, ck, math, [&](auto k) {
+        using K = decltype(k);
+        if constexpr (K::bk == BK_GRID && K::ck == CK_GRID)
+            if (shared) return f(k, std::true_type{});
+        f(k, std::false_type{});
+    });
+}
+
 hipError_t launch_trace64(const Trace64Args &a, int bk, int ck, int math, int block,
                           hipStream_t stream)
 {
@@ -910,16 +908,17 @@ hipError_t launch_trace64(const Trace64Args &a, int bk, int ck, int math, int bl
     const dim3 grid((unsigned)(a.ray_blocks + (a.t_out ? 1 : 0)));
     const int nout = (a.xo != nullptr) + (a.yo != nullptr) + (a.kxo != nullptr) +
                      (a.kyo != nullptr);
-    dispatch_kinds(bk, ck, math, [&](auto k) {
+    dispatch_kinds64(bk, ck, math, a.shared != 0, [&](auto k, auto sh) {
         using KK = decltype(k);
+        constexpr bool SH = decltype(sh)::value;
         if (nout == 0)
-            hipLaunchKernelGGL((trace64_kernel<KK::bk, KK::ck, KK::math, 0>), grid, dim3(block),
+            hipLaunchKernelGGL((trace64_kernel<KK::bk, KK::ck, SH, KK::math, 0>), grid, dim3(block),
                                0, stream, a);
         else if (nout == 4)
-            hipLaunchKernelGGL((trace64_kernel<KK::bk, KK::ck, KK::math, 1>), grid, dim3(block),
+            hipLaunchKernelGGL((trace64_kernel<KK::bk, KK::ck, SH, KK::math, 1>), grid, dim3(block),
                                0, stream, a);
         else
-            hipLaunchKernelGGL((trace64_kernel<KK::bk, KK::ck, KK::math, 2>), grid, dim3(block),
+            hipLaunchKernelGGL((trace64_kernel<KK::bk, KK::ck, SH, KK::math, 2>), grid, dim3(block),
                                0, stream, a);
     });
     return hipGetLastError();
@@ -932,16 +931,17 @@ hipError_t launch_adjoint(const AdjointArgs &a, int bk, int ck, int math, int wa
     if (a.stride <= 0 || a.work_ld < a.n_rays) return hipErrorInvalidValue;
     if (waves != 1 && waves != 2 && waves != 4) return hipErrorInvalidValue;
     const dim3 grid((unsigned)((a.n_rays + 63) / 64));    // 64 rays per workgroup
-    dispatch_kinds(bk, ck, math, [&](auto k) {
+    dispatch_kinds64(bk, ck, math, a.shared != 0, [&](auto k, auto sh) {
         using KK = decltype(k);
+        constexpr bool SH = decltype(sh)::value;
         if (waves == 4)
-            hipLaunchKernelGGL((adjoint_lin_kernel<KK::bk, KK::ck, KK::math, 2>), grid,
+            hipLaunchKernelGGL((adjoint_lin_kernel<KK::bk, KK::ck, SH, KK::math, 2>), grid,
                                dim3(4 * 64), 0, stream, a);
         else if (waves == 2)
-            hipLaunchKernelGGL((adjoint_kernel<KK::bk, KK::ck, KK::math>), grid,
+            hipLaunchKernelGGL((adjoint_kernel<KK::bk, KK::ck, SH, KK::math>), grid,
                                dim3(ADJ_BLOCK), 0, stream, a);
         else
-            hipLaunchKernelGGL((adjoint_seq_kernel<KK::bk, KK::ck, KK::math>), grid, dim3(64),
+            hipLaunchKernelGGL((adjoint_seq_kernel<KK::bk, KK::ck, SH, KK::math>), grid, dim3(64),
                                0, stream, a);
     });
     return hipGetLastError();
@@ -957,16 +957,6 @@ hipError_t launch_rhs64(const Rhs64Args &a, int bk, int ck, int math, hipStream_
         hipLaunchKernelGGL((rhs64_kernel<KK::bk, KK::ck, KK::math>), grid, dim3(block), 0, stream,
                            a);
     });
-    return hipGetLastError();
-}
-
-hipError_t launch_build_m64(const M64BuildArgs &a, hipStream_t stream)
-{
-    const int64_t ncell = (a.nx - 1) * (a.ny - 1);
-    if (ncell <= 0) return hipSuccess;
-    const int block = 256;
-    hipLaunchKernelGGL(build_m64_kernel, dim3((unsigned)((ncell + block - 1) / block)),
-                       dim3(block), 0, stream, a);
     return hipGetLastError();
 }
 

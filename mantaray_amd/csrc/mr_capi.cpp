@@ -313,19 +313,27 @@ std::vector<double2> axis_cells64(const std::vector<double> &a)
     return c;
 }
 
-// per-cell fast thresholds of the fp64 mode: the f64 index's cell
-// [T[i], T[i+1]) narrowed to the open node interval (a[i], a[i+1]), so that a
-// target inside on both axes is in the cell and on none of its node lines
-// (an interval that comes out empty holds no target: every target of that
-// cell then takes the full query)
-std::vector<double2> axis_fast64(const std::vector<double> &a)
+// per-cell axis data of the fp64 mode (AxisCell64)
+std::vector<AxisCell64> axis_cells_fp64(const std::vector<double> &a)
 {
     const std::vector<double> t = thresholds64(a);
-    std::vector<double2> c(a.size() - 1);
-    for (size_t i = 0; i + 1 < a.size(); i++)
-        c[i] = make_double2(std::max(t[i], std::nextafter(a[i], INFINITY)),
-                            std::min(t[i + 1], a[i + 1]));
+    std::vector<AxisCell64> c(a.size() - 1);
+    for (size_t i = 0; i + 1 < a.size(); i++) {
+        c[i].lo = std::max(t[i], std::nextafter(a[i], INFINITY));
+        c[i].hi = std::min(std::nextafter(t[i + 1], -INFINITY), std::nextafter(a[i + 1], -INFINITY));
+        c[i].a = a[i];
+        c[i].r = 1.0 / (a[i + 1] - a[i]);
+    }
     return c;
+}
+
+// smallest nonzero cell size along an axis
+double smallest_cell(const std::vector<double> &a)
+{
+    double m = INFINITY;
+    for (size_t i = 0; i + 1 < a.size(); i++)
+        if (a[i + 1] != a[i]) m = std::min(m, std::fabs(a[i + 1] - a[i]));
+    return m;
 }
 
 std::vector<float2> axis_pairs(const std::vector<float> &a)
@@ -542,37 +550,29 @@ int build64(const mr_field &f, DevTables &t)
         v.oob_from = (uint32_t)(bathy ? first_oob_cell(f.nx, f.ny, (int64_t)f.a.size())
                                       : std::min(first_oob_cell(f.nx, f.ny, (int64_t)f.a.size()),
                                                  first_oob_cell(f.nx, f.ny, (int64_t)f.b.size())));
-        v.last_a = (uint32_t)std::max<int64_t>(0, (int64_t)f.a.size() - 1);
-        v.last_b = (uint32_t)std::max<int64_t>(0, (int64_t)f.b.size() - 1);
         v.gx0 = (float)ax[0]; v.gy0 = (float)ay[0];
         v.ginv_x = (float)v.inv_sx; v.ginv_y = (float)v.inv_sy;
         v.gmax_x = (float)(f.nx - 2); v.gmax_y = (float)(f.ny - 2);
-        // the fast thresholds of the f64 index (p - a0)/|a1 - a0| on these
-        // axes, and the node pairs of each cell
-        std::vector<double2> xt = axis_fast64(ax), yt = axis_fast64(ay);
-        std::vector<double2> xp(ax.size() - 1), yp(ay.size() - 1);
-        for (size_t i = 0; i + 1 < ax.size(); i++) xp[i] = make_double2(ax[i], ax[i + 1]);
-        for (size_t i = 0; i + 1 < ay.size(); i++) yp[i] = make_double2(ay[i], ay[i + 1]);
+        std::vector<AxisCell64> xc = axis_cells_fp64(ax), yc = axis_cells_fp64(ay);
+        // cells whose determinant underflows err as det == 0: no fast
+        // intervals then, so that the full query decides
+        if (smallest_cell(ax) * smallest_cell(ay) == 0.0)
+            for (AxisCell64 &c : xc) c.lo = c.hi = NAN;
         double *dax, *day;
-        double2 *dm, *dxt, *dyt, *dxp, *dyp;
+        AxisCell64 *dxc, *dyc;
         int rc = dev_upload(t, ax.data(), ax.size(), &dax);
         if (!rc) rc = dev_upload(t, ay.data(), ay.size(), &day);
-        if (!rc) rc = dev_upload(t, xt.data(), xt.size(), &dxt);
-        if (!rc) rc = dev_upload(t, yt.data(), yt.size(), &dyt);
-        if (!rc) rc = dev_upload(t, xp.data(), xp.size(), &dxp);
-        if (!rc) rc = dev_upload(t, yp.data(), yp.size(), &dyp);
-        if (!rc) rc = dev_alloc(t, (size_t)((f.nx - 1) * (f.ny - 1)), &dm);
+        if (!rc) rc = dev_upload(t, xc.data(), xc.size(), &dxc);
+        if (!rc) rc = dev_upload(t, yc.data(), yc.size(), &dyc);
         if (rc) return rc;
-        M64BuildArgs ma;
-        ma.nx = f.nx; ma.ny = f.ny; ma.ax = dax; ma.ay = day; ma.m = dm;
-        MR_HIP_TRY(launch_build_m64(ma, 0));
-        t.p64.xt = dxt; t.p64.yt = dyt; t.p64.xp = dxp; t.p64.yp = dyp; t.p64.m = dm;
+        t.p64.xc = dxc; t.p64.yc = dyc; t.p64.xn = dax; t.p64.yn = day;
     }
     Grid64View *dv;
     int rc = dev_upload(t, &v, 1, &dv);
     if (rc) return rc;
     MR_HIP_TRY(hipDeviceSynchronize());
     t.view64 = dv;
+    t.p64.view = dv;
     return MR_OK;
 }
 
@@ -665,6 +665,19 @@ int tuned_block(int64_t n_rays)
     return (int)(64 * waves);
 }
 
+// true when a gridded depth and a gridded current have the same f64 axes, so
+// that the fp64 kernels hold one cell for both
+bool same_axes64(const mr_field *b, const mr_field *c)
+{
+    if (b->kind != MR_BATHY_GRID || c->kind != MR_CURRENT_GRID) return false;
+    auto same = [](const std::vector<float> &f, const std::vector<double> &d) {
+        return f.size() == d.size() &&
+               std::equal(f.begin(), f.end(), d.begin(),
+                          [](float p, double q) { return (double)p == q; });
+    };
+    return same(b->xf, c->xd) && same(b->yf, c->yd);
+}
+
 // mr_rhs_many in fp64 mode
 int rhs64_many(const mr_field *bathy, const mr_field *current, int64_t n, const double *s,
                double *ds, const mr_options &o)
@@ -737,6 +750,7 @@ int trace64_device(const mr_field *bathy, const mr_field *current, const double 
     a.solout = o.solout;
     a.stride = stride;
     a.ckpt = ckpt;
+    a.shared = same_axes64(bathy, current) ? 1 : 0;
     const int block = o.block_size ? o.block_size : tuned_block(n_rays);
     if ((n_rays + block - 1) / block >= (int64_t)INT32_MAX)
         return fail(MR_ERR_UNSUPPORTED, "too many rays for one launch");
@@ -1142,6 +1156,7 @@ int adjoint_run(const mr_field *bathy, const mr_field *current, const double *de
     a.grads.depth = g_depth;
     a.grads.u = g_u;
     a.grads.v = g_v;
+    a.shared = same_axes64(bathy, current) ? 1 : 0;
     MR_HIP_TRY(launch_adjoint(a, bathy_kind_of(bathy), current_kind_of(current), o.math, waves,
                               stream));
     return MR_OK;

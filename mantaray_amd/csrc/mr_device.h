@@ -846,6 +846,26 @@ __device__ __forceinline__ float rec_fast(const RecSlot<BK, CK, SH> &s, double x
     return off;
 }
 
+// Copy a field view from device memory into per-lane registers.  The loads
+// go through a lane-varying (always zero) offset so they are vector loads
+// and the view lives in VGPRs for the whole kernel: the scalar register file
+// cannot hold both views next to the loop's own scalars, and re-reading
+// them with scalar loads puts a load latency into every evaluation.
+template <class View>
+__device__ __forceinline__ View load_view(const void *p)
+{
+    static_assert(sizeof(View) % 4 == 0, "view size");
+    int zero;
+    __asm__ volatile("v_mov_b32 %0, 0" : "=v"(zero));
+    const int *src = reinterpret_cast<const int *>(p) + zero;
+    int buf[sizeof(View) / 4];
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(View) / 4); ++i) buf[i] = src[i];
+    View v;
+    __builtin_memcpy(&v, buf, sizeof(View));
+    return v;
+}
+
 // Whether any lane of the wave has c, as a wave-uniform value the compiler
 // cannot fold back into c (the empty asm).  A rare block guarded as
 //   if (__builtin_expect(wave_any(c), 0)) { __asm__ volatile(""); if (c) ... }

@@ -12,20 +12,22 @@
 //
 //   index   (p - a0) / |a1 - a0|         (cartesian_current.rs:244, in f64)
 //   cell    floor, or n-2 on the last node (cartesian_current.rs:283-339)
-//   value   ((a00 + a10 u) + a01 w) + (a11 u) w, u = m01 (y - y_j),
-//           w = m10 (x - x_i)               (interpolator.rs:59-83, in f64)
+//   value   ((a00 + a10 u) + a01 w) + (a11 u) w, u = (y - y_j) RN(1/(y_j+1 - y_j)),
+//           w = (x - x_i) RN(1/(x_i+1 - x_i))   (interpolator.rs:59-83, in f64)
 //   slopes  (D - A) RN(1/(x1 - x0)), (B - A) RN(1/(y1 - y0))
 //
-//   (the slopes are the cell difference times the rounded reciprocal of the
-//   signed spacing, within an ulp of the reference's quotient)
+//   (the change of basis m01 = -dtx/det, m10 = -bty/det with det = -dtx bty
+//   is the reciprocal of the cell's size along each axis, here rounded once;
+//   the slopes are the cell difference times the rounded reciprocal of the
+//   signed first spacing, within an ulp of the reference's quotient)
 //
 // Field values come from kernel arguments (pointers to the raw f64 arrays),
 // so a caller can differentiate with respect to them and change them between
-// calls without rebuilding anything; what depends only on the axes (cell
-// thresholds, node pairs, the change of basis m01, m10) is tabulated once per
-// field.  As in the reference mode, each lane holds cells in registers (a
-// Slot64 per field) and loads the cell a coming evaluation will most likely
-// need ahead of it.
+// calls without rebuilding anything; what depends only on the axes (an
+// AxisCell64 per axis cell) is tabulated once per field.  As in the reference
+// mode, each lane holds cells in registers (a Slot64 per field, or one for
+// both where they lie on the same grid) and loads the cell a coming
+// evaluation will most likely need ahead of it.
 //
 // Linearisation.  With u, w the bilinear fractions of the query, the value is
 //   v = wA A + wB B + wC C + wD D,  wA = (1-u)(1-w), wB = u(1-w), wC = u w,
@@ -56,7 +58,6 @@ struct Grid64View {
     int nx, ny, ncx;                      // grid; ncx = nx - 1
     int an;                               // ArrayDepth (an x an)
     uint32_t oob_from;                    // first cell (row-major) with a corner past the data
-    uint32_t last_a, last_b;              // last index of each value array
     double a0x, a0y;                      // first coordinate of each axis
     double sx, sy, inv_sx, inv_sy;        // |a1 - a0| and RN(1/|a1 - a0|)
     double nxm1, nym1;                    // n - 1
@@ -67,13 +68,24 @@ struct Grid64View {
     float gmax_x, gmax_y;                 // (f32)(n - 2)
 };
 
+// What a query needs of cell i along one axis.  [lo, hi] is the cell's fast
+// interval: the f64 index's cell [T[i], T[i+1]) narrowed to the open interval
+// between the cell's nodes (a[i], a[i+1]), both ends included (empty as lo >
+// hi or NaN).  A target inside on both axes is in the cell and on none of
+// its node lines, so the bilinear value needs neither the corner exit nor
+// the det == 0 exit; other targets of the cell (rare: the node coordinates
+// themselves, and cells that err) take the full query.
+struct AxisCell64 {                       // 32 B
+    double lo, hi;
+    double a, r;                          // a[i]; RN(1/(a[i+1] - a[i]))
+};
+
 // Device arrays of a field in fp64 mode (kernel arguments).
 struct Grid64Ptrs {
-    const double2 *xt, *yt;               // per axis cell i: fast thresholds, [T[i], T[i+1])
-                                          // narrowed to the open node interval
-    const double2 *xp, *yp;               // per axis cell i: (a[i], a[i+1]) in f64
-    const double2 *m;                     // per cell, row-major: (m01, m10); NaN m01 marks det == 0
+    const AxisCell64 *xc, *yc;            // per axis cell
+    const double *xn, *yn;                // node coordinates
     const float *arr;                     // ArrayDepth values
+    const void *view;                     // the field's Grid64View, for the full queries
 };
 
 // A gridded value at a point with what its derivatives need.
@@ -90,24 +102,17 @@ struct Cell64 {
     double u, w;
 };
 
-// One cell of a gridded field held per lane: its fast thresholds, node
-// coordinates, change of basis, and the four corners of NV value arrays
-// (depth; or u and v).  The fast thresholds of cell i on an axis are the
-// f64 index's cell [T[i], T[i+1]) narrowed to the open interval between the
-// cell's nodes (a[i], a[i+1]): a target inside them on both axes is in the
-// cell and on none of its node lines, so the bilinear value needs neither
-// the corner exit nor the node case of the det == 0 exit.  Targets of the
-// cell on a node line (rare: the node coordinates themselves) take the full
-// query, which locates them by the index.  valid is false for a cell with a
-// corner past the data and for a slot never loaded; thresholds start as NaN,
-// so such a slot contains no point.
+// One cell held per lane: its axis cells and the four corners of NV value
+// arrays (depth; u and v; or all three), as the pairs (A, D) and (B, C) that
+// lie next to each other in memory.  A slot holds only cells whose corners
+// all lie in the data; one never loaded has NaN intervals, which contain no
+// point.
 template <int NV>
 struct Slot64 {
-    double2 tx = {MR_NAN_INIT, MR_NAN_INIT}, ty = {MR_NAN_INIT, MR_NAN_INIT};
-    double2 xp = {0.0, 0.0}, yp = {0.0, 0.0}, m = {0.0, 0.0};
-    double v[NV][4] = {};                 // A, B, C, D
+    mr_d2 xt = {MR_NAN_INIT, MR_NAN_INIT}, yt = {MR_NAN_INIT, MR_NAN_INIT};   // (lo, hi)
+    mr_d2 xa = {0.0, 0.0}, ya = {0.0, 0.0};                                   // (a, r)
+    mr_d2 ad[NV] = {}, bc[NV] = {};
     uint32_t iA = 0;
-    bool valid = false;
 };
 
 // Cell of (x, y), or ok = false where the reference's index or corner
@@ -126,115 +131,131 @@ __device__ __forceinline__ bool locate64(const Grid64View &G, double x, double y
     return ok;
 }
 
-template <int NV>
-__device__ __forceinline__ bool slot64_inside(const Slot64<NV> &s, double x, double y)
+// How far (x, y) is outside the slot's fast interval, as a word that is
+// below OUT64 exactly inside: the distances to the four bounds are all
+// non-negative and finite there, and the high words of negative, infinite
+// and NaN doubles are all at or above 0x7ff00000.  (Four f64 compares and
+// the scalar ANDs of their masks took longer; f64 min and max would have
+// their loaded operands quieted first.)
+constexpr uint32_t OUT64 = 0x7ff00000u;
+
+__device__ __forceinline__ uint32_t hi_word(double v)
 {
-    return s.valid & (x >= s.tx.x) & (x < s.tx.y) & (y >= s.ty.x) & (y < s.ty.y);
+    return (uint32_t)(__builtin_bit_cast(uint64_t, v) >> 32);
 }
 
-// Start loading cell (i1, j1) into s.  Corner indices are clamped into the
-// value arrays, so a cell with a corner past the data (never valid) loads
-// in-bounds values that are never used.
+template <int NV>
+__device__ __forceinline__ uint32_t off_slot64(const Slot64<NV> &s, double x, double y)
+{
+    const uint32_t a = hi_word(x - s.xt.x), b = hi_word(s.xt.y - x);
+    const uint32_t c = hi_word(y - s.yt.x), d = hi_word(s.yt.y - y);
+    return __builtin_elementwise_max(__builtin_elementwise_max(a, b),
+                                     __builtin_elementwise_max(c, d));
+}
+
+// two neighbouring values of an array
+__device__ __forceinline__ mr_d2 gld_pair(const double *p, uint32_t i)
+{
+    typedef double pair __attribute__((ext_vector_type(2), aligned(8)));
+    return *(const MR_GLOBAL pair *)((const MR_GLOBAL char *)p + i * 8u);
+}
+
+// Start loading cell (i1, j1) into s, for a cell whose corners lie in the
+// data; vals: the NV value arrays.
 template <int NV>
 __device__ __forceinline__ void slot64_load(const Grid64View &G, const Grid64Ptrs &P,
-                                            const double *va, const double *vb, Slot64<NV> &s,
+                                            const double *const (&vals)[NV], Slot64<NV> &s,
                                             int i1, int j1)
 {
-    const uint32_t cell = (uint32_t)j1 * (uint32_t)G.ncx + (uint32_t)i1;
-    s.tx = gldd2(P.xt, (uint32_t)i1 * 16u);
-    s.ty = gldd2(P.yt, (uint32_t)j1 * 16u);
-    s.xp = gldd2(P.xp, (uint32_t)i1 * 16u);
-    s.yp = gldd2(P.yp, (uint32_t)j1 * 16u);
-    s.m = gldd2(P.m, cell * 16u);
-    const uint32_t iA = (uint32_t)G.nx * (uint32_t)j1 + (uint32_t)i1;
-    const uint32_t idx[4] = {iA, iA + (uint32_t)G.nx, iA + (uint32_t)G.nx + 1u, iA + 1u};
+    const MR_GLOBAL mr_d2 *xc =
+        (const MR_GLOBAL mr_d2 *)((const MR_GLOBAL char *)P.xc + (uint32_t)i1 * 32u);
+    const MR_GLOBAL mr_d2 *yc =
+        (const MR_GLOBAL mr_d2 *)((const MR_GLOBAL char *)P.yc + (uint32_t)j1 * 32u);
+    s.xt = xc[0];
+    s.xa = xc[1];
+    s.yt = yc[0];
+    s.ya = yc[1];
+    const uint32_t iA = __umul24((uint32_t)G.nx, (uint32_t)j1) + (uint32_t)i1;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        s.v[0][c] = gld(va, __builtin_elementwise_min(idx[c], G.last_a));
-        if (NV > 1) s.v[NV - 1][c] = gld(vb, __builtin_elementwise_min(idx[c], G.last_b));
+    for (int q = 0; q < NV; ++q) {
+        s.ad[q] = gld_pair(vals[q], iA);
+        s.bc[q] = gld_pair(vals[q], iA + (uint32_t)G.nx);
     }
     s.iA = iA;
-    s.valid = cell < G.oob_from;
 }
 
 // Start loading the cell that (x, y) most likely lies in (guessed in f32,
-// clamped into the grid; used only to choose what to load).
+// clamped into the grid; used only to choose what to load), unless a corner
+// of it is past the data (oob: the first such cell).
 template <int NV>
 __device__ __forceinline__ void slot64_prefetch(const Grid64View &G, const Grid64Ptrs &P,
-                                                const double *va, const double *vb,
+                                                const double *const (&vals)[NV], uint32_t oob,
                                                 Slot64<NV> &s, double x, double y)
 {
     const int i1 = guess_cell((float)x, G.gx0, G.ginv_x, G.gmax_x);
     const int j1 = guess_cell((float)y, G.gy0, G.ginv_y, G.gmax_y);
-    slot64_load<NV>(G, P, va, vb, s, i1, j1);
+    if (__umul24((uint32_t)j1, (uint32_t)G.ncx) + (uint32_t)i1 < oob)
+        slot64_load<NV>(G, P, vals, s, i1, j1);
 }
 
-// Make s hold the cell of (x, y): lanes whose slot does not contain the
-// point locate it (the reference's f64 index) and load it, then wait.
-// Returns false where the reference's lookup errs.
-template <int NV>
-__device__ __forceinline__ bool slot64_query(const Grid64View &G, const Grid64Ptrs &P,
-                                             const double *va, const double *vb, Slot64<NV> &s,
-                                             double x, double y)
+// interpolator::bilinear in f64 on a cell (ad, bc: its corners; (x0, rx),
+// (y0, ry): its origin and reciprocal sizes), without its exits, and the
+// cell-difference slopes.
+__device__ __forceinline__ Val64 cell64_value(const Grid64View &G, mr_d2 ad, mr_d2 bc, mr_d2 xa,
+                                              mr_d2 ya, double u, double w)
 {
-    bool ok = slot64_inside(s, x, y);
-    if (__any(!ok)) {
-        const bool miss = !ok;
-        int i1, j1;
-        const bool okn = locate64(G, x, y, i1, j1);
-        if (miss & okn) slot64_load<NV>(G, P, va, vb, s, i1, j1);
-        wait_vmem();
-        ok = ok | (miss & okn);
-    }
-    return ok;
-}
-
-// interpolator::bilinear in f64 on the slot's cell for value array q, with
-// its corner exit (a target on a node returns that corner, first of A, B,
-// C, D; EXITS false leaves it out, for a target inside the slot's fast
-// thresholds, which is on no node), and the cell-difference slopes.  The
-// det == 0 exit is the caller's (m01 is NaN there).
-template <int NV, bool EXITS = true>
-__device__ __forceinline__ Val64 slot64_value(const Grid64View &G, const Slot64<NV> &s, int q,
-                                              double x, double y, Cell64 &c)
-{
-    const double vA = s.v[q][0], vB = s.v[q][1], vC = s.v[q][2], vD = s.v[q][3];
-    const double a10 = vB - vA, a01 = vD - vA;
-    const double a11 = ((vC - vA) - a10) - a01;
-    c.iA = s.iA;
-    c.u = s.m.x * (y - s.yp.x);
-    c.w = s.m.y * (x - s.xp.x);
+    const double a10 = bc.x - ad.x, a01 = ad.y - ad.x;
+    const double a11 = ((bc.y - ad.x) - a10) - a01;
     Val64 r;
-    r.val = ((vA + a10 * c.u) + a01 * c.w) + (a11 * c.u) * c.w;
-    if (EXITS) {
-        const bool ex = x == s.xp.x, exd = x == s.xp.y, eya = y == s.yp.x, eyb = y == s.yp.y;
-        if ((ex | exd) & (eya | eyb))
-            r.val = ex ? (eya ? vA : vB) : (eyb ? vC : vD);
-    }
-    r.gx = (vD - vA) * G.rxs;
-    r.gy = (vB - vA) * G.rys;
-    r.dx = (a01 + a11 * c.u) * s.m.y;
-    r.dy = (a10 + a11 * c.w) * s.m.x;
+    r.val = ((ad.x + a10 * u) + a01 * w) + (a11 * u) * w;
+    r.gx = a01 * G.rxs;
+    r.gy = a10 * G.rys;
+    r.dx = (a01 + a11 * u) * xa.y;
+    r.dy = (a10 + a11 * w) * ya.y;
     return r;
 }
 
-// the det == 0 exit: m01 is NaN, unless the target is on a node (EXITS
-// false: a target inside the fast thresholds, on no node)
-template <int NV, bool EXITS = true>
-__device__ __forceinline__ bool slot64_det_ok(const Slot64<NV> &s, double x, double y)
+// the bilinear fractions of a target in the slot's cell
+template <int NV>
+__device__ __forceinline__ Cell64 slot64_cell(const Slot64<NV> &s, double x, double y)
 {
-    if (!EXITS) return !__builtin_isnan(s.m.x);
-    const bool node = ((x == s.xp.x) | (x == s.xp.y)) & ((y == s.yp.x) | (y == s.yp.y));
-    return node | !__builtin_isnan(s.m.x);
+    return Cell64{s.iA, s.ya.y * (y - s.ya.x), s.xa.y * (x - s.xa.x)};
 }
 
-// Bathymetry in fp64 mode.  Returns ok = false where the reference errs;
-// h is NaN (not an error) for a NaN point (cartesian_netcdf3.rs:102-105) and
-// outside an ArrayDepth.  cell is meaningful for BK_GRID only.
+// The full query of the N value arrays of a gridded field at (x, y): its
+// cell by the reference's index, with the exits of interpolator::bilinear (a
+// target on a node returns that corner, first of A, B, C, D; det == 0 errs
+// anywhere else).  Returns false where the reference errs.
+template <int N>
+__device__ __forceinline__ bool full64(const Grid64View &G, const Grid64Ptrs &P,
+                                       const double *const (&vals)[N], double x, double y,
+                                       Val64 (&v)[N], Cell64 &c)
+{
+    int i1, j1;
+    bool ok = locate64(G, x, y, i1, j1);
+    Slot64<N> s;
+    if (ok) slot64_load<N>(G, P, vals, s, i1, j1);
+    const double xb = ok ? P.xn[i1 + 1] : 0.0, yb = ok ? P.yn[j1 + 1] : 0.0;
+    wait_vmem();
+    c = slot64_cell<N>(s, x, y);
+    const bool xl = x == s.xa.x, xr = x == xb, yl = y == s.ya.x, yr = y == yb;
+    const bool node = (xl | xr) & (yl | yr);
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        v[q] = cell64_value(G, s.ad[q], s.bc[q], s.xa, s.ya, c.u, c.w);
+        if (node) v[q].val = xl ? (yl ? s.ad[q].x : s.bc[q].x) : (yr ? s.bc[q].y : s.ad[q].y);
+    }
+    return ok & (node | ((xb - s.xa.x) * (yb - s.ya.x) != 0.0));
+}
+
+// Bathymetry in fp64 mode, analytic kinds in place and gridded depth by the
+// full query.  Returns ok = false where the reference errs; h is NaN (not an
+// error) for a NaN point (cartesian_netcdf3.rs:102-105) and outside an
+// ArrayDepth.  cell is meaningful for BK_GRID only.
 template <int BK>
 __device__ __forceinline__ bool bathy64(const Grid64View &B, const Grid64Ptrs &P,
-                                        const double *depth, Slot64<1> &bs, double x, double y,
-                                        Val64 &h, Cell64 &cell)
+                                        const double *depth, double x, double y, Val64 &h,
+                                        Cell64 &cell)
 {
     cell.iA = 0; cell.u = 0.0; cell.w = 0.0;
     h.dx = 0.0; h.dy = 0.0;
@@ -259,9 +280,10 @@ __device__ __forceinline__ bool bathy64(const Grid64View &B, const Grid64Ptrs &P
         h.val = (double)P.arr[xi * (uint64_t)B.an + yi];
         return true;
     } else {                                               // cartesian_netcdf3.rs:98-135
-        bool ok = slot64_query<1>(B, P, depth, depth, bs, x, y);
-        h = slot64_value<1>(B, bs, 0, x, y, cell);
-        ok = ok & slot64_det_ok<1>(bs, x, y);
+        const double *const vals[1] = {depth};
+        Val64 v[1];
+        bool ok = full64<1>(B, P, vals, x, y, v, cell);
+        h = v[0];
         if (nn) {
             h.val = MR_NAN; h.gx = MR_NAN; h.gy = MR_NAN;
             ok = true;
@@ -270,12 +292,13 @@ __device__ __forceinline__ bool bathy64(const Grid64View &B, const Grid64Ptrs &P
     }
 }
 
-// Current in fp64 mode; ok = false where the reference errs (no NaN guard:
-// a NaN point errs, cartesian_current.rs:492-495).
+// Current in fp64 mode, a gridded one by the full query; ok = false where
+// the reference errs (no NaN guard: a NaN point errs,
+// cartesian_current.rs:492-495).
 template <int CK>
 __device__ __forceinline__ bool current64(const Grid64View &C, const Grid64Ptrs &P,
-                                          const double *cu, const double *cv, Slot64<2> &cs,
-                                          double x, double y, Val64 &u, Val64 &v, Cell64 &cell)
+                                          const double *cu, const double *cv, double x, double y,
+                                          Val64 &u, Val64 &v, Cell64 &cell)
 {
     cell.iA = 0; cell.u = 0.0; cell.w = 0.0;
     if (CK == CK_CONSTANT) {                               // constant_current.rs:66-76
@@ -284,10 +307,12 @@ __device__ __forceinline__ bool current64(const Grid64View &C, const Grid64Ptrs 
         v.gx = v.gy = v.dx = v.dy = 0.0;
         return true;
     } else {                                               // cartesian_current.rs:487-542
-        bool ok = slot64_query<2>(C, P, cu, cv, cs, x, y);
-        u = slot64_value<2>(C, cs, 0, x, y, cell);
-        v = slot64_value<2>(C, cs, 1, x, y, cell);
-        return ok & slot64_det_ok<2>(cs, x, y);
+        const double *const vals[2] = {cu, cv};
+        Val64 w[2];
+        const bool ok = full64<2>(C, P, vals, x, y, w, cell);
+        u = w[0];
+        v = w[1];
+        return ok;
     }
 }
 
@@ -296,21 +321,49 @@ struct Fields64 {
     const double *depth, *u, *v;
 };
 
-// The cells a lane holds, for the evaluation in hand (q) and the next (n).
+// The cells a lane holds for one evaluation.  SH: depth and current lie on
+// the same f64 axes, so one slot (b) holds depth, u and v; the tests,
+// fractions and axis cells of a second one are saved.
+template <int BK, int CK, bool SH>
 struct Slots64 {
-    Slot64<1> b;
+    Slot64<SH ? 3 : 1> b;
     Slot64<2> c;
 };
 
-// The cells that (x, y) most likely lies in, loaded into s whatever it
-// holds (a ray's first cells, or a segment's).
-template <int BK, int CK>
+// Load the cells that (x, y) most likely lies in: every one (a ray's first
+// cells, or a segment's), or those of held that do not contain it.
+template <int BK, int CK, bool SH, bool ALL>
+__device__ __forceinline__ void load64(const Grid64View &B, const Grid64Ptrs &BP,
+                                       const Grid64View &C, const Grid64Ptrs &CP,
+                                       const Fields64 &F, const Slots64<BK, CK, SH> &held,
+                                       Slots64<BK, CK, SH> &s, double x, double y)
+{
+    if constexpr (SH) {
+        const double *const vals[3] = {F.depth, F.u, F.v};
+        if (ALL || off_slot64(held.b, x, y) >= OUT64)
+            slot64_prefetch<3>(C, CP, vals, __builtin_elementwise_min(B.oob_from, C.oob_from),
+                               s.b, x, y);
+    } else {
+        if constexpr (BK == BK_GRID) {
+            const double *const vals[1] = {F.depth};
+            if (ALL || off_slot64(held.b, x, y) >= OUT64)
+                slot64_prefetch<1>(B, BP, vals, B.oob_from, s.b, x, y);
+        }
+        if constexpr (CK == CK_GRID) {
+            const double *const vals[2] = {F.u, F.v};
+            if (ALL || off_slot64(held.c, x, y) >= OUT64)
+                slot64_prefetch<2>(C, CP, vals, C.oob_from, s.c, x, y);
+        }
+    }
+}
+
+template <int BK, int CK, bool SH>
 __device__ __forceinline__ void load_guess64(const Grid64View &B, const Grid64Ptrs &BP,
                                              const Grid64View &C, const Grid64Ptrs &CP,
-                                             const Fields64 &F, Slots64 &s, double x, double y)
+                                             const Fields64 &F, Slots64<BK, CK, SH> &s, double x,
+                                             double y)
 {
-    if (BK == BK_GRID) slot64_prefetch<1>(B, BP, F.depth, F.depth, s.b, x, y);
-    if (CK == CK_GRID) slot64_prefetch<2>(C, CP, F.u, F.v, s.c, x, y);
+    load64<BK, CK, SH, true>(B, BP, C, CP, F, s, s, x, y);
 }
 
 // s_waitcnt on the vector memory count alone, for counts up to 63 (gfx9
@@ -324,58 +377,106 @@ __device__ __forceinline__ void vm_wait_upto()
 }
 
 // Start loading, into n, the cells of (x, y) that q does not hold.
-template <int BK, int CK>
+template <int BK, int CK, bool SH>
 __device__ __forceinline__ void prefetch64(const Grid64View &B, const Grid64Ptrs &BP,
                                            const Grid64View &C, const Grid64Ptrs &CP,
-                                           const Fields64 &F, const Slots64 &q, Slots64 &n,
-                                           double x, double y)
+                                           const Fields64 &F, const Slots64<BK, CK, SH> &q,
+                                           Slots64<BK, CK, SH> &n, double x, double y)
 {
-    if (BK == BK_GRID && !slot64_inside<1>(q.b, x, y))
-        slot64_prefetch<1>(B, BP, F.depth, F.depth, n.b, x, y);
-    if (CK == CK_GRID && !slot64_inside<2>(q.c, x, y))
-        slot64_prefetch<2>(C, CP, F.u, F.v, n.c, x, y);
+    load64<BK, CK, SH, false>(B, BP, C, CP, F, q, n, x, y);
 }
 
-// WaveRayPath::system in fp64 mode, with the cells held in sl.  As rhs()
-// does for the reference precision, every lane first evaluates with the
-// cells in hand (no branch, no load: the gridded queries' own operations for
-// a target inside the slot's cell), and the lanes whose target is not inside
-// them evaluate again with the full queries, which locate and load cells.
-template <int BK, int CK, int MATH>
-__device__ __forceinline__ void rhs64(const Grid64View &B, const Grid64Ptrs &BP,
-                                      const Grid64View &C, const Grid64Ptrs &CP,
-                                      const Fields64 &F, Slots64 &sl, const FastConsts &K,
-                                      double x, double y, double kx, double ky, double &dx,
-                                      double &dy, double &dkx, double &dky)
-{
+// The fields of one fp64 evaluation, with their cells.
+struct Point64 {
     Val64 h, u, v;
     Cell64 bc, cc;
     bool okb, okc;
-    bool slow = false;
-    if (BK == BK_GRID) {
-        slow = !slot64_inside<1>(sl.b, x, y);
-        h = slot64_value<1, false>(B, sl.b, 0, x, y, bc);
-        okb = slot64_det_ok<1, false>(sl.b, x, y);
+};
+
+// The fields at (x, y) from the cells in hand: the gridded queries' own
+// operations for a target inside the slots' fast intervals, with no branch
+// and no load.  Returns OUT64 or more where that does not hold (a target
+// outside them, a NaN target), and those lanes must take point64_full.
+template <int BK, int CK, bool SH>
+__device__ __forceinline__ uint32_t point64_fast(const Grid64View &B, const Grid64Ptrs &BP,
+                                                 const Grid64View &C, const Grid64Ptrs &CP,
+                                                 const Fields64 &F,
+                                                 const Slots64<BK, CK, SH> &sl, double x,
+                                                 double y, Point64 &p)
+{
+    uint32_t off = 0;
+    p.okb = true;
+    p.okc = true;
+    if constexpr (BK == BK_GRID) {
+        off = off_slot64(sl.b, x, y);
+        p.bc = slot64_cell(sl.b, x, y);
+        p.h = cell64_value(B, sl.b.ad[0], sl.b.bc[0], sl.b.xa, sl.b.ya, p.bc.u, p.bc.w);
     } else {
-        okb = bathy64<BK>(B, BP, F.depth, sl.b, x, y, h, bc);
+        p.okb = bathy64<BK>(B, BP, F.depth, x, y, p.h, p.bc);
     }
-    if (CK == CK_GRID) {
-        slow = slow | !slot64_inside<2>(sl.c, x, y);
-        u = slot64_value<2, false>(C, sl.c, 0, x, y, cc);
-        v = slot64_value<2, false>(C, sl.c, 1, x, y, cc);
-        okc = slot64_det_ok<2, false>(sl.c, x, y);
+    if constexpr (SH) {
+        p.cc = p.bc;
+        p.u = cell64_value(C, sl.b.ad[1], sl.b.bc[1], sl.b.xa, sl.b.ya, p.cc.u, p.cc.w);
+        p.v = cell64_value(C, sl.b.ad[2], sl.b.bc[2], sl.b.xa, sl.b.ya, p.cc.u, p.cc.w);
+    } else if constexpr (CK == CK_GRID) {
+        const uint32_t offc = off_slot64(sl.c, x, y);
+        off = __builtin_elementwise_max(off, offc);
+        p.cc = slot64_cell(sl.c, x, y);
+        p.u = cell64_value(C, sl.c.ad[0], sl.c.bc[0], sl.c.xa, sl.c.ya, p.cc.u, p.cc.w);
+        p.v = cell64_value(C, sl.c.ad[1], sl.c.bc[1], sl.c.xa, sl.c.ya, p.cc.u, p.cc.w);
     } else {
-        okc = current64<CK>(C, CP, F.u, F.v, sl.c, x, y, u, v, cc);
+        p.okc = current64<CK>(C, CP, F.u, F.v, x, y, p.u, p.v, p.cc);
     }
-    odes<MATH>(K, okb ? h.val : MR_NAN, h.gx, h.gy, okc, u.val, v.val, u.gx, u.gy, v.gx, v.gy,
-               kx, ky, dx, dy, dkx, dky);
-    if (__builtin_expect(wave_any(slow), 0)) {
+    return off;
+}
+
+// ... and by the full queries, on views loaded for the occasion: most of a
+// view serves only them, and held in registers all the time it would push
+// what every evaluation uses into accumulation registers (or scratch).
+template <int BK, int CK>
+__device__ __forceinline__ void point64_full(const Grid64Ptrs &BP, const Grid64Ptrs &CP,
+                                             const Fields64 &F, double x, double y, Point64 &p)
+{
+    const Grid64View B = load_view<Grid64View>(BP.view);
+    const Grid64View C = load_view<Grid64View>(CP.view);
+    p.okb = bathy64<BK>(B, BP, F.depth, x, y, p.h, p.bc);
+    p.okc = current64<CK>(C, CP, F.u, F.v, x, y, p.u, p.v, p.cc);
+}
+
+// Whether any lane must take point64_full, as one compare and one scalar
+// branch: the mask intrinsic is not folded into the test inside the block,
+// which is laid out after the loop.
+template <int BK, int CK>
+__device__ __forceinline__ bool any_off64(uint32_t off)
+{
+    if (BK != BK_GRID && CK != CK_GRID) return false;
+    return __builtin_expect(__builtin_amdgcn_uicmp(off, OUT64, 35 /* >= */) != 0, 0);
+}
+
+// WaveRayPath::system in fp64 mode, with the cells held in sl.  As rhs_rec()
+// does for the reference precision, every lane first evaluates with the
+// cells in hand, and the lanes whose target is not inside them evaluate
+// again with the full queries.
+template <int BK, int CK, bool SH, int MATH>
+__device__ __forceinline__ void rhs64(const Grid64View &B, const Grid64Ptrs &BP,
+                                      const Grid64View &C, const Grid64Ptrs &CP,
+                                      const Fields64 &F, const Slots64<BK, CK, SH> &sl,
+                                      const FastConsts &K, double x, double y, double kx,
+                                      double ky, double &dx, double &dy, double &dkx,
+                                      double &dky)
+{
+    Point64 p;
+    auto system = [&] {
+        odes<MATH>(K, p.okb ? p.h.val : MR_NAN, p.h.gx, p.h.gy, p.okc, p.u.val, p.v.val, p.u.gx,
+                   p.u.gy, p.v.gx, p.v.gy, kx, ky, dx, dy, dkx, dky);
+    };
+    const uint32_t off = point64_fast<BK, CK, SH>(B, BP, C, CP, F, sl, x, y, p);
+    system();
+    if (any_off64<BK, CK>(off)) {
         __asm__ volatile("");
-        if (slow) {                    // a NaN target lands here too
-            okb = bathy64<BK>(B, BP, F.depth, sl.b, x, y, h, bc);
-            okc = current64<CK>(C, CP, F.u, F.v, sl.c, x, y, u, v, cc);
-            odes<MATH>(K, okb ? h.val : MR_NAN, h.gx, h.gy, okc, u.val, v.val, u.gx, u.gy,
-                       v.gx, v.gy, kx, ky, dx, dy, dkx, dky);
+        if (off >= OUT64) {
+            point64_full<BK, CK>(BP, CP, F, x, y, p);
+            system();
         }
     }
 }
@@ -502,13 +603,15 @@ __device__ constexpr bool depth_is_flat()
 // Whether lin_apply reads field f of a linearisation record for the field
 // kinds BK, CK (the only fields the ring is given): the depth terms (16-20,
 // 23, 24) for gridded depth, the current's (21, 22, 25, 26) for a gridded
-// current, and with a flat depth not the four zeros of M's x and y rows.
-template <int BK, int CK>
+// current, and with a flat depth not the four zeros of M's x and y rows.  On
+// shared cells (SH) the current's fractions serve the depth too.
+template <int BK, int CK, bool SH>
 __device__ constexpr bool lin_field_used(int f)
 {
     if (f < 16)
         return !depth_is_flat<BK>() || f == 0 || f == 1 || f == 4 || f == 5 || f >= 8;
     if (f == 27) return true;
+    if (SH && (f == 23 || f == 24)) return false;
     if (f <= 20 || f == 23 || f == 24) return BK == BK_GRID;
     return CK == CK_GRID;
 }
@@ -593,48 +696,30 @@ __device__ __forceinline__ void lin_record(const FastConsts &K, const Val64 &h, 
                        (CK == CK_GRID && okc) ? cc.iA : 0xFFFFFFFFu);
 }
 
-template <int BK, int CK>
+template <int BK, int CK, bool SH>
 __device__ __forceinline__ void rhs64_lin(const Grid64View &B, const Grid64Ptrs &BP,
                                           const Grid64View &C, const Grid64Ptrs &CP,
-                                          const Fields64 &F, Slots64 &sl, const FastConsts &K,
-                                          double x, double y, double kx, double ky,
-                                          double R[LIN_N])
+                                          const Fields64 &F, const Slots64<BK, CK, SH> &sl,
+                                          const FastConsts &K, double x, double y, double kx,
+                                          double ky, double R[LIN_N])
 {
     // as rhs64: first with the cells in hand, then the full queries for the
     // lanes whose target is not inside them
-    Val64 h, u, v;
-    Cell64 bc, cc;
-    bool okb, okc;
-    bool slow = false;
-    if (BK == BK_GRID) {
-        slow = !slot64_inside<1>(sl.b, x, y);
-        h = slot64_value<1, false>(B, sl.b, 0, x, y, bc);
-        okb = slot64_det_ok<1, false>(sl.b, x, y);
-    } else {
-        okb = bathy64<BK>(B, BP, F.depth, sl.b, x, y, h, bc);
-    }
-    if (CK == CK_GRID) {
-        slow = slow | !slot64_inside<2>(sl.c, x, y);
-        u = slot64_value<2, false>(C, sl.c, 0, x, y, cc);
-        v = slot64_value<2, false>(C, sl.c, 1, x, y, cc);
-        okc = slot64_det_ok<2, false>(sl.c, x, y);
-    } else {
-        okc = current64<CK>(C, CP, F.u, F.v, sl.c, x, y, u, v, cc);
-    }
-    lin_record<BK, CK>(K, h, u, v, bc, cc, okb, okc, kx, ky, R);
-    if (__builtin_expect(wave_any(slow), 0)) {
+    Point64 p;
+    const uint32_t off = point64_fast<BK, CK, SH>(B, BP, C, CP, F, sl, x, y, p);
+    lin_record<BK, CK>(K, p.h, p.u, p.v, p.bc, p.cc, p.okb, p.okc, kx, ky, R);
+    if (any_off64<BK, CK>(off)) {
         __asm__ volatile("");
-        if (slow) {
-            okb = bathy64<BK>(B, BP, F.depth, sl.b, x, y, h, bc);
-            okc = current64<CK>(C, CP, F.u, F.v, sl.c, x, y, u, v, cc);
-            lin_record<BK, CK>(K, h, u, v, bc, cc, okb, okc, kx, ky, R);
+        if (off >= OUT64) {
+            point64_full<BK, CK>(BP, CP, F, x, y, p);
+            lin_record<BK, CK>(K, p.h, p.u, p.v, p.bc, p.cc, p.okb, p.okc, kx, ky, R);
         }
     }
 }
 
 // Applies a linearisation record R to the cotangent g: z = M g, and the
 // field-value cotangents to the accumulators.
-template <int BK, int CK>
+template <int BK, int CK, bool SH>
 __device__ __forceinline__ void lin_apply(const double R[LIN_N], const Grid64View &B,
                                           const Grid64View &C, const Grads64 &Gr, Accs64 &acc,
                                           const double g[4], double z[4])
@@ -651,7 +736,7 @@ __device__ __forceinline__ void lin_apply(const double R[LIN_N], const Grid64Vie
     unpack_cells(R[27], ib, ic);
     if (BK == BK_GRID && Gr.depth && ib != 0xFFFFFFFFu) {
         const double hbar = ((R[16] * g[0] + R[17] * g[1]) + R[18] * g[2]) + R[19] * g[3];
-        Cell64 cell{ib, R[23], R[24]};
+        Cell64 cell{ib, R[SH ? 25 : 23], R[SH ? 26 : 24]};
         acc_add(acc.h, Gr.depth, (uint32_t)B.nx, cell, B.rxs, B.rys, hbar, g[2] * R[20],
                 g[3] * R[20]);
     }
@@ -670,44 +755,27 @@ __device__ __forceinline__ void lin_apply(const double R[LIN_N], const Grid64Vie
 // accumulators.  The dispersion terms are evaluated with the closed forms of
 // the fast mode whatever the forward's math mode: only the derivative
 // depends on them.  The state must be one at which rhs64 is finite.
-template <int BK, int CK>
+template <int BK, int CK, bool SH>
 __device__ __forceinline__ void rhs64_vjp(const Grid64View &B, const Grid64Ptrs &BP,
                                           const Grid64View &C, const Grid64Ptrs &CP,
-                                          const Fields64 &F, Slots64 &sl, const Grads64 &Gr,
-                                          Accs64 &acc, const FastConsts &K, double x, double y,
-                                          double kx, double ky, double g0, double g1, double g2,
-                                          double g3, double &bx, double &by, double &bkx,
-                                          double &bky)
+                                          const Fields64 &F, const Slots64<BK, CK, SH> &sl,
+                                          const Grads64 &Gr, Accs64 &acc, const FastConsts &K,
+                                          double x, double y, double kx, double ky, double g0,
+                                          double g1, double g2, double g3, double &bx,
+                                          double &by, double &bkx, double &bky)
 {
     // the field values as in rhs64: from the cells in hand, then the full
     // queries for the lanes whose target is not inside them (the product and
     // the accumulation below run once, after both)
-    Val64 h, u, v;
-    Cell64 bc, cc;
-    bool okb, okc;
-    bool slow = false;
-    if (BK == BK_GRID) {
-        slow = !slot64_inside<1>(sl.b, x, y);
-        h = slot64_value<1, false>(B, sl.b, 0, x, y, bc);
-        okb = slot64_det_ok<1, false>(sl.b, x, y);
-    } else {
-        okb = bathy64<BK>(B, BP, F.depth, sl.b, x, y, h, bc);
-    }
-    if (CK == CK_GRID) {
-        slow = slow | !slot64_inside<2>(sl.c, x, y);
-        u = slot64_value<2, false>(C, sl.c, 0, x, y, cc);
-        v = slot64_value<2, false>(C, sl.c, 1, x, y, cc);
-        okc = slot64_det_ok<2, false>(sl.c, x, y);
-    } else {
-        okc = current64<CK>(C, CP, F.u, F.v, sl.c, x, y, u, v, cc);
-    }
-    if (__builtin_expect(wave_any(slow), 0)) {
+    Point64 p;
+    const uint32_t off = point64_fast<BK, CK, SH>(B, BP, C, CP, F, sl, x, y, p);
+    if (any_off64<BK, CK>(off)) {
         __asm__ volatile("");
-        if (slow) {
-            okb = bathy64<BK>(B, BP, F.depth, sl.b, x, y, h, bc);
-            okc = current64<CK>(C, CP, F.u, F.v, sl.c, x, y, u, v, cc);
-        }
+        if (off >= OUT64) point64_full<BK, CK>(BP, CP, F, x, y, p);
     }
+    const Val64 &h = p.h, &u = p.u, &v = p.v;
+    const Cell64 &bc = p.bc, &cc = p.cc;
+    const bool okb = p.okb, okc = p.okc;
     const double hh = h.val;
     const double k2 = __builtin_fma(kx, kx, ky * ky);
     const double rk = rsq_nr(k2);                       // 1/k

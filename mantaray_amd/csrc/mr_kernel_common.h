@@ -28,26 +28,6 @@ __device__ __forceinline__ void vm_wait()
     __builtin_amdgcn_s_waitcnt(0x0F70 | N);
 }
 
-// Copy a field view from device memory into per-lane registers.  The loads
-// go through a lane-varying (always zero) offset so they are vector loads
-// and the view lives in VGPRs for the whole kernel: the scalar register file
-// cannot hold both views next to the loop's own scalars, and re-reading
-// them with scalar loads puts a load latency into every evaluation.
-template <class View>
-__device__ __forceinline__ View load_view(const void *p)
-{
-    static_assert(sizeof(View) % 4 == 0, "view size");
-    int zero;
-    __asm__ volatile("v_mov_b32 %0, 0" : "=v"(zero));
-    const int *src = reinterpret_cast<const int *>(p) + zero;
-    int buf[sizeof(View) / 4];
-#pragma unroll
-    for (int i = 0; i < (int)(sizeof(View) / 4); ++i) buf[i] = src[i];
-    View v;
-    __builtin_memcpy(&v, buf, sizeof(View));
-    return v;
-}
-
 // Have a loaded view in registers at this point: each word is an input of
 // an empty asm statement, so the compiler waits for the view's loads here
 // and knows them complete in the code that follows (a loop after this does

@@ -125,6 +125,7 @@ struct Trace64Args {
     int solout;
     int stride;                        // checkpoint every stride steps
     double *ckpt;                      // [n_ckpt][4][n_rays], may be null
+    int shared;                        // depth and current gridded on the same f64 axes
 };
 
 // Reverse sweep of the discrete RK4 adjoint.
@@ -144,6 +145,7 @@ struct AdjointArgs {
     int64_t work_ld;                   // >= blocks * block threads
     double *g_x0, *g_y0, *g_kx0, *g_ky0;     // may be null
     Grads64 grads;                     // gradient grids, cleared by the caller
+    int shared;                        // as in Trace64Args
 };
 
 struct Rhs64Args {
@@ -153,12 +155,6 @@ struct Rhs64Args {
     int64_t n;
     const double *s;
     double *ds;
-};
-
-struct M64BuildArgs {
-    int64_t nx, ny;
-    const double *ax, *ay;
-    double2 *m;
 };
 
 hipError_t launch_trace(const TraceArgs &a, int bk, int ck, int math, int block,
@@ -182,7 +178,6 @@ hipError_t launch_trace64(const Trace64Args &a, int bk, int ck, int math, int bl
 hipError_t launch_adjoint(const AdjointArgs &a, int bk, int ck, int math, int waves,
                           hipStream_t stream);
 hipError_t launch_rhs64(const Rhs64Args &a, int bk, int ck, int math, hipStream_t stream);
-hipError_t launch_build_m64(const M64BuildArgs &a, hipStream_t stream);
 hipError_t launch_fill(double *p, int64_t n, double v, hipStream_t stream);
 // the device address of this device's MR_ADJOINT_SCRATCH_BYTES scratch array
 // (looked up on the device's first call, then cached)

@@ -1,0 +1,104 @@
+"""The fp64-interpolation trace on its cell slots, against the oracle in that
+mode: depth and current on the same axes (one slot for both) or not, axes
+uniform, jittered, with a repeated node (cells of zero size, which err),
+descending, or with value arrays that end before the grid does; states on
+nodes, on cell lines, off the grid and NaN.  Row counts and NaN patterns are
+identical, positions within 1e-7 m and wavenumbers within 1e-9 of their scale
+(the tolerances of the other fp64 traces).  And the reverse sweeps on shared
+axes give the gradients of the same fields held apart (the current's grid
+with one more row, which no ray reaches): both are sums of the same terms,
+equal to 1e-11 of each gradient's scale.
+"""
+import numpy as np
+import pytest
+
+from _helpers import random_states
+
+pytestmark = pytest.mark.gpu
+
+
+def _axis(rng, n, form):
+    a = 40.0 * np.arange(n) - 75.0
+    if form == "jittered":
+        a[1:] += rng.uniform(-8.0, 8.0, n - 1)
+    elif form == "repeated node":
+        a[n // 2:] -= 40.0
+    elif form == "descending":
+        a = a[::-1].copy()
+    return a.astype(np.float32).astype(np.float64)
+
+
+def _fields(nx, ny, form, shared):
+    rng = np.random.default_rng(nx * 100 + ny)
+    x, y = _axis(rng, nx, form), _axis(rng, ny, "jittered" if form == "jittered" else "uniform")
+    X, Y = np.meshgrid(x, y)
+    depth = 14.0 + 8.0 * np.sin(X / 90.0) * np.cos(Y / 70.0) + rng.normal(0.0, 1.0, X.shape)
+    cx, cy = x, y
+    if not shared:
+        cy = np.append(y, y[-1] + 40.0)
+    U = 0.6 * np.sin(cy / 80.0)[:, None] + rng.normal(0.0, 0.1, (cy.size, cx.size))
+    V = 0.5 * np.cos(cx / 60.0)[None, :] + rng.normal(0.0, 0.1, (cy.size, cx.size))
+    d, u, v = depth.ravel(), U.ravel(), V.ravel()
+    if form == "short data":
+        d, u, v = d[:-2 * nx - 3], u[:-nx], v[:-nx - 5]
+    return x, y, d, cx, cy, u, v
+
+
+FORMS = ("uniform", "jittered", "repeated node", "descending", "short data")
+
+
+@pytest.mark.parametrize("shared", [True, False])
+@pytest.mark.parametrize("form", FORMS)
+@pytest.mark.parametrize("nx,ny", [(2, 4), (5, 9), (23, 14)])
+def test_trace(oracle_mod, nx, ny, form, shared):
+    import mantaray_amd as mr
+    x, y, d, cx, cy, u, v = _fields(nx, ny, form, shared)
+    x32, y32 = x.astype(np.float32), y.astype(np.float32)
+    cfg = {"bathy": {"x": np.sort(np.append(x, [x.min() - 40.0, x.max() + 40.0])), "y": y}}
+    s = random_states(nx + ny, cfg, 256)
+    args = (*s.T.copy(), 0.0, 20.0, 0.8)
+    ref = oracle_mod.trace_many(oracle_mod.Bathymetry.grid(x32, y32, d),
+                                oracle_mod.Current.grid(cx, cy, u, v), *args,
+                                prec=oracle_mod.PREC_FP64_INTERP)
+    b, c = mr.Bathymetry.from_arrays(x32, y32, d), mr.Current.from_arrays(cx, cy, u, v)
+    if x[0] == x[1]:                                     # refused, as in reference precision
+        with pytest.raises(mr._capi.MantarayError, match="zero spacing"):
+            mr.trace_many(b, c, *args, precision="fp64")
+        return
+    got = mr.trace_many(b, c, *args, precision="fp64")
+    assert np.array_equal(got["len"], ref["len"])
+    for k in ("x", "y", "kx", "ky"):
+        assert np.array_equal(np.isnan(got[k]), np.isnan(ref[k])), k
+    assert max(np.nanmax(np.abs(got[k] - ref[k])) for k in ("x", "y")) <= 1e-7
+    scale = np.nanmax(np.abs(ref["kx"])) + np.nanmax(np.abs(ref["ky"]))
+    assert max(np.nanmax(np.abs(got[k] - ref[k])) for k in ("kx", "ky")) <= 1e-9 * scale
+
+
+@pytest.mark.parametrize("block", [64, 128, 256])
+@pytest.mark.parametrize("n_rays,stride,rows", [(1, 7, False), (65, 50, True), (200, 13, False)])
+def test_gradients(block, n_rays, stride, rows):
+    import torch
+
+    import mantaray_amd as mr
+    from mantaray_amd import adjoint
+    x, y, d, cx, cy, u, v = _fields(23, 14, "jittered", False)
+    rng = np.random.default_rng(n_rays)
+    s = [torch.tensor(a, device="cuda:0") for a in
+         (rng.uniform(x[2], x[-3], n_rays), rng.uniform(y[1], y[-2], n_rays),
+          rng.uniform(-0.2, 0.2, n_rays), rng.uniform(-0.2, 0.2, n_rays))]
+    b = mr.Bathymetry.from_arrays(x.astype(np.float32), y.astype(np.float32), d)
+    steps, dt = 40, 0.7
+    T = (steps - 0.5) * dt
+    g = np.random.default_rng(1)
+    g_end = torch.tensor(g.normal(size=(n_rays, 4)), device="cuda:0")
+    g_rows = {k: torch.tensor(g.normal(size=(steps + 1, n_rays)), device="cuda:0")
+              for k in ("x", "ky")} if rows else None
+    grads = []
+    for m in (y.size, cy.size):                          # on shared axes, then apart
+        c = mr.Current.from_arrays(cx, cy[:m], u[: m * 23], v[: m * 23])
+        f = adjoint.trace_fp64(b, c, *s, 0.0, T, dt, stride=stride)
+        r = adjoint.adjoint(b, c, f, 0.0, T, dt, stride, g_end=g_end, g_rows=g_rows,
+                            block_size=block)
+        grads.append({k: t.cpu().numpy()[: 14 * 23 if k in "uv" else None] for k, t in r.items()})
+    for k, want in grads[1].items():
+        assert np.abs(grads[0][k] - want).max() <= 1e-11 * np.abs(want).max(), k
