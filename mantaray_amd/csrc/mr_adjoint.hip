@@ -21,6 +21,11 @@
 // order over them.
 #include <mutex>
 
+// The fp64 mode owes the reference its algorithm, not its roundings: products
+// and sums of one expression become FMAs here (in the front end, so that
+// every kernel a function is inlined into rounds alike).
+#pragma clang fp contract(on)
+
 #include "mantaray_capi.h"
 #include "mr_kernels.h"
 #include "mr_kernel_common.h"
