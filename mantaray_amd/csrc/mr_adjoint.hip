@@ -281,55 +281,48 @@ __global__ void __launch_bounds__(256) trace64_kernel(Trace64Args a)
 //   z1 = J(Y1)^T kb1
 //   lam <- lam + z1 + z2 + z3 + z4
 // and the field-value cotangents of the four products go to the grids.
-template <int BK, int CK, bool SH>
+//
+// The cells are those of two slots with fixed roles, the forward step's
+// scheme in reverse: the stage points pair up as Y3 and Y2, and Y1 with the
+// Y4 of the step before it in time, which is swept next.  sa serves Y4 and
+// Y1, sb Y3 and Y2; sa is refilled after Y4 for Y1 (known), sb after Y2 for
+// the next step's Y3 (nx, ny, known too), each two evaluations before its
+// next use, so no slot is copied and a lane that changes cells does not wait
+// for memory.  AHEAD loads were issued since sb's refill (the caller's, of
+// the next step's data): the wait before sa's refill leaves those in flight,
+// and the wait before sb's covers them.
+template <int BK, int CK, bool SH, int AHEAD>
 __device__ __forceinline__ void rk4_step_adjoint(const Grid64View &B, const Grid64Ptrs &BP,
                                                  const Grid64View &C, const Grid64Ptrs &CP,
-                                                 const Fields64 &F, Slots64<BK, CK, SH> &sn,
-                                                 const Grads64 &Gr, Accs64 &acc,
-                                                 const FastConsts &K, double dt, double half,
-                                                 double sixth, const double s[4],
-                                                 const double ys[3][4], double lam[4])
+                                                 const Fields64 &F, Slots64<BK, CK, SH> &sa,
+                                                 Slots64<BK, CK, SH> &sb, const Grads64 &Gr,
+                                                 Sums64<BK, CK, SH> &sums, const FastConsts &K,
+                                                 double dt, double half, double sixth,
+                                                 const double s[4], const double ys[3][4],
+                                                 const double &nx, const double &ny,
+                                                 double lam[4])
 {
-    double kb[4][4];
+    double w[4], kb[4];                // lam dt/6; the stage's cotangent
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const double w = lam[q] * sixth;
-        kb[0][q] = w; kb[3][q] = w;
-        kb[1][q] = 2.0 * w; kb[2][q] = 2.0 * w;
-    }
-    double Y[4][2];                    // (x, y) of the four stage points
-    Y[0][0] = s[0]; Y[0][1] = s[1];
-#pragma unroll
-    for (int st = 1; st < 4; ++st) {
-        Y[st][0] = ys[st - 1][0];
-        Y[st][1] = ys[st - 1][1];
-    }
-    Slots64<BK, CK, SH> sq = sn;
+    for (int q = 0; q < 4; ++q) kb[q] = w[q] = lam[q] * sixth;
 #pragma unroll
     for (int st = 3; st >= 0; --st) {
-        double Yk[2];
-        if (st == 0) {
-            Yk[0] = s[2]; Yk[1] = s[3];
-        } else {
-            Yk[0] = ys[st - 1][2];
-            Yk[1] = ys[st - 1][3];
-        }
-        // The stage points pair up: Y2 lies with Y1, and Y0 (this step's
-        // start) with the previous step's Y3.  Stages 4 and 2 (st 3, 1) start
-        // loading the cells of the pair that follows (known exactly: Y2, Y0),
-        // stages 3 and 1 (st 2, 0) take them up.
-        if (st == 2 || st == 0)
-            sq = sn;
-        else
-            prefetch64<BK, CK, SH>(B, BP, C, CP, F, sq, sn, Y[st - 1][0], Y[st - 1][1]);
+        const double *Y = st == 0 ? s : ys[st - 1];
         double z[4] = {0.0, 0.0, 0.0, 0.0};
-        rhs64_vjp<BK, CK, SH>(B, BP, C, CP, F, sq, Gr, acc, K, Y[st][0], Y[st][1], Yk[0], Yk[1],
-                          kb[st][0], kb[st][1], kb[st][2], kb[st][3], z[0], z[1], z[2], z[3]);
-        if (st == 0) sn = sq;          // the cells in hand, for the previous step's Y3
+        rhs64_vjp<BK, CK, SH>(B, BP, C, CP, F, (st == 0 || st == 3) ? sa : sb, Gr, sums, K, Y[0],
+                              Y[1], Y[2], Y[3], kb[0], kb[1], kb[2], kb[3], z[0], z[1], z[2],
+                              z[3]);
+        if (st == 3) {
+            vm_wait_upto<AHEAD>();
+            prefetch64<BK, CK, SH>(B, BP, C, CP, F, sa, sa, s[0], s[1]);
+        } else if (st == 1) {
+            vm_wait_upto<0>();
+            prefetch64<BK, CK, SH>(B, BP, C, CP, F, sb, sb, nx, ny);
+        }
         if (st > 0) {
-            const double hs = st < 3 ? half : dt;
+            const double hs = st < 3 ? half : dt, c = st > 1 ? 2.0 : 1.0;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) kb[st - 1][q] += z[q] * hs;
+            for (int q = 0; q < 4; ++q) kb[q] = __builtin_fma(z[q], hs, c * w[q]);
         }
 #pragma unroll
         for (int q = 0; q < 4; ++q) lam[q] += z[q];
@@ -416,8 +409,9 @@ __global__ void __launch_bounds__(ADJ_BLOCK) adjoint_kernel(AdjointArgs a)
         if (a.g_kx) lam[2] += a.g_kx[o];
         if (a.g_ky) lam[3] += a.g_ky[o];
     }
-    Slots64<BK, CK, SH> sn;                                        // cells for the next evaluation
-    Accs64 acc;
+    Slots64<BK, CK, SH> sa, sb;        // the step adjoint's two cell slots
+    __shared__ double queue[Sums64<BK, CK, SH>::words + 1];
+    Sums64<BK, CK, SH> sums(queue);
     for (int t = 0; t <= cmax + 1; ++t) {
         const int c = cmax - t + 1;
         if (t >= 1 && c <= cmax_r) {
@@ -428,6 +422,9 @@ __global__ void __launch_bounds__(ADJ_BLOCK) adjoint_kernel(AdjointArgs a)
             // ahead, while the step before them is swept
             double nxt[16];
             work_get(wk, ld, r, nseg - 1, nxt, [](int) { return true; });
+            // the sweep starts at the segment's last stage points
+            load_guess64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sa, nxt[12], nxt[13]);
+            load_guess64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sb, nxt[8], nxt[9]);
             for (int j = nseg - 1; j >= 0; --j) {
                 double ys[3][4], y[4];
 #pragma unroll
@@ -437,13 +434,12 @@ __global__ void __launch_bounds__(ADJ_BLOCK) adjoint_kernel(AdjointArgs a)
                     ys[1][q] = nxt[8 + q];
                     ys[2][q] = nxt[12 + q];
                 }
-                if (j >= 1) {
-                    work_get(wk, ld, r, j - 1, nxt, [](int) { return true; });
-                }
-                if (j == nseg - 1)     // the sweep starts at the segment's last stage point
-                    prefetch64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sn, sn, ys[2][0], ys[2][1]);
-                rk4_step_adjoint<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sn, a.grads, acc, K, dt, half,
-                                         sixth, y, ys, lam);
+                // (the first step loads its own again: always eight loads, so
+                // that the step can tell them from its cells')
+                work_get(wk, ld, r, __builtin_elementwise_max(j - 1, 0), nxt,
+                         [](int) { return true; });
+                rk4_step_adjoint<BK, CK, SH, 8>(B, a.bp, C, a.cp, a.f, sa, sb, a.grads, sums, K,
+                                                dt, half, sixth, y, ys, nxt[8], nxt[9], lam);
                 const int64_t o = (i0 + j) * nr + r;
                 if (a.g_x) lam[0] += a.g_x[o];
                 if (a.g_y) lam[1] += a.g_y[o];
@@ -453,16 +449,12 @@ __global__ void __launch_bounds__(ADJ_BLOCK) adjoint_kernel(AdjointArgs a)
         }
         __syncthreads();
     }
+    sums.finish(a.grads, (uint32_t)B.nx, (uint32_t)C.nx);
     if (!active) return;
     if (a.g_x0) a.g_x0[r] = lam[0];
     if (a.g_y0) a.g_y0[r] = lam[1];
     if (a.g_kx0) a.g_kx0[r] = lam[2];
     if (a.g_ky0) a.g_ky0[r] = lam[3];
-    if (BK == BK_GRID && a.grads.depth) acc_flush(acc.h, a.grads.depth, (uint32_t)B.nx);
-    if (CK == CK_GRID) {
-        if (a.grads.u) acc_flush(acc.u, a.grads.u, (uint32_t)C.nx);
-        if (a.grads.v) acc_flush(acc.v, a.grads.v, (uint32_t)C.nx);
-    }
 }
 
 // The reverse sweep on one wave per 64 rays, for launches with many more
@@ -503,10 +495,11 @@ __global__ void __launch_bounds__(64) adjoint_seq_kernel(AdjointArgs a)
         if (a.g_kx) lam[2] += a.g_kx[o];
         if (a.g_ky) lam[3] += a.g_ky[o];
     }
-    // the recomputation's two cell slots; the sweep then uses sa (both are
-    // loaded whole at each segment's start)
+    // the two cell slots, of the recomputation and then of the sweep (both
+    // are loaded whole at the start of each)
     Slots64<BK, CK, SH> sa, sb;
-    Accs64 acc;
+    __shared__ double queue[Sums64<BK, CK, SH>::words + 1];
+    Sums64<BK, CK, SH> sums(queue);
     double *wk = a.work;                               // the first half of the buffer
     for (int c = cmax; c >= 0; --c) {
         if (c <= cmax_r) {
@@ -528,6 +521,9 @@ __global__ void __launch_bounds__(64) adjoint_seq_kernel(AdjointArgs a)
             // and sweep it back, each step's data loaded one step ahead
             double nxt[16];
             work_get(wk, ld, r, nseg - 1, nxt, [](int) { return true; });
+            // the sweep starts at the segment's last stage points
+            load_guess64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sa, nxt[12], nxt[13]);
+            load_guess64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sb, nxt[8], nxt[9]);
             for (int j = nseg - 1; j >= 0; --j) {
                 double ys[3][4], y[4];
 #pragma unroll
@@ -537,13 +533,12 @@ __global__ void __launch_bounds__(64) adjoint_seq_kernel(AdjointArgs a)
                     ys[1][q] = nxt[8 + q];
                     ys[2][q] = nxt[12 + q];
                 }
-                if (j >= 1) {
-                    work_get(wk, ld, r, j - 1, nxt, [](int) { return true; });
-                }
-                if (j == nseg - 1)     // the sweep starts at the segment's last stage point
-                    prefetch64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sa, sa, ys[2][0], ys[2][1]);
-                rk4_step_adjoint<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sa, a.grads, acc, K, dt, half,
-                                         sixth, y, ys, lam);
+                // (the first step loads its own again: always eight loads, so
+                // that the step can tell them from its cells')
+                work_get(wk, ld, r, __builtin_elementwise_max(j - 1, 0), nxt,
+                         [](int) { return true; });
+                rk4_step_adjoint<BK, CK, SH, 8>(B, a.bp, C, a.cp, a.f, sa, sb, a.grads, sums, K,
+                                                dt, half, sixth, y, ys, nxt[8], nxt[9], lam);
                 const int64_t o = (i0 + j) * nr + r;
                 if (a.g_x) lam[0] += a.g_x[o];
                 if (a.g_y) lam[1] += a.g_y[o];
@@ -552,16 +547,168 @@ __global__ void __launch_bounds__(64) adjoint_seq_kernel(AdjointArgs a)
             }
         }
     }
+    sums.finish(a.grads, (uint32_t)B.nx, (uint32_t)C.nx);
     if (!active) return;
     if (a.g_x0) a.g_x0[r] = lam[0];
     if (a.g_y0) a.g_y0[r] = lam[1];
     if (a.g_kx0) a.g_kx0[r] = lam[2];
     if (a.g_ky0) a.g_ky0[r] = lam[3];
-    if (BK == BK_GRID && a.grads.depth) acc_flush(acc.h, a.grads.depth, (uint32_t)B.nx);
-    if (CK == CK_GRID) {
-        if (a.grads.u) acc_flush(acc.u, a.grads.u, (uint32_t)C.nx);
-        if (a.grads.v) acc_flush(acc.v, a.grads.v, (uint32_t)C.nx);
+}
+
+// The reverse sweep on one wave per 64 rays for a flat depth, with the stage
+// points formed again instead of stored.  adjoint_seq_kernel's work buffer
+// takes 128 bytes for each ray and step, written and read: at 262,144 rays x
+// 3000 steps 200 GB, 40 ms of traffic.  Here the recomputation stores the
+// states alone (32 bytes), and each reverse step runs its stages forward
+// once, with the linearisation of each beside its derivative (they share all
+// but a few operations); the records of the first three wait in LDS (26 KB
+// a wave, which four waves a CU have) until the cotangent chain comes to
+// them.  Not for a depth with a gradient: its records would not fit.  With
+// the queued sums, on a 2048 x 2048 current, forward and sweep 89.6 -> 64.7
+// ms (the forward is 13.5 of them); the queue alone, before its pairs shared
+// requests and with the stored stage points, cost 2 ms.  What is left is the
+// issue of about 1350 vector instructions a step.
+template <int BK, int CK, int MATH>
+__global__ void __launch_bounds__(64) adjoint_flat_kernel(AdjointArgs a)
+{
+    constexpr int NF = lin_place<BK, CK, false>(LIN_N);    // fields of a record
+    __shared__ double rec[3][NF][64];
+    __shared__ double queue[Sums64<BK, CK, false>::words + 1];
+    const int64_t nr = a.n_rays;
+    const int lane = (int)threadIdx.x;
+    const int64_t rr = (int64_t)blockIdx.x * 64 + lane;
+    const bool active = rr < nr;
+    const int64_t r = active ? rr : nr - 1;
+    const Grid64View B = load_view<Grid64View>(a.B);
+    const Grid64View C = load_view<Grid64View>(a.C);
+    const FastConsts K = load_consts();
+    const double dt = a.dt, half = a.half, sixth = a.sixth;
+    const int stride = a.stride;
+    const int64_t ld = a.work_ld;
+    const bool dead = all_nan4(a.end[4 * r], a.end[4 * r + 1], a.end[4 * r + 2],
+                               a.end[4 * r + 3]);
+    const int64_t m = (int64_t)a.len[r] - (dead ? 2 : 1);
+    const int cmax_r = (active && m >= 1) ? (int)((m - 1) / stride) : -1;
+    const int cmax = wave_max(cmax_r);
+    double lam[4] = {0.0, 0.0, 0.0, 0.0};
+    if (active && m >= 0) {
+        if (a.g_end && !dead) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) lam[q] = a.g_end[4 * r + q];
+        }
+        const int64_t o = m * nr + r;
+        if (a.g_x) lam[0] += a.g_x[o];
+        if (a.g_y) lam[1] += a.g_y[o];
+        if (a.g_kx) lam[2] += a.g_kx[o];
+        if (a.g_ky) lam[3] += a.g_ky[o];
     }
+    Slots64<BK, CK, false> sa, sb;
+    Sums64<BK, CK, false> sums(queue);
+    // the states of a segment's steps, as two pairs each
+    double2 *const wk = reinterpret_cast<double2 *>(a.work) + r;
+    auto put = [&](int j, const double s[4]) {
+        wk[(2 * (int64_t)j) * ld] = make_double2(s[0], s[1]);
+        wk[(2 * (int64_t)j + 1) * ld] = make_double2(s[2], s[3]);
+    };
+    auto get = [&](int j, double s[4]) {
+        const double2 p = wk[(2 * (int64_t)j) * ld], k = wk[(2 * (int64_t)j + 1) * ld];
+        s[0] = p.x; s[1] = p.y; s[2] = k.x; s[3] = k.y;
+    };
+    for (int c = cmax; c >= 0; --c) {
+        if (c <= cmax_r) {
+            const int64_t i0 = (int64_t)c * stride;
+            const int nseg = (int)__builtin_elementwise_min((int64_t)stride, m - i0);
+            // recompute the segment from its checkpoint
+            const double *cp = a.ckpt + ((int64_t)c * 4) * nr + r;
+            double s[4] = {cp[0], cp[nr], cp[2 * nr], cp[3 * nr]};
+            load_guess64<BK, CK, false>(B, a.bp, C, a.cp, a.f, sa, s[0], s[1]);
+            load_guess64<BK, CK, false>(B, a.bp, C, a.cp, a.f, sb, s[0], s[1]);
+            put(0, s);
+            for (int j = 1; j < nseg; ++j) {
+                double k[3][4], ys[3][4], n[4];
+                rk4_step64<BK, CK, false, MATH, 2>(B, a.bp, C, a.cp, a.f, K, sa, sb, dt, half,
+                                                   sixth, s, k, ys, n);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) s[q] = n[q];
+                put(j, s);
+            }
+            // and sweep it back; s is the last step's state, and each step
+            // loads the one before it while it runs.  The slots: sa serves
+            // stages 0 and 3, sb 1 and 2 (rk4_step64); sa is refilled after
+            // stage 0 for stage 3 and after stage 3 for the step before's
+            // stage 0 (its state is known), sb after stage 2 for that step's
+            // midpoint.
+            for (int j = nseg - 1; j >= 0; --j) {
+                double prev[4];
+                get(__builtin_elementwise_max(j - 1, 0), prev);
+                double R[LIN_N], Y[4], d[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) Y[q] = s[q];
+#pragma unroll
+                for (int st = 0; st < 4; ++st) {
+                    rhs64_with_lin<BK, CK>(B, a.bp, C, a.cp, a.f, (st == 0 || st == 3) ? sa : sb,
+                                           K, Y, R, d);
+                    if (st == 0) {
+                        vm_wait_upto<2>();
+                        prefetch64<BK, CK, false>(B, a.bp, C, a.cp, a.f, sa, sa,
+                                                  __builtin_fma(d[0], dt, s[0]),
+                                                  __builtin_fma(d[1], dt, s[1]));
+                    } else if (st == 2) {
+                        vm_wait_upto<0>();
+                        prefetch64<BK, CK, false>(B, a.bp, C, a.cp, a.f, sb, sb,
+                                                  0.5 * (s[0] + prev[0]), 0.5 * (s[1] + prev[1]));
+                    } else if (st == 3) {
+                        vm_wait_upto<0>();
+                        prefetch64<BK, CK, false>(B, a.bp, C, a.cp, a.f, sa, sa, prev[0],
+                                                  prev[1]);
+                    }
+                    if (st < 3) {
+                        const double hs = st < 2 ? half : dt;
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) Y[q] = __builtin_fma(d[q], hs, s[q]);
+#pragma unroll
+                        for (int f = 0; f < LIN_N; ++f)
+                            if (lin_field_used<BK, CK, false>(f))
+                                rec[st][lin_place<BK, CK, false>(f)][lane] = R[f];
+                    }
+                }
+                double w[4], kb[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) kb[q] = w[q] = lam[q] * sixth;
+#pragma unroll
+                for (int st = 3; st >= 0; --st) {
+                    if (st < 3) {
+#pragma unroll
+                        for (int f = 0; f < LIN_N; ++f)
+                            R[f] = lin_field_used<BK, CK, false>(f)
+                                       ? rec[st][lin_place<BK, CK, false>(f)][lane] : 0.0;
+                    }
+                    double z[4];
+                    lin_apply_flat<BK, CK>(R, C, a.grads, sums, kb, z);
+                    if (st > 0) {
+                        const double hs = st < 3 ? half : dt, cf = st > 1 ? 2.0 : 1.0;
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) kb[q] = __builtin_fma(z[q], hs, cf * w[q]);
+                    }
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) lam[q] += z[q];
+                }
+                const int64_t o = (i0 + j) * nr + r;
+                if (a.g_x) lam[0] += a.g_x[o];
+                if (a.g_y) lam[1] += a.g_y[o];
+                if (a.g_kx) lam[2] += a.g_kx[o];
+                if (a.g_ky) lam[3] += a.g_ky[o];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) s[q] = prev[q];
+            }
+        }
+    }
+    sums.finish(a.grads, (uint32_t)B.nx, (uint32_t)C.nx);
+    if (!active) return;
+    if (a.g_x0) a.g_x0[r] = lam[0];
+    if (a.g_y0) a.g_y0[r] = lam[1];
+    if (a.g_kx0) a.g_kx0[r] = lam[2];
+    if (a.g_ky0) a.g_ky0[r] = lam[3];
 }
 
 // The reverse sweep with the linearisations on waves of their own.  A
@@ -945,6 +1092,9 @@ hipError_t launch_adjoint(const AdjointArgs &a, int bk, int ck, int math, int wa
         else if (waves == 2)
             hipLaunchKernelGGL((adjoint_kernel<KK::bk, KK::ck, SH, KK::math>), grid,
                                dim3(ADJ_BLOCK), 0, stream, a);
+        else if constexpr (KK::bk == BK_CONSTANT || KK::bk == BK_ARRAY)
+            hipLaunchKernelGGL((adjoint_flat_kernel<KK::bk, KK::ck, KK::math>), grid, dim3(64),
+                               0, stream, a);
         else
             hipLaunchKernelGGL((adjoint_seq_kernel<KK::bk, KK::ck, SH, KK::math>), grid, dim3(64),
                                0, stream, a);

@@ -525,38 +525,132 @@ __device__ __forceinline__ void acc_add(CornerAcc &s, double *grad, uint32_t nx,
     s.d += vbar * ((1.0 - u) * w) + gx;
 }
 
-// acc_add for the current's two grids at once: u and v are gridded on the
-// same axes, so one cell test serves both (the test and its scalar branch
-// are half of acc_add's cost on the common path).  The sums of a grid not
-// wanted (null gu or gv) are formed and never added.  Used by the sweeps
-// that apply the vector-Jacobian product in the wave that forms it; the
-// four-wave sweep's chain ran slower with it (1.7 %) and keeps acc_add.
-__device__ __forceinline__ void acc_add_uv(CornerAcc &su, CornerAcc &sv, double *gu, double *gv,
-                                           uint32_t nx, const Cell64 &cell, double rxs,
-                                           double rys, double ubar, double uxbar, double uybar,
-                                           double vbar, double vxbar, double vybar)
+// The sums of the sweeps whose wave forms the vector-Jacobian products
+// (rhs64_vjp), which also loads cells while it accumulates.  vmcnt counts
+// atomics with loads and retires both in order, so an atomic issued when a
+// lane leaves its cell holds up the next cell's loads, for a microsecond and
+// more on a grid larger than L2; and with 64 lanes some lane leaves its cell
+// in most steps, a few lanes an instruction.  So the sums of a left cell go
+// to a queue in LDS, and once it holds a wave's worth, all lanes add one
+// entry each.  N arrays on one grid share the cell test (u and v; on shared
+// axes the depth too).
+constexpr int QUEUE64 = 128;               // entries; at most 63 before a push of up to 64
+
+template <int N>
+struct CellSums {
+    uint32_t iA = 0xFFFFFFFFu;             // no cell yet
+    double s[N][4] = {};                   // corners A, B, C, D
+};
+
+// A wave's queue in LDS: [1 + 4 N][QUEUE64] doubles, each entry's cell and
+// sums, and the number of entries after them.  The number lives in LDS as
+// well: lanes join and leave the sweep at their own steps, and a register
+// copy of a lane that sat out a push would be stale.
+template <int N>
+struct CellQueue {
+    double *e;
+    static constexpr int words = (1 + 4 * N) * QUEUE64 + 1;
+    __device__ __forceinline__ int *count() const
+    {
+        return reinterpret_cast<int *>(e + (words - 1));
+    }
+};
+
+// lanes of mask below this one
+__device__ __forceinline__ int lanes_below(uint64_t mask)
 {
-    const bool moved = cell.iA != su.iA;
-    if (__builtin_expect(wave_any(moved), 0)) {
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                          __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+// Adds the queue's last entries to the gradient grids (null: not wanted)
+// until fewer than `keep` are left.  Two neighbouring lanes take one entry,
+// corners A and D and then B and C, which lie next to each other: the two
+// atomics of a pair go out as one request (every request goes to memory, and
+// their number is what the drains cost).
+template <int N>
+__device__ __forceinline__ void queue_drain(CellQueue<N> &q, double *const (&grad)[N],
+                                            uint32_t nx, int keep)
+{
+    const uint64_t active = __builtin_amdgcn_ballot_w64(true);
+    const int n = __popcll(active), rank = lanes_below(active);
+    int count = *q.count();
+    // (an odd lane out, as when a wave's last lane drains alone, takes both
+    // corners by turns)
+    const int pairs = n > 1 ? n / 2 : 1, side = n > 1 ? rank & 1 : 0;
+    while (count >= keep) {
+        const int take = __builtin_elementwise_min(pairs, count);
+        if ((n > 1 ? rank / 2 : 0) < take) {
+            const double *e = q.e + (count - take + rank / 2);
+            const uint32_t iA = (uint32_t)__builtin_bit_cast(uint64_t, e[0]);
+            for (int d = side; d < 2; d += n > 1 ? 2 : 1) {
+                // sums A, B, C, D at 1 .. 4
+#pragma unroll
+                for (int k = 0; k < N; ++k) {
+                    if (!grad[k]) continue;
+                    unsafeAtomicAdd(grad[k] + iA + d, e[(4 * k + (d ? 4 : 1)) * QUEUE64]);
+                    unsafeAtomicAdd(grad[k] + iA + nx + d, e[(4 * k + (d ? 3 : 2)) * QUEUE64]);
+                }
+            }
+        }
+        count -= take;
+    }
+    *q.count() = count;
+}
+
+// Puts the sums of the lanes that have any into the queue (leave: the lanes
+// to take), and empties it down to less than a wave's worth.
+template <int N>
+__device__ __forceinline__ void queue_push(CellQueue<N> &q, CellSums<N> &s, bool leave,
+                                           double *const (&grad)[N], uint32_t nx)
+{
+    const bool put = leave & (s.iA != 0xFFFFFFFFu);
+    const uint64_t mask = __builtin_amdgcn_ballot_w64(put);
+    const int count = *q.count();
+    if (put) {
+        double *e = q.e + (count + lanes_below(mask));
+        e[0] = __builtin_bit_cast(double, (uint64_t)s.iA);
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) e[(1 + 4 * k + c) * QUEUE64] = s.s[k][c];
+    }
+    *q.count() = count + __popcll(mask);
+    // (other lanes of the wave read them back)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    queue_drain<N>(q, grad, nx, 64);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// Adds the cotangents of one query to the sums of its cell: vb on the
+// interpolated values, gxb and gyb on the cell-difference slopes.
+template <int N>
+__device__ __forceinline__ void sums_add(CellSums<N> &s, CellQueue<N> &q,
+                                         double *const (&grad)[N], uint32_t nx,
+                                         const Cell64 &cell, double rxs, double rys,
+                                         const double (&vb)[N], const double (&gxb)[N],
+                                         const double (&gyb)[N])
+{
+    if (__builtin_expect(__builtin_amdgcn_uicmp(cell.iA, s.iA, 33 /* != */) != 0, 0)) {
         __asm__ volatile("");
+        const bool moved = cell.iA != s.iA;
+        queue_push<N>(q, s, moved, grad, nx);
         if (moved) {
-            if (gu) acc_flush(su, gu, nx);
-            if (gv) acc_flush(sv, gv, nx);
-            su.iA = cell.iA;
-            sv.iA = cell.iA;
+            s = CellSums<N>{};
+            s.iA = cell.iA;
         }
     }
     const double u = cell.u, w = cell.w;
-    const double ux = uxbar * rxs, uy = uybar * rys;
-    su.a += ubar * ((1.0 - u) * (1.0 - w)) - ux - uy;
-    su.b += ubar * (u * (1.0 - w)) + uy;
-    su.c += ubar * (u * w);
-    su.d += ubar * ((1.0 - u) * w) + ux;
-    const double vx = vxbar * rxs, vy = vybar * rys;
-    sv.a += vbar * ((1.0 - u) * (1.0 - w)) - vx - vy;
-    sv.b += vbar * (u * (1.0 - w)) + vy;
-    sv.c += vbar * (u * w);
-    sv.d += vbar * ((1.0 - u) * w) + vx;
+    const double u1 = 1.0 - u, w1 = 1.0 - w;
+    const double wa = u1 * w1, wb = u * w1, wc = u * w, wd = u1 * w;   // corner weights
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        const double gx = gxb[k] * rxs, gy = gyb[k] * rys;
+        s.s[k][0] += vb[k] * wa - (gx + gy);
+        s.s[k][1] += vb[k] * wb + gy;
+        s.s[k][2] += vb[k] * wc;
+        s.s[k][3] += vb[k] * wd + gx;
+    }
 }
 
 // Gradient grids of an adjoint sweep (null: not wanted).
@@ -566,6 +660,49 @@ struct Grads64 {
 
 struct Accs64 {
     CornerAcc h, u, v;
+};
+
+// The sums and queues of a sweep with rhs64_vjp: of the depth alone and of
+// the current's two arrays, or of all three on shared axes.
+template <int BK, int CK, bool SH>
+struct Sums64 {
+    static constexpr int NB = SH ? 3 : 1;
+    static constexpr int words = (BK == BK_GRID ? CellQueue<NB>::words : 0) +
+                                 (!SH && CK == CK_GRID ? CellQueue<2>::words : 0);
+    CellSums<NB> b;
+    CellSums<2> c;
+    CellQueue<NB> qb;
+    CellQueue<2> qc;
+
+    // lds: `words` doubles of the wave's own
+    __device__ __forceinline__ explicit Sums64(double *lds)
+    {
+        qb.e = lds;
+        qc.e = lds + (BK == BK_GRID ? CellQueue<NB>::words : 0);
+        if (BK == BK_GRID) *qb.count() = 0;
+        if (!SH && CK == CK_GRID) *qc.count() = 0;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    // the last sums of every lane, called by the whole wave
+    __device__ __forceinline__ void finish(const Grads64 &Gr, uint32_t bnx, uint32_t cnx)
+    {
+        if constexpr (SH) {
+            double *const g[3] = {Gr.depth, Gr.u, Gr.v};
+            queue_push<3>(qb, b, true, g, bnx);
+            queue_drain<3>(qb, g, bnx, 1);
+        } else {
+            if constexpr (BK == BK_GRID) {
+                double *const g[1] = {Gr.depth};
+                queue_push<1>(qb, b, true, g, bnx);
+                queue_drain<1>(qb, g, bnx, 1);
+            }
+            if constexpr (CK == CK_GRID) {
+                double *const g[2] = {Gr.u, Gr.v};
+                queue_push<2>(qc, c, true, g, cnx);
+                queue_drain<2>(qc, g, cnx, 1);
+            }
+        }
+    }
 };
 
 // The linearisation of rhs64 at one stage point, as a record of LIN_N
@@ -622,7 +759,7 @@ template <int BK, int CK>
 __device__ __forceinline__ void lin_record(const FastConsts &K, const Val64 &h, const Val64 &u,
                                            const Val64 &v, const Cell64 &bc, const Cell64 &cc,
                                            bool okb, bool okc, double kx, double ky,
-                                           double R[LIN_N])
+                                           double R[LIN_N], double *cg_over_k = nullptr)
 {
     const double hh = h.val;
     const double k2 = __builtin_fma(kx, kx, ky * ky);
@@ -651,6 +788,7 @@ __device__ __forceinline__ void lin_record(const FastConsts &K, const Val64 &h, 
         const double Nq = 2.0 * S * (1.0 - q * T);
         const double cg_k = K.half_g * rs * (hh * Nq - N * cg * rs);
         const double tk = cg * rk;
+        if (cg_over_k) *cg_over_k = tk;
         const double a = cg_k - tk;
         R[0] = u.dx; R[1] = v.dx; R[2] = 0.0; R[3] = 0.0;
         R[4] = u.dy; R[5] = v.dy; R[6] = 0.0; R[7] = 0.0;
@@ -749,6 +887,71 @@ __device__ __forceinline__ void lin_apply(const double R[LIN_N], const Grid64Vie
     }
 }
 
+// The fields of a record that lin_apply reads, and where each stands among
+// them.
+template <int BK, int CK, bool SH>
+__device__ constexpr int lin_place(int f)
+{
+    int n = 0;
+    for (int g = 0; g < f; ++g) n += lin_field_used<BK, CK, SH>(g) ? 1 : 0;
+    return n;
+}
+
+// rhs64 and its linearisation at once, for a flat depth (depth_is_flat): the
+// record R and the derivatives, which share the field values and dispersion
+// terms.
+template <int BK, int CK>
+__device__ __forceinline__ void rhs64_with_lin(const Grid64View &B, const Grid64Ptrs &BP,
+                                               const Grid64View &C, const Grid64Ptrs &CP,
+                                               const Fields64 &F,
+                                               const Slots64<BK, CK, false> &sl,
+                                               const FastConsts &K, const double s[4],
+                                               double R[LIN_N], double d[4])
+{
+    static_assert(depth_is_flat<BK>(), "no depth gradient");
+    Point64 p;
+    auto eval = [&] {
+        double tk;
+        lin_record<BK, CK>(K, p.h, p.u, p.v, p.bc, p.cc, p.okb, p.okc, s[2], s[3], R, &tk);
+        d[0] = __builtin_fma(tk, s[2], p.u.val);
+        d[1] = __builtin_fma(tk, s[3], p.v.val);
+        d[2] = -(s[2] * p.u.gx + s[3] * p.v.gx);
+        d[3] = -(s[2] * p.u.gy + s[3] * p.v.gy);
+    };
+    const uint32_t off = point64_fast<BK, CK, false>(B, BP, C, CP, F, sl, s[0], s[1], p);
+    eval();
+    if (any_off64<BK, CK>(off)) {
+        __asm__ volatile("");
+        if (off >= OUT64) {
+            point64_full<BK, CK>(BP, CP, F, s[0], s[1], p);
+            eval();
+        }
+    }
+}
+
+// lin_apply for a flat depth, with the sums of a sweep that queues them
+template <int BK, int CK>
+__device__ __forceinline__ void lin_apply_flat(const double R[LIN_N], const Grid64View &C,
+                                               const Grads64 &Gr, Sums64<BK, CK, false> &sums,
+                                               const double g[4], double z[4])
+{
+    static_assert(depth_is_flat<BK>(), "no depth gradient");
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        z[i] = R[4 * i] * g[0] + R[4 * i + 1] * g[1];
+        if (i >= 2) z[i] += R[4 * i + 2] * g[2] + R[4 * i + 3] * g[3];
+    }
+    if constexpr (CK == CK_GRID) {
+        uint32_t ib, ic;
+        unpack_cells(R[27], ib, ic);
+        double *const grad[2] = {Gr.u, Gr.v};
+        if ((Gr.u || Gr.v) && ic != 0xFFFFFFFFu)
+            sums_add<2>(sums.c, sums.qc, grad, (uint32_t)C.nx, Cell64{ic, R[25], R[26]}, C.rxs,
+                        C.rys, {g[0], g[1]}, {-g[2] * R[21], -g[2] * R[22]},
+                        {-g[3] * R[21], -g[3] * R[22]});
+    }
+}
+
 // Vector-Jacobian product of rhs64 at (x, y, kx, ky): given the cotangent
 // (g0, g1, g2, g3) of (dx/dt, dy/dt, dkx/dt, dky/dt), adds the state
 // cotangent to (bx, by, bkx, bky) and the field-value cotangents to the
@@ -759,9 +962,9 @@ template <int BK, int CK, bool SH>
 __device__ __forceinline__ void rhs64_vjp(const Grid64View &B, const Grid64Ptrs &BP,
                                           const Grid64View &C, const Grid64Ptrs &CP,
                                           const Fields64 &F, const Slots64<BK, CK, SH> &sl,
-                                          const Grads64 &Gr, Accs64 &acc, const FastConsts &K,
-                                          double x, double y, double kx, double ky, double g0,
-                                          double g1, double g2, double g3, double &bx,
+                                          const Grads64 &Gr, Sums64<BK, CK, SH> &sums,
+                                          const FastConsts &K, double x, double y, double kx,
+                                          double ky, double g0, double g1, double g2, double g3, double &bx,
                                           double &by, double &bkx, double &bky)
 {
     // the field values as in rhs64: from the cells in hand, then the full
@@ -785,18 +988,22 @@ __device__ __forceinline__ void rhs64_vjp(const Grid64View &B, const Grid64Ptrs 
     double e, em;
     exp_pair(q, e, em, K);                               // e = exp(-2q), em = 1 - e
     const double ope = 1.0 + e;
-    const double D = rcp_nr(em * ope);
+    // 1/((1-e)(1+e)) and 1/sigma from one reciprocal square root, as in
+    // lin_record
+    const double gk = K.g * k;
+    const double W = rsq_nr((gk * em) * ope);
+    const double D = gk * (W * W);
     const double iope = em * D;
     const double T = em * iope;                         // tanh q
     const double S = (4.0 * e) * (iope * iope);         // sech^2 q
-    const double gkT = (K.g * k) * T;
-    const double rs = rsq_nr(gkT);                      // 1/sigma
+    const double rs = W * ope;                          // 1/sigma
     const double N = __builtin_fma(q, S, T);
     const double cg = K.half_g * N * rs;
     const double Nq = 2.0 * S * (1.0 - q * T);
     const double cg_k = K.half_g * rs * (hh * Nq - N * cg * rs);
     const double P = g0 * ex + g1 * ey;                 // cotangent of cg
     const double tk = cg * rk;
+    double hvb = 0.0, hgx = 0.0, hgy = 0.0;             // cotangents of the depth query
     if (depth_is_flat<BK>()) {
         // no depth gradient: the terms of c and of the depth cotangent vanish
         bkx += (cg_k * P) * ex + tk * (g0 - P * ex) - g2 * u.gx - g3 * u.gy;
@@ -805,7 +1012,7 @@ __device__ __forceinline__ void rhs64_vjp(const Grid64View &B, const Grid64Ptrs 
         by += g0 * u.dy + g1 * v.dy;
     } else {
         const double invT = (ope * ope) * D;            // 1/tanh q
-        const double sigma = gkT * rs;
+        const double sigma = (gk * T) * rs;
         const double c = (-2.0 * k) * e * sigma * D;
         const double sig_h = K.half_g * (k * k) * S * rs;   // d sigma / dh
         const double cg_h = K.half_g * rs * (k * Nq - N * sig_h * rs);
@@ -818,13 +1025,30 @@ __device__ __forceinline__ void rhs64_vjp(const Grid64View &B, const Grid64Ptrs 
         bky += (cg_k * P) * ey + tk * (g1 - P * ey) + (c_k * cbar) * ey - g2 * v.gx - g3 * v.gy;
         bx += hbar * h.dx + g0 * u.dx + g1 * v.dx;
         by += hbar * h.dy + g0 * u.dy + g1 * v.dy;
-        // (a state of a finite row never errs; the guards keep a misuse in bounds)
-        if (BK == BK_GRID && Gr.depth && okb)
-            acc_add(acc.h, Gr.depth, (uint32_t)B.nx, bc, B.rxs, B.rys, hbar, g2 * c, g3 * c);
+        hvb = hbar;
+        hgx = g2 * c;
+        hgy = g3 * c;
     }
-    if (CK == CK_GRID && okc)
-        acc_add_uv(acc.u, acc.v, Gr.u, Gr.v, (uint32_t)C.nx, cc, C.rxs, C.rys, g0, -g2 * kx,
-                   -g3 * kx, g1, -g2 * ky, -g3 * ky);
+    // (a state of a finite row never errs; the guards keep a misuse in bounds)
+    if constexpr (SH) {
+        double *const g[3] = {Gr.depth, Gr.u, Gr.v};
+        if ((Gr.depth || Gr.u || Gr.v) && okb && okc)
+            sums_add<3>(sums.b, sums.qb, g, (uint32_t)C.nx, cc, C.rxs, C.rys, {hvb, g0, g1},
+                        {hgx, -g2 * kx, -g2 * ky}, {hgy, -g3 * kx, -g3 * ky});
+    } else {
+        if constexpr (BK == BK_GRID) {
+            double *const g[1] = {Gr.depth};
+            if (Gr.depth && okb)
+                sums_add<1>(sums.b, sums.qb, g, (uint32_t)B.nx, bc, B.rxs, B.rys, {hvb}, {hgx},
+                            {hgy});
+        }
+        if constexpr (CK == CK_GRID) {
+            double *const g[2] = {Gr.u, Gr.v};
+            if ((Gr.u || Gr.v) && okc)
+                sums_add<2>(sums.c, sums.qc, g, (uint32_t)C.nx, cc, C.rxs, C.rys, {g0, g1},
+                            {-g2 * kx, -g2 * ky}, {-g3 * kx, -g3 * ky});
+        }
+    }
 }
 
 }  // namespace mr
