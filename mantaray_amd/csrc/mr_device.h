@@ -617,7 +617,12 @@ __device__ __forceinline__ void exp_pair_full(double q, double &e, double &em,
 // point: depth h (NaN where the bathymetry errs), its gradient, the current
 // and its gradients, and okc = false where the current errs.
 
-template <int MATH>
+// FLAT: the depth's gradient is zero everywhere (ConstantDepth, ArrayDepth);
+// STILL: the current's is (ConstantCurrent).  Their terms are exact zeros
+// wherever the rest is finite, and a NaN W, which any error leaves, still
+// makes every derivative NaN; left out, they save 4 of about 65 operations
+// each.
+template <int MATH, bool FLAT, bool STILL>
 __device__ __forceinline__ void odes(const FastConsts &K, double h, double hx, double hy,
                                      bool okc, double u, double v, double ux, double uy,
                                      double vx, double vy, double kx, double ky, double &dx,
@@ -662,8 +667,8 @@ __device__ __forceinline__ void odes(const FastConsts &K, double h, double hx, d
         const double c = (K.g * k) * (k * (-2.0 * (ei * W)));
         dx = __builtin_fma(cgr, kx, u);
         dy = __builtin_fma(cgr, ky, v);
-        dkx = __builtin_fma(-ky, vx, __builtin_fma(-kx, ux, c * hx));    // :146-147
-        dky = __builtin_fma(-ky, vy, __builtin_fma(-kx, uy, c * hy));
+        dkx = FLAT ? W * 0.0 : c * hx;                      // :146-147
+        dky = FLAT ? dkx : c * hy;
     } else {
         // Every provider error, h <= 0 (or NaN), k <= 0 (or NaN) and a
         // non-finite k*h give all-NaN derivatives in the reference (an
@@ -701,10 +706,21 @@ __device__ __forceinline__ void odes(const FastConsts &K, double h, double hx, d
         const double c = (-K.qg * k2) * (ei4 * W2);
         dx = __builtin_fma(cgr, kx, u);                     // cg cos(atan2(ky, kx)) + u
         dy = __builtin_fma(cgr, ky, v);
-        // (c hx - kx ux) - ky vx with one rounding per term
-        dkx = __builtin_fma(-ky, vx, __builtin_fma(-kx, ux, c * hx));
-        dky = __builtin_fma(-ky, vy, __builtin_fma(-kx, uy, c * hy));
+        dkx = FLAT ? W2 * 0.0 : c * hx;
+        dky = FLAT ? dkx : c * hy;
     }
+    if (!STILL) {
+        // (c hx - kx ux) - ky vx with one rounding per term
+        dkx = __builtin_fma(-ky, vx, __builtin_fma(-kx, ux, dkx));
+        dky = __builtin_fma(-ky, vy, __builtin_fma(-kx, uy, dky));
+    }
+}
+
+// FLAT of a depth kind
+template <int BK>
+__device__ constexpr bool depth_is_flat()
+{
+    return BK == BK_CONSTANT || BK == BK_ARRAY;
 }
 
 // The gridded queries for a target inside the slot's cell and on none of
@@ -899,14 +915,14 @@ __device__ __forceinline__ void rhs_rec(const BathyView &B, const BathyPtrs &BP,
     const float off = rec_fast<BK, CK, SH>(ss, x, y, h, hx, hy, u, v, ux, uy, vx, vy);
     if (BK != BK_GRID) h = bathy_query<BK>(B, BP, bs, x, y, hx, hy);
     if (CK != CK_GRID) current_query<CK>(C, CP, cs, x, y, u, v, ux, uy, vx, vy);
-    odes<MATH>(K, h, hx, hy, true, u, v, ux, uy, vx, vy, kx, ky, dx, dy, dkx, dky);
+    odes<MATH, depth_is_flat<BK>(), CK == CK_CONSTANT>(K, h, hx, hy, true, u, v, ux, uy, vx, vy, kx, ky, dx, dy, dkx, dky);
     if (BK == BK_GRID || CK == CK_GRID) {
         if (__builtin_expect(__builtin_amdgcn_fcmpf(off, 0.0f, 14) != 0, 0)) {
             __asm__ volatile("");
             if (!(off == 0.0f)) {
                 const double h2 = bathy_query<BK>(B, BP, bs, x, y, hx, hy);
                 const bool okc = current_query<CK>(C, CP, cs, x, y, u, v, ux, uy, vx, vy);
-                odes<MATH>(K, h2, hx, hy, okc, u, v, ux, uy, vx, vy, kx, ky, dx, dy, dkx, dky);
+                odes<MATH, depth_is_flat<BK>(), CK == CK_CONSTANT>(K, h2, hx, hy, okc, u, v, ux, uy, vx, vy, kx, ky, dx, dy, dkx, dky);
             }
         }
     }
@@ -932,21 +948,21 @@ __device__ __forceinline__ void rhs(const BathyView &B, const BathyPtrs &BP, Bat
                                        : bathy_query<BK>(B, BP, bs, x, y, hx, hy);
         const bool okc = CK == CK_GRID ? current_fast(cs, x, y, u, v, ux, uy, vx, vy, sc)
                                        : current_query<CK>(C, CP, cs, x, y, u, v, ux, uy, vx, vy);
-        odes<MATH>(K, h, hx, hy, okc, u, v, ux, uy, vx, vy, kx, ky, dx, dy, dkx, dky);
+        odes<MATH, depth_is_flat<BK>(), CK == CK_CONSTANT>(K, h, hx, hy, okc, u, v, ux, uy, vx, vy, kx, ky, dx, dy, dkx, dky);
         const bool slow = sb | sc;
         if (__builtin_expect(wave_any(slow), 0)) {
             __asm__ volatile("");
             if (slow) {
                 const double h2 = bathy_query<BK>(B, BP, bs, x, y, hx, hy);
                 const bool okc2 = current_query<CK>(C, CP, cs, x, y, u, v, ux, uy, vx, vy);
-                odes<MATH>(K, h2, hx, hy, okc2, u, v, ux, uy, vx, vy, kx, ky, dx, dy, dkx, dky);
+                odes<MATH, depth_is_flat<BK>(), CK == CK_CONSTANT>(K, h2, hx, hy, okc2, u, v, ux, uy, vx, vy, kx, ky, dx, dy, dkx, dky);
             }
         }
         return;
     }
     const double h = bathy_query<BK>(B, BP, bs, x, y, hx, hy);       // odes :120-127
     const bool okc = current_query<CK>(C, CP, cs, x, y, u, v, ux, uy, vx, vy);   // :130
-    odes<MATH>(K, h, hx, hy, okc, u, v, ux, uy, vx, vy, kx, ky, dx, dy, dkx, dky);
+    odes<MATH, depth_is_flat<BK>(), CK == CK_CONSTANT>(K, h, hx, hy, okc, u, v, ux, uy, vx, vy, kx, ky, dx, dy, dkx, dky);
 }
 
 // all four NaN: fmin returns its non-NaN operand, so the minimum of four is

@@ -467,7 +467,7 @@ __device__ __forceinline__ void rhs64(const Grid64View &B, const Grid64Ptrs &BP,
 {
     Point64 p;
     auto system = [&] {
-        odes<MATH>(K, p.okb ? p.h.val : MR_NAN, p.h.gx, p.h.gy, p.okc, p.u.val, p.v.val, p.u.gx,
+        odes<MATH, depth_is_flat<BK>(), CK == CK_CONSTANT>(K, p.okb ? p.h.val : MR_NAN, p.h.gx, p.h.gy, p.okc, p.u.val, p.v.val, p.u.gx,
                    p.u.gy, p.v.gx, p.v.gy, kx, ky, dx, dy, dkx, dky);
     };
     const uint32_t off = point64_fast<BK, CK, SH>(B, BP, C, CP, F, sl, x, y, p);
@@ -728,20 +728,12 @@ __device__ __forceinline__ void unpack_cells(double v, uint32_t &b, uint32_t &c)
     c = (uint32_t)(u >> 32);
 }
 
-// Whether the depth has no gradient anywhere (ConstantDepth, ArrayDepth:
-// their queries return zero slopes and zero derivatives), so that every
-// depth-gradient term of the linearisation vanishes.
-template <int BK>
-__device__ constexpr bool depth_is_flat()
-{
-    return BK == BK_CONSTANT || BK == BK_ARRAY;
-}
-
 // Whether lin_apply reads field f of a linearisation record for the field
-// kinds BK, CK (the only fields the ring is given): the depth terms (16-20,
-// 23, 24) for gridded depth, the current's (21, 22, 25, 26) for a gridded
-// current, and with a flat depth not the four zeros of M's x and y rows.  On
-// shared cells (SH) the current's fractions serve the depth too.
+// kinds BK, CK (the only fields a ring is given): the depth terms (16-20, 23,
+// 24) for gridded depth, the current's (21, 22, 25, 26) for a gridded
+// current, and with a flat depth (depth_is_flat: zero slopes and derivatives)
+// not the four zeros of M's x and y rows.  On shared cells (SH) the current's
+// fractions serve the depth too.
 template <int BK, int CK, bool SH>
 __device__ constexpr bool lin_field_used(int f)
 {
