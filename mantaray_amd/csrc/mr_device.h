@@ -896,16 +896,53 @@ __device__ __forceinline__ bool wave_any(bool c)
     return m != 0;
 }
 
+// Where the full queries of rhs_rec find the fields: in the registers of the
+// kernel, or loaded again when they run (rarely), which frees 16 to 60
+// registers between times.  That matters where it keeps a kernel within 256
+// registers, two waves a SIMD: the batch kernel on both record modes, and
+// the trace on two fields' own records once there are that many waves (the
+// grids of rk4_step_rec's comment, end states: 72,000 rays 5.05 -> 4.03 ms;
+// at 30,011 rays it costs 2 %).  The trace on shared records is within them
+// anyway and ran 1.3 % slower with reloaded views (65,536 rays x 5000 steps).
+struct FullInPlace {
+    const BathyView &b;
+    const BathyPtrs &bp_;
+    const CurrentView &c;
+    const CurrentPtrs &cp_;
+    __device__ __forceinline__ const BathyView &B() const { return b; }
+    __device__ __forceinline__ const CurrentView &C() const { return c; }
+    __device__ __forceinline__ const BathyPtrs &bp() const { return bp_; }
+    __device__ __forceinline__ const CurrentPtrs &cp() const { return cp_; }
+};
+struct FullViews {                     // the views again, the pointers in place
+    const void *b;
+    const BathyPtrs &bp_;
+    const void *c;
+    const CurrentPtrs &cp_;
+    __device__ __forceinline__ BathyView B() const { return load_view<BathyView>(b); }
+    __device__ __forceinline__ CurrentView C() const { return load_view<CurrentView>(c); }
+    __device__ __forceinline__ const BathyPtrs &bp() const { return bp_; }
+    __device__ __forceinline__ const CurrentPtrs &cp() const { return cp_; }
+};
+template <class Scene>
+struct FullScene {                     // all of it, from a lane's scene
+    const Scene *s;
+    __device__ __forceinline__ BathyView B() const { return load_view<BathyView>(s->B); }
+    __device__ __forceinline__ CurrentView C() const { return load_view<CurrentView>(s->C); }
+    __device__ __forceinline__ BathyPtrs bp() const { return s->bp; }
+    __device__ __forceinline__ CurrentPtrs cp() const { return s->cp; }
+};
+
 // WaveRayPath::system (wave_ray_path.rs:220-234) around odes (:118-150) with
 // the cell records in hand: every lane evaluates from them in one block of
 // straight-line code; lanes outside a record's fast region evaluate again
 // through the full queries (bathy_query, current_query), which find and load
 // their cells and handle nodes and errors.  An analytic field is evaluated
 // in place.
-template <int BK, int CK, bool SH, int MATH>
+template <int BK, int CK, bool SH, int MATH, class Full>
 __device__ __forceinline__ void rhs_rec(const BathyView &B, const BathyPtrs &BP,
                                         const CurrentView &C, const CurrentPtrs &CP,
-                                        const RecSlot<BK, CK, SH> &ss, const FastConsts &K,
+                                        const Full &full, const RecSlot<BK, CK, SH> &ss, const FastConsts &K,
                                         double x, double y, double kx, double ky, double &dx,
                                         double &dy, double &dkx, double &dky)
 {
@@ -920,8 +957,9 @@ __device__ __forceinline__ void rhs_rec(const BathyView &B, const BathyPtrs &BP,
         if (__builtin_expect(__builtin_amdgcn_fcmpf(off, 0.0f, 14) != 0, 0)) {
             __asm__ volatile("");
             if (!(off == 0.0f)) {
-                const double h2 = bathy_query<BK>(B, BP, bs, x, y, hx, hy);
-                const bool okc = current_query<CK>(C, CP, cs, x, y, u, v, ux, uy, vx, vy);
+                const double h2 = bathy_query<BK>(full.B(), full.bp(), bs, x, y, hx, hy);
+                const bool okc =
+                    current_query<CK>(full.C(), full.cp(), cs, x, y, u, v, ux, uy, vx, vy);
                 odes<MATH, depth_is_flat<BK>(), CK == CK_CONSTANT>(K, h2, hx, hy, okc, u, v, ux, uy, vx, vy, kx, ky, dx, dy, dkx, dky);
             }
         }

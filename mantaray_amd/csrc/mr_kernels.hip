@@ -170,12 +170,12 @@ __device__ __forceinline__ void rec_refill(const BathyView &B, const CurrentView
     }
 }
 
-template <int BK, int CK, bool SH, int MATH, bool DY, int NST, class OnStop>
+template <int BK, int CK, bool SH, int MATH, bool DY, int NST, class Full, class OnStop>
 __device__ __forceinline__ void rk4_step_rec(const BathyView &B, const BathyPtrs &BP,
                                              const CurrentView &C, const CurrentPtrs &CP,
-                                             const RecPtrs &R, RecSlot<BK, CK, SH> &sa,
-                                             RecSlot<BK, CK, SH> &sb, const FastConsts &K,
-                                             double &px, double &py, double dt, double half,
+                                             const Full &full, const RecPtrs &R,
+                                             RecSlot<BK, CK, SH> &sa, RecSlot<BK, CK, SH> &sb,
+                                             const FastConsts &K, double &px, double &py, double dt, double half,
                                              double sixth, float g1, float g3, int solout,
                                              double x, double y, double kx, double ky,
                                              double o[4], bool &stop_before, OnStop &&on_stop)
@@ -196,8 +196,8 @@ __device__ __forceinline__ void rk4_step_rec(const BathyView &B, const BathyPtrs
                                    __builtin_fmaf((float)py, g, (float)y));
         }
         double dx, dy, dkx, dky;
-        rhs_rec<BK, CK, SH, MATH>(B, BP, C, CP, (st == 0 || st == 3) ? sa : sb, K, sx, sy, skx,
-                                  sky, dx, dy, dkx, dky);
+        rhs_rec<BK, CK, SH, MATH>(B, BP, C, CP, full, (st == 0 || st == 3) ? sa : sb, K, sx, sy,
+                                  skx, sky, dx, dy, dkx, dky);
         px = dx; py = dy;
         if (st == 0) {
             // the MR_SOLOUT_NEXT_DERIV test, as in rk4_step
@@ -276,7 +276,10 @@ __device__ __forceinline__ void store_row_nt(__amdgpu_buffer_rsrc_t d, uint32_t 
 // stores every row, with no branch around the stores.  OUT: 0 no
 // trajectories, 1 all four components, 2 any subset.
 // REC: REC_NONE (rk4_step, no cell records), REC_SHARED or REC_OWN
-// (rk4_step_rec on the shared-cell records, or on each gridded field's own);
+// (rk4_step_rec on the shared-cell records, or on each gridded field's own),
+// or REC_OWN_MANY: with the records of two fields, REC_OWN's views in
+// registers push the kernel past 256 of them, to one wave a SIMD, which is
+// the faster form only while there is no second one;
 // DYAD: dt a power of two (rk4_step_rec's DY).
 template <int BK, int CK, int MATH, int OUT, int REC, bool DYAD>
 __global__ void __launch_bounds__(256) trace_kernel(TraceArgs a)
@@ -391,10 +394,16 @@ __global__ void __launch_bounds__(256) trace_kernel(TraceArgs a)
                     }
                     len = -(len + 1);
                 };
+                auto full = [&] {
+                    if constexpr (REC == REC_OWN_MANY)
+                        return FullViews{a.B, a.bp, a.C, a.cp};
+                    else
+                        return FullInPlace{B, a.bp, C, a.cp};
+                };
                 if constexpr (REC != REC_NONE)
                     rk4_step_rec<BK, CK, SH, MATH, DYAD, NST>(
-                        B, a.bp, C, a.cp, a.rec, sa, sb, K, px, py, dt, half, sixth, g1, g3, so,
-                        x, y, kx, ky, o, stop_before, on_stop);
+                        B, a.bp, C, a.cp, full(), a.rec, sa, sb, K, px, py, dt, half, sixth, g1,
+                        g3, so, x, y, kx, ky, o, stop_before, on_stop);
                 else
                     rk4_step<BK, CK, MATH>(B, a.bp, bn, C, a.cp, cn, K, px, py, dt, half,
                                            sixth, so, x, y, kx, ky, o, stop_before, on_stop);
@@ -465,6 +474,7 @@ __global__ void __launch_bounds__(256) batch_kernel(BatchArgs a)
     CurrentSlot cn;
     RecSlot<BK, CK, SH> sa, sb;
     RecPtrs rec{};
+    const SceneDesc *scene = nullptr;
     double x = 0.0, y = 0.0, kx = 0.0, ky = 0.0, px = 0.0, py = 0.0;
     double dt = 0.0, half = 0.0, sixth = 0.0;
     int64_t local = 0, n_steps = 0, step = 0, len = 1;
@@ -499,6 +509,7 @@ __global__ void __launch_bounds__(256) batch_kernel(BatchArgs a)
                     step = 0; len = 1; px = 0.0; py = 0.0;
                     if (REC != REC_NONE) {
                         rec = S->rec;
+                        scene = S;
                         rec_prefetch<BK, CK, SH>(B, C, rec, sa, sb, x, y);
                     } else {
                         bn = BathySlot{};
@@ -520,7 +531,7 @@ __global__ void __launch_bounds__(256) batch_kernel(BatchArgs a)
                 bool stop_before;
                 if constexpr (REC != REC_NONE)
                     rk4_step_rec<BK, CK, SH, MATH, false, 0>(
-                        B, bp, C, cp, rec, sa, sb, K, px, py, dt, half, sixth, (float)dt,
+                        B, bp, C, cp, FullScene<SceneDesc>{scene}, rec, sa, sb, K, px, py, dt, half, sixth, (float)dt,
                         (float)(dt + half), a.solout, x, y, kx, ky, o, stop_before, [] {});
                 else
                     rk4_step<BK, CK, MATH>(B, bp, bn, C, cp, cn, K, px, py, dt, half, sixth,
@@ -794,6 +805,9 @@ hipError_t launch_trace(const TraceArgs &a, int bk, int ck, int math, int block,
         if constexpr (any)
             if (a.records == REC_NONE)
                 return launch(k, std::integral_constant<int, REC_NONE>{}, std::false_type{});
+        if constexpr (both)
+            if (a.records == REC_OWN_MANY)
+                return by_step(k, std::integral_constant<int, REC_OWN_MANY>{});
         by_step(k, std::integral_constant<int, REC_OWN>{});
     });
     return hipGetLastError();

@@ -131,3 +131,29 @@ def test_grid_past_the_record_limit(mr, oracle_mod, nx):
     for k, tol in (("x", 1e-6), ("y", 1e-6), ("kx", 1e-9), ("ky", 1e-9)):
         assert np.array_equal(np.isnan(got[k]), np.isnan(ref[k]))
         assert np.nanmax(np.abs(got[k] - ref[k])) <= tol
+
+
+@pytest.mark.parametrize("n_rays", [65_536, 65_537, 70_001])
+def test_more_waves_than_simds(mr, oracle_mod, n_rays):
+    """Two gridded fields on grids of their own, on both sides of the ray
+    count at which waves share SIMDs (256 CUs x 256 lanes): the same rays as
+    in a launch of a few give the same end states bitwise, in single traces
+    and in batches of two scenes."""
+    import torch
+
+    from mantaray_amd.batch import Batch
+    ((b, c), _), s = _fields(mr, oracle_mod, "two grids", 34, 9, "jittered")
+    few = mr.trace_many(b, c, *s.T, 0.0, 11.0, 0.7, trajectories=False)
+    i = np.arange(n_rays) % s.shape[0]
+    ic = [torch.tensor(np.ascontiguousarray(s[i, q]), device="cuda:0") for q in range(4)]
+    many = mr.trace_many_device(b, c, *ic, 0.0, 11.0, 0.7, trajectories=False)
+    assert np.array_equal(many["len"].cpu().numpy(), few["len"][i])
+    assert np.array_equal(many["end"].cpu().numpy(), few["end"][i], equal_nan=True)
+    half = n_rays // 2
+    batch = Batch([{"bathymetry": b, "current": c, "t0": 0.0, "t_end": 11.0, "dt": 0.7,
+                    **{k: v[p] for k, v in zip(("x0", "y0", "kx0", "ky0"), ic)}}
+                   for p in (slice(0, half), slice(half, None))])
+    batch.run()
+    end = torch.cat([o["end"] for o in batch.results()]).cpu().numpy()
+    assert np.array_equal(end, few["end"][i], equal_nan=True)
+    batch.close()
