@@ -444,13 +444,15 @@ __device__ __forceinline__ void point64_full(const Grid64Ptrs &BP, const Grid64P
 }
 
 // Whether any lane must take point64_full, as one compare and one scalar
-// branch: the mask intrinsic is not folded into the test inside the block,
-// which is laid out after the loop.
+// branch: the mask intrinsic is not folded into the test inside the block.
+// The callers mark it unlikely (an expectation inside this function would be
+// lost when it is inlined), so that the block is laid out after the loop; in
+// its place it costs a taken branch at every evaluation.
 template <int BK, int CK>
 __device__ __forceinline__ bool any_off64(uint32_t off)
 {
     if (BK != BK_GRID && CK != CK_GRID) return false;
-    return __builtin_expect(__builtin_amdgcn_uicmp(off, OUT64, 35 /* >= */) != 0, 0);
+    return __builtin_amdgcn_uicmp(off, OUT64, 35 /* >= */) != 0;
 }
 
 // WaveRayPath::system in fp64 mode, with the cells held in sl.  As rhs_rec()
@@ -472,7 +474,7 @@ __device__ __forceinline__ void rhs64(const Grid64View &B, const Grid64Ptrs &BP,
     };
     const uint32_t off = point64_fast<BK, CK, SH>(B, BP, C, CP, F, sl, x, y, p);
     system();
-    if (any_off64<BK, CK>(off)) {
+    if (__builtin_expect(any_off64<BK, CK>(off), 0)) {
         __asm__ volatile("");
         if (off >= OUT64) {
             point64_full<BK, CK>(BP, CP, F, x, y, p);
@@ -838,7 +840,7 @@ __device__ __forceinline__ void rhs64_lin(const Grid64View &B, const Grid64Ptrs 
     Point64 p;
     const uint32_t off = point64_fast<BK, CK, SH>(B, BP, C, CP, F, sl, x, y, p);
     lin_record<BK, CK>(K, p.h, p.u, p.v, p.bc, p.cc, p.okb, p.okc, kx, ky, R);
-    if (any_off64<BK, CK>(off)) {
+    if (__builtin_expect(any_off64<BK, CK>(off), 0)) {
         __asm__ volatile("");
         if (off >= OUT64) {
             point64_full<BK, CK>(BP, CP, F, x, y, p);
@@ -912,7 +914,7 @@ __device__ __forceinline__ void rhs64_with_lin(const Grid64View &B, const Grid64
     };
     const uint32_t off = point64_fast<BK, CK, false>(B, BP, C, CP, F, sl, s[0], s[1], p);
     eval();
-    if (any_off64<BK, CK>(off)) {
+    if (__builtin_expect(any_off64<BK, CK>(off), 0)) {
         __asm__ volatile("");
         if (off >= OUT64) {
             point64_full<BK, CK>(BP, CP, F, s[0], s[1], p);
@@ -964,7 +966,7 @@ __device__ __forceinline__ void rhs64_vjp(const Grid64View &B, const Grid64Ptrs 
     // the accumulation below run once, after both)
     Point64 p;
     const uint32_t off = point64_fast<BK, CK, SH>(B, BP, C, CP, F, sl, x, y, p);
-    if (any_off64<BK, CK>(off)) {
+    if (__builtin_expect(any_off64<BK, CK>(off), 0)) {
         __asm__ volatile("");
         if (off >= OUT64) point64_full<BK, CK>(BP, CP, F, x, y, p);
     }
