@@ -157,3 +157,46 @@ def test_more_waves_than_simds(mr, oracle_mod, n_rays):
     end = torch.cat([o["end"] for o in batch.results()]).cpu().numpy()
     assert np.array_equal(end, few["end"][i], equal_nan=True)
     batch.close()
+
+
+@pytest.mark.parametrize("a0,sp,n", [(-1000.0, 0.1, 41), (-7.0, 7.0, 3), (1.0e7, 3.3, 17),
+                                     (3.0e-30, 7.0e-31, 9), (2.0, -0.7, 12), (-2.0e30, 1.7e29, 30)])
+def test_cell_lines_of_awkward_axes(mr, oracle_mod, a0, sp, n):
+    """Points within two units in the last place of every cell line, in f32
+    and f64, on axes that cross zero, lie far from it, descend, or have
+    extreme spacings: the cell each falls in, seen in the cell's slopes, is
+    the oracle's.  A neighbouring cell's slope differs by order one; the
+    tolerance is that of the right-hand-side tests."""
+    x = a0 + sp * np.arange(n)
+    x = x.astype(np.float32).astype(np.float64)
+    y = np.array([0.0, 10.0, 20.0])
+    rng = np.random.default_rng(n)
+    depth = rng.uniform(8.0, 30.0, (3, n))
+    U, V = rng.uniform(-1.0, 1.0, (2, 3, n))
+    px = []
+    for f in (np.float32, np.float64):
+        for to in (-np.inf, np.inf):
+            q = x.astype(f)
+            for _ in range(3):
+                px.append(q.astype(np.float64))
+                q = np.nextafter(q, f(to))
+    px = np.concatenate(px)
+    s = np.stack([px, np.full(px.size, 6.5), np.full(px.size, 0.07),
+                  np.full(px.size, -0.03)], axis=1)
+    y32 = y.astype(np.float32)
+    for grid in ("depth", "current"):
+        if grid == "depth":
+            b, ob = (g(x.astype(np.float32), y32, depth)
+                     for g in (mr.Bathymetry.from_arrays, oracle_mod.Bathymetry.grid))
+            c, oc = mr.Current.constant(0.3, -0.2), oracle_mod.Current.constant(0.3, -0.2)
+        else:
+            b, ob = mr.Bathymetry.constant(12.5), oracle_mod.Bathymetry.constant(12.5)
+            c, oc = (g(x, y, U, V) for g in (mr.Current.from_arrays, oracle_mod.Current.grid))
+        ds = mr.rhs(b, c, s, math="literal")
+        ref, _ = oracle_mod.system_many(ob, oc, s)
+        assert np.array_equal(np.isnan(ds), np.isnan(ref)), grid
+        assert np.isfinite(ref).any(), grid
+        ok = np.isfinite(ref)
+        scale = np.max(np.abs(np.where(ok, ref, 0.0)), axis=0)
+        assert np.array_equal(ds[~ok & ~np.isnan(ref)], ref[~ok & ~np.isnan(ref)]), grid
+        assert np.max(np.abs(ds - ref)[ok] / np.broadcast_to(scale, ds.shape)[ok]) <= 1e-12, grid
