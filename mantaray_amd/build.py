@@ -6,7 +6,8 @@ compiles the HIP kernels, the NetCDF-3 reader and the C ABI with hipcc into
 mantaray_amd/libmantaray_hip.so (one object per source, compiled in
 parallel under mantaray_amd/_build/, then linked).  Floating-point flags:
 -ffp-contract=off on host and device (no FMA contraction, as rustc never
-contracts), no fast-math, IEEE f32 division/sqrt and f32 denormals (the HIP
+contracts; mr_adjoint.hip, whose fp64 mode has its own roundings, turns
+contraction within an expression on by pragma), no fast-math, IEEE f32 division/sqrt and f32 denormals (the HIP
 defaults).
 
 Packed FP32 instructions are disabled for the device code with the target

@@ -4,10 +4,13 @@
 //   trace64_kernel   ManyRays::trace_many (src/ray.rs:98-127) with every
 //                    field query in f64 (mr_device64.h); optionally stores the
 //                    state every `stride` steps (checkpoints).
-//   adjoint_kernel   reverse sweep of the discrete adjoint of the RK4 loop:
+//   adjoint_lin_kernel, adjoint_kernel, adjoint_flat_kernel,
+//   adjoint_seq_kernel
+//                    reverse sweep of the discrete adjoint of the RK4 loop:
 //                    gradients of a loss on the rows (or the last row) with
 //                    respect to the initial states and to the gridded depth,
-//                    u and v values.
+//                    u and v values; on four waves, two or one per 64 rays,
+//                    by the size of the launch.
 //   rhs64_kernel     WaveRayPath::system in fp64 mode at a batch of states.
 //   fill             constant fill (gradient grids start at zero).
 //
@@ -77,6 +80,12 @@ hipError_t adjoint_scratch(void **ptr)
 // cells its slot holds, so no slot is ever copied.  Every evaluation tests
 // the cells it uses and queries again where they are not the target's, so
 // the slots choose only what is waited for, never a value.
+//
+// It is bound by its own instruction issue, as trace_kernel's step: cell
+// tests on one compare, corners as pairs and one slot for fields on shared
+// axes took a forward and sweep of 16,384 rays x 2000 steps 6.18 -> 5.66 ms
+// and one of 4,099 x 600 on a gridded depth and current 3.11 -> 2.54; FMA
+// contraction took these to 5.46 and 2.38.
 //
 // Before each refill the step waits for the vector memory operations issued
 // up to then but the last NST (the caller's stores after the step before,
@@ -464,7 +473,9 @@ __global__ void __launch_bounds__(ADJ_BLOCK) adjoint_kernel(AdjointArgs a)
 // (adjoint_kernel) keep the recomputing wave about half idle, since a sweep
 // step costs about twice a forward step, and each holds a SIMD of its own;
 // once the launch has waves enough to fill every SIMD several times over,
-// one wave doing both takes about a quarter less SIMD time.
+// one wave doing both takes about a quarter less SIMD time.  Launched for
+// depths with a gradient; a flat depth has adjoint_flat_kernel (65,536 rays x
+// 1000 steps 4.1 ms against 5.9 for a gridded depth here).
 template <int BK, int CK, bool SH, int MATH>
 __global__ void __launch_bounds__(64) adjoint_seq_kernel(AdjointArgs a)
 {
@@ -567,7 +578,9 @@ __global__ void __launch_bounds__(64) adjoint_seq_kernel(AdjointArgs a)
 // the queued sums, on a 2048 x 2048 current, forward and sweep 89.6 -> 64.7
 // ms (the forward is 13.5 of them); the queue alone, before its pairs shared
 // requests and with the stored stage points, cost 2 ms.  What is left is the
-// issue of about 1350 vector instructions a step.
+// issue of about 1350 vector instructions a step (63 to 64 ms with the
+// later changes to every fp64 evaluation: zero terms left out, slow paths
+// out of line).
 template <int BK, int CK, int MATH>
 __global__ void __launch_bounds__(64) adjoint_flat_kernel(AdjointArgs a)
 {

@@ -1164,7 +1164,13 @@ int adjoint_run(const mr_field *bathy, const mr_field *current, const double *de
     // workgroup up to one per CU (latency-bound: recompute | two linearise |
     // chain), two up to two per CU (recompute | sweep), one beyond (each wave
     // recomputes and sweeps in turn, the least SIMD time once the launch fills
-    // the GPU); block_size 64, 128 or 256 forces one, two or four
+    // the GPU); block_size 64, 128 or 256 forces one, two or four.  1000 steps
+    // (sweep, ms; one / two / four waves), flat depth and gridded depth:
+    //   16,384 rays  3.88 / 2.49 / 1.48    4.83 / 3.56 / 2.10
+    //   24,576       4.05 / 2.97 / 2.95
+    //   32,768       4.05 / 3.09 / 3.18    5.04 / 3.85 / 4.17
+    //   49,152       4.07 / 5.73 / 4.52
+    //   65,536       4.14 / 6.13 / 6.12    5.89 / 7.71 / 8.25
     const int cus = cu_count();
     const int64_t groups = (n_rays + 63) / 64;
     int waves = groups <= cus ? 4 : groups <= 2 * (int64_t)cus ? 2 : 1;

@@ -447,7 +447,8 @@ __device__ __forceinline__ void point64_full(const Grid64Ptrs &BP, const Grid64P
 // branch: the mask intrinsic is not folded into the test inside the block.
 // The callers mark it unlikely (an expectation inside this function would be
 // lost when it is inlined), so that the block is laid out after the loop; in
-// its place it costs a taken branch at every evaluation.
+// its place it costs a taken branch at every evaluation (16,384 rays x 2000
+// steps of a forward and its sweep 5.32 -> 5.20 ms).
 template <int BK, int CK>
 __device__ __forceinline__ bool any_off64(uint32_t off)
 {

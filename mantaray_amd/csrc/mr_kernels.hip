@@ -134,9 +134,11 @@ __device__ __forceinline__ void rk4_step(const BathyView &B, const BathyPtrs &BP
 // a 1024 x 768 depth under a constant current 1.90 -> 1.44 ms.  Taking
 // instructions out of the common path (row-major records, the factors 2 and
 // 4 of the dispersion in its constants, the slow test on one compare and
-// branch, the row offset as the step count) then gave 2.55 and 1.36 ms, and
-// 5.60 -> 5.42 ms on 65,536 rays x 5000 steps on shared cells (there the
-// clock drops as the lanes idle less: the load is near the power limit).
+// branch, the row offset as the step count) then gave 2.55 and 1.36 ms (2.48
+// and 1.30 with later changes, among them the terms of a constant current
+// left out), and 5.60 -> 5.42 ms on 65,536 rays x 5000 steps on shared cells
+// (there the clock drops as the lanes idle less: the load is near the power
+// limit).
 
 // The refill of one slot for the point (gx, gy).  The records' offsets are
 // formed before the tests, in every step: some lane of the wave refills in
