@@ -697,7 +697,7 @@ __global__ void __launch_bounds__(64) adjoint_flat_kernel(AdjointArgs a)
                                        ? rec[st][lin_place<BK, CK, false>(f)][lane] : 0.0;
                     }
                     double z[4];
-                    lin_apply_flat<BK, CK>(R, C, a.grads, sums, kb, z);
+                    lin_apply(R, B, C, a.grads, sums, kb, z);
                     if (st > 0) {
                         const double hs = st < 3 ? half : dt, cf = st > 1 ? 2.0 : 1.0;
 #pragma unroll
@@ -952,7 +952,7 @@ __global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs 
         else lin_role(std::integral_constant<int, 0>{});
     } else {
         double lam[4] = {0.0, 0.0, 0.0, 0.0};          // the cotangent
-        Accs64 acc;
+        Sums64<BK, CK, SH, NoQueue> sums(nullptr);
         if (active && m >= 0) {
             if (a.g_end && !dead) {
 #pragma unroll
@@ -994,7 +994,7 @@ __global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs 
                                             ? ring[(rho - 1) & 1][st - 1][f][lane] : 0.0;
                         }
                         double z[4];
-                        lin_apply<BK, CK, SH>(R, B, C, a.grads, acc, kb[st], z);
+                        lin_apply(R, B, C, a.grads, sums, kb[st], z);
                         if (st > 0) {
                             const double hs = st < 3 ? half : dt;
 #pragma unroll
@@ -1012,16 +1012,12 @@ __global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs 
             }
             __syncthreads();
         }
+        sums.finish(a.grads, (uint32_t)B.nx, (uint32_t)C.nx);
         if (!active) return;
         if (a.g_x0) a.g_x0[r] = lam[0];
         if (a.g_y0) a.g_y0[r] = lam[1];
         if (a.g_kx0) a.g_kx0[r] = lam[2];
         if (a.g_ky0) a.g_ky0[r] = lam[3];
-        if (BK == BK_GRID && a.grads.depth) acc_flush(acc.h, a.grads.depth, (uint32_t)B.nx);
-        if (CK == CK_GRID) {
-            if (a.grads.u) acc_flush(acc.u, a.grads.u, (uint32_t)C.nx);
-            if (a.grads.v) acc_flush(acc.v, a.grads.v, (uint32_t)C.nx);
-        }
     }
 }
 

@@ -485,57 +485,17 @@ __device__ __forceinline__ void rhs64(const Grid64View &B, const Grid64Ptrs &BP,
 }
 
 // ---------------------------------------------------------------------------
-// Adjoint accumulation into a value grid.  A ray stays in one cell for many
-// evaluations, so each lane sums its contributions to the four corners of
-// the cell in hand and adds them to the gradient grid (hardware f64 atomics)
-// only when it moves to another cell, and once at the end.
-
-struct CornerAcc {
-    uint32_t iA = 0xFFFFFFFFu;            // no cell yet
-    double a = 0.0, b = 0.0, c = 0.0, d = 0.0;
-};
-
-__device__ __forceinline__ void acc_flush(CornerAcc &s, double *grad, uint32_t nx)
-{
-    if (s.iA != 0xFFFFFFFFu) {
-        unsafeAtomicAdd(grad + s.iA, s.a);
-        unsafeAtomicAdd(grad + s.iA + nx, s.b);
-        unsafeAtomicAdd(grad + s.iA + nx + 1u, s.c);
-        unsafeAtomicAdd(grad + s.iA + 1u, s.d);
-    }
-    s.a = 0.0; s.b = 0.0; s.c = 0.0; s.d = 0.0;
-}
-
-// Adds the cotangent of one query to the corners of its cell: vbar on the
-// interpolated value, gxbar and gybar on the two cell-difference slopes.
-__device__ __forceinline__ void acc_add(CornerAcc &s, double *grad, uint32_t nx,
-                                        const Cell64 &cell, double rxs, double rys, double vbar,
-                                        double gxbar, double gybar)
-{
-    const bool moved = cell.iA != s.iA;
-    if (__builtin_expect(wave_any(moved), 0)) {
-        __asm__ volatile("");
-        if (moved) {
-            acc_flush(s, grad, nx);
-            s.iA = cell.iA;
-        }
-    }
-    const double u = cell.u, w = cell.w;
-    const double gx = gxbar * rxs, gy = gybar * rys;
-    s.a += vbar * ((1.0 - u) * (1.0 - w)) - gx - gy;
-    s.b += vbar * (u * (1.0 - w)) + gy;
-    s.c += vbar * (u * w);
-    s.d += vbar * ((1.0 - u) * w) + gx;
-}
-
-// The sums of the sweeps whose wave forms the vector-Jacobian products
-// (rhs64_vjp), which also loads cells while it accumulates.  vmcnt counts
-// atomics with loads and retires both in order, so an atomic issued when a
-// lane leaves its cell holds up the next cell's loads, for a microsecond and
-// more on a grid larger than L2; and with 64 lanes some lane leaves its cell
-// in most steps, a few lanes an instruction.  So the sums of a left cell go
-// to a queue in LDS, and once it holds a wave's worth, all lanes add one
-// entry each.  N arrays on one grid share the cell test (u and v; on shared
+// Adjoint accumulation into the value grids.  A ray stays in one cell for
+// many evaluations, so each lane sums its contributions to the four corners of
+// the cell in hand, and the gradient grid takes them (hardware f64 atomics)
+// only when it moves to another cell, and once at the end.  With 64 lanes
+// some lane leaves its cell in most steps, a few lanes an instruction; and
+// vmcnt counts atomics with loads and retires both in order, so in a wave
+// that also loads cells an atomic holds up the next cell's loads, for a
+// microsecond and more on a grid larger than L2.  So the sums of a left cell
+// go to a queue in LDS, and once it holds a wave's worth, all lanes add one
+// entry each.  A wave that loads no cells (the chain of the four-wave sweep)
+// adds them at once (NoQueue).  N arrays on one grid share the cell test (u and v; on shared
 // axes the depth too).
 constexpr int QUEUE64 = 128;               // entries; at most 63 before a push of up to 64
 
@@ -625,10 +585,38 @@ __device__ __forceinline__ void queue_push(CellQueue<N> &q, CellSums<N> &s, bool
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
+// In a queue's place where a lane's sums go straight to the grids: in the
+// chain wave of the four-wave sweep (16,384 rays x 2000 steps) the queue took
+// 3.04 ms over a flat depth and 3.74 on shared axes, this 2.81 and 3.50, and
+// sums with a cell test for each array 2.91 and 4.09.
+template <int N>
+struct NoQueue {
+    static constexpr int words = 0;
+};
+template <int N>
+__device__ __forceinline__ void queue_push(NoQueue<N> &, CellSums<N> &s, bool leave,
+                                           double *const (&grad)[N], uint32_t nx)
+{
+    if (leave & (s.iA != 0xFFFFFFFFu)) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            if (!grad[k]) continue;
+            unsafeAtomicAdd(grad[k] + s.iA, s.s[k][0]);
+            unsafeAtomicAdd(grad[k] + s.iA + nx, s.s[k][1]);
+            unsafeAtomicAdd(grad[k] + s.iA + nx + 1u, s.s[k][2]);
+            unsafeAtomicAdd(grad[k] + s.iA + 1u, s.s[k][3]);
+        }
+    }
+}
+template <int N>
+__device__ __forceinline__ void queue_drain(NoQueue<N> &, double *const (&)[N], uint32_t, int)
+{
+}
+
 // Adds the cotangents of one query to the sums of its cell: vb on the
 // interpolated values, gxb and gyb on the cell-difference slopes.
-template <int N>
-__device__ __forceinline__ void sums_add(CellSums<N> &s, CellQueue<N> &q,
+template <int N, class Queue>
+__device__ __forceinline__ void sums_add(CellSums<N> &s, Queue &q,
                                          double *const (&grad)[N], uint32_t nx,
                                          const Cell64 &cell, double rxs, double rys,
                                          const double (&vb)[N], const double (&gxb)[N],
@@ -637,7 +625,7 @@ __device__ __forceinline__ void sums_add(CellSums<N> &s, CellQueue<N> &q,
     if (__builtin_expect(__builtin_amdgcn_uicmp(cell.iA, s.iA, 33 /* != */) != 0, 0)) {
         __asm__ volatile("");
         const bool moved = cell.iA != s.iA;
-        queue_push<N>(q, s, moved, grad, nx);
+        queue_push(q, s, moved, grad, nx);
         if (moved) {
             s = CellSums<N>{};
             s.iA = cell.iA;
@@ -661,52 +649,83 @@ struct Grads64 {
     double *depth, *u, *v;
 };
 
-struct Accs64 {
-    CornerAcc h, u, v;
-};
-
-// The sums and queues of a sweep with rhs64_vjp: of the depth alone and of
-// the current's two arrays, or of all three on shared axes.
-template <int BK, int CK, bool SH>
+// The sums and queues of a sweep: of the depth alone and of the current's two
+// arrays, or of all three on shared axes.
+template <int BK, int CK, bool SH, template <int> class Queue = CellQueue>
 struct Sums64 {
     static constexpr int NB = SH ? 3 : 1;
-    static constexpr int words = (BK == BK_GRID ? CellQueue<NB>::words : 0) +
-                                 (!SH && CK == CK_GRID ? CellQueue<2>::words : 0);
+    static constexpr bool queued = Queue<1>::words > 0;
+    static constexpr int words = (BK == BK_GRID ? Queue<NB>::words : 0) +
+                                 (!SH && CK == CK_GRID ? Queue<2>::words : 0);
     CellSums<NB> b;
     CellSums<2> c;
-    CellQueue<NB> qb;
-    CellQueue<2> qc;
+    Queue<NB> qb;
+    Queue<2> qc;
 
     // lds: `words` doubles of the wave's own
     __device__ __forceinline__ explicit Sums64(double *lds)
     {
-        qb.e = lds;
-        qc.e = lds + (BK == BK_GRID ? CellQueue<NB>::words : 0);
-        if (BK == BK_GRID) *qb.count() = 0;
-        if (!SH && CK == CK_GRID) *qc.count() = 0;
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if constexpr (queued) {
+            qb.e = lds;
+            qc.e = lds + (BK == BK_GRID ? Queue<NB>::words : 0);
+            if (BK == BK_GRID) *qb.count() = 0;
+            if (!SH && CK == CK_GRID) *qc.count() = 0;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
     }
     // the last sums of every lane, called by the whole wave
     __device__ __forceinline__ void finish(const Grads64 &Gr, uint32_t bnx, uint32_t cnx)
     {
         if constexpr (SH) {
             double *const g[3] = {Gr.depth, Gr.u, Gr.v};
-            queue_push<3>(qb, b, true, g, bnx);
-            queue_drain<3>(qb, g, bnx, 1);
+            queue_push(qb, b, true, g, bnx);
+            queue_drain(qb, g, bnx, 1);
         } else {
             if constexpr (BK == BK_GRID) {
                 double *const g[1] = {Gr.depth};
-                queue_push<1>(qb, b, true, g, bnx);
-                queue_drain<1>(qb, g, bnx, 1);
+                queue_push(qb, b, true, g, bnx);
+                queue_drain(qb, g, bnx, 1);
             }
             if constexpr (CK == CK_GRID) {
                 double *const g[2] = {Gr.u, Gr.v};
-                queue_push<2>(qc, c, true, g, cnx);
-                queue_drain<2>(qc, g, cnx, 1);
+                queue_push(qc, c, true, g, cnx);
+                queue_drain(qc, g, cnx, 1);
             }
         }
     }
 };
+
+// Adds one evaluation's field cotangents to the sums: hvb, hgx, hgy those of
+// the depth query, g that of the derivatives (whose first two are also those
+// of u and v), at the wavenumber (kx, ky).
+template <int BK, int CK, bool SH, template <int> class Queue>
+__device__ __forceinline__ void fields_add(const Grid64View &B, const Grid64View &C,
+                                           const Grads64 &Gr, Sums64<BK, CK, SH, Queue> &sums,
+                                           const Cell64 &bc, bool okb, const Cell64 &cc, bool okc,
+                                           double hvb, double hgx, double hgy, const double g[4],
+                                           double kx, double ky)
+{
+    // (a state of a finite row never errs; the guards keep a misuse in bounds)
+    if constexpr (SH) {
+        double *const grad[3] = {Gr.depth, Gr.u, Gr.v};
+        if ((Gr.depth || Gr.u || Gr.v) && okb && okc)
+            sums_add(sums.b, sums.qb, grad, (uint32_t)C.nx, cc, C.rxs, C.rys, {hvb, g[0], g[1]},
+                        {hgx, -g[2] * kx, -g[2] * ky}, {hgy, -g[3] * kx, -g[3] * ky});
+    } else {
+        if constexpr (BK == BK_GRID) {
+            double *const grad[1] = {Gr.depth};
+            if (Gr.depth && okb)
+                sums_add(sums.b, sums.qb, grad, (uint32_t)B.nx, bc, B.rxs, B.rys, {hvb}, {hgx},
+                            {hgy});
+        }
+        if constexpr (CK == CK_GRID) {
+            double *const grad[2] = {Gr.u, Gr.v};
+            if ((Gr.u || Gr.v) && okc)
+                sums_add(sums.c, sums.qc, grad, (uint32_t)C.nx, cc, C.rxs, C.rys, {g[0], g[1]},
+                            {-g[2] * kx, -g[2] * ky}, {-g[3] * kx, -g[3] * ky});
+        }
+    }
+}
 
 // The linearisation of rhs64 at one stage point, as a record of LIN_N
 // doubles, so that the cotangent chain can run apart from the (costlier)
@@ -851,35 +870,27 @@ __device__ __forceinline__ void rhs64_lin(const Grid64View &B, const Grid64Ptrs 
 }
 
 // Applies a linearisation record R to the cotangent g: z = M g, and the
-// field-value cotangents to the accumulators.
-template <int BK, int CK, bool SH>
+// field-value cotangents to the sums.
+template <int BK, int CK, bool SH, template <int> class Queue>
 __device__ __forceinline__ void lin_apply(const double R[LIN_N], const Grid64View &B,
-                                          const Grid64View &C, const Grads64 &Gr, Accs64 &acc,
-                                          const double g[4], double z[4])
+                                          const Grid64View &C, const Grads64 &Gr,
+                                          Sums64<BK, CK, SH, Queue> &sums, const double g[4],
+                                          double z[4])
 {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        if (depth_is_flat<BK>() && i < 2)      // R[2], R[3], R[6], R[7] are zero
-            z[i] = R[4 * i] * g[0] + R[4 * i + 1] * g[1];
-        else
-            z[i] = ((R[4 * i] * g[0] + R[4 * i + 1] * g[1]) + R[4 * i + 2] * g[2]) +
-                   R[4 * i + 3] * g[3];
+        z[i] = R[4 * i] * g[0] + R[4 * i + 1] * g[1];
+        if (!depth_is_flat<BK>() || i >= 2)    // (R[2], R[3], R[6], R[7] are zero)
+            z[i] += R[4 * i + 2] * g[2] + R[4 * i + 3] * g[3];
     }
     uint32_t ib, ic;
     unpack_cells(R[27], ib, ic);
-    if (BK == BK_GRID && Gr.depth && ib != 0xFFFFFFFFu) {
-        const double hbar = ((R[16] * g[0] + R[17] * g[1]) + R[18] * g[2]) + R[19] * g[3];
-        Cell64 cell{ib, R[SH ? 25 : 23], R[SH ? 26 : 24]};
-        acc_add(acc.h, Gr.depth, (uint32_t)B.nx, cell, B.rxs, B.rys, hbar, g[2] * R[20],
-                g[3] * R[20]);
-    }
-    if (CK == CK_GRID && ic != 0xFFFFFFFFu) {
-        Cell64 cell{ic, R[25], R[26]};
-        if (Gr.u) acc_add(acc.u, Gr.u, (uint32_t)C.nx, cell, C.rxs, C.rys, g[0], -g[2] * R[21],
-                          -g[3] * R[21]);
-        if (Gr.v) acc_add(acc.v, Gr.v, (uint32_t)C.nx, cell, C.rxs, C.rys, g[1], -g[2] * R[22],
-                          -g[3] * R[22]);
-    }
+    double hbar = 0.0;
+    if (BK == BK_GRID)
+        hbar = (R[16] * g[0] + R[17] * g[1]) + (R[18] * g[2] + R[19] * g[3]);
+    fields_add(B, C, Gr, sums, Cell64{ib, R[23], R[24]}, ib != 0xFFFFFFFFu,
+                           Cell64{ic, R[25], R[26]}, ic != 0xFFFFFFFFu, hbar, g[2] * R[20],
+                           g[3] * R[20], g, R[21], R[22]);
 }
 
 // The fields of a record that lin_apply reads, and where each stands among
@@ -921,29 +932,6 @@ __device__ __forceinline__ void rhs64_with_lin(const Grid64View &B, const Grid64
             point64_full<BK, CK>(BP, CP, F, s[0], s[1], p);
             eval();
         }
-    }
-}
-
-// lin_apply for a flat depth, with the sums of a sweep that queues them
-template <int BK, int CK>
-__device__ __forceinline__ void lin_apply_flat(const double R[LIN_N], const Grid64View &C,
-                                               const Grads64 &Gr, Sums64<BK, CK, false> &sums,
-                                               const double g[4], double z[4])
-{
-    static_assert(depth_is_flat<BK>(), "no depth gradient");
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        z[i] = R[4 * i] * g[0] + R[4 * i + 1] * g[1];
-        if (i >= 2) z[i] += R[4 * i + 2] * g[2] + R[4 * i + 3] * g[3];
-    }
-    if constexpr (CK == CK_GRID) {
-        uint32_t ib, ic;
-        unpack_cells(R[27], ib, ic);
-        double *const grad[2] = {Gr.u, Gr.v};
-        if ((Gr.u || Gr.v) && ic != 0xFFFFFFFFu)
-            sums_add<2>(sums.c, sums.qc, grad, (uint32_t)C.nx, Cell64{ic, R[25], R[26]}, C.rxs,
-                        C.rys, {g[0], g[1]}, {-g[2] * R[21], -g[2] * R[22]},
-                        {-g[3] * R[21], -g[3] * R[22]});
     }
 }
 
@@ -1024,26 +1012,8 @@ __device__ __forceinline__ void rhs64_vjp(const Grid64View &B, const Grid64Ptrs 
         hgx = g2 * c;
         hgy = g3 * c;
     }
-    // (a state of a finite row never errs; the guards keep a misuse in bounds)
-    if constexpr (SH) {
-        double *const g[3] = {Gr.depth, Gr.u, Gr.v};
-        if ((Gr.depth || Gr.u || Gr.v) && okb && okc)
-            sums_add<3>(sums.b, sums.qb, g, (uint32_t)C.nx, cc, C.rxs, C.rys, {hvb, g0, g1},
-                        {hgx, -g2 * kx, -g2 * ky}, {hgy, -g3 * kx, -g3 * ky});
-    } else {
-        if constexpr (BK == BK_GRID) {
-            double *const g[1] = {Gr.depth};
-            if (Gr.depth && okb)
-                sums_add<1>(sums.b, sums.qb, g, (uint32_t)B.nx, bc, B.rxs, B.rys, {hvb}, {hgx},
-                            {hgy});
-        }
-        if constexpr (CK == CK_GRID) {
-            double *const g[2] = {Gr.u, Gr.v};
-            if ((Gr.u || Gr.v) && okc)
-                sums_add<2>(sums.c, sums.qc, g, (uint32_t)C.nx, cc, C.rxs, C.rys, {g0, g1},
-                            {-g2 * kx, -g2 * ky}, {-g3 * kx, -g3 * ky});
-        }
-    }
+    const double g[4] = {g0, g1, g2, g3};
+    fields_add(B, C, Gr, sums, bc, okb, cc, okc, hvb, hgx, hgy, g, kx, ky);
 }
 
 }  // namespace mr
