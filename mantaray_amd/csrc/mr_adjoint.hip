@@ -740,7 +740,7 @@ __global__ void __launch_bounds__(64) adjoint_flat_kernel(AdjointArgs a)
 // Segment c's K steps take K rounds; segment cmax is recomputed alone first
 // and the chain trails by one round: (cmax + 2) K + 1 rounds in all.  A
 // round costs about 4/NL stage linearisations, against eight in the
-// two-wave sweep.  Meant for launches of at most one workgroup per CU, where
+// two-wave sweep.  Meant for launches of a workgroup or two per CU, where
 // the sweep is latency-bound (the LDS ring holds one workgroup per CU).  NL
 // = 2 is the one launched: with NL = 4 the six waves share SIMDs and the
 // 256 registers a wave then gets spill.

@@ -1161,19 +1161,23 @@ int adjoint_run(const mr_field *bathy, const mr_field *current, const double *de
         return rc;
     }
     // the sweep kernel by workgroups (64 rays each) per CU: four waves per
-    // workgroup up to one per CU (latency-bound: recompute | two linearise |
-    // chain), two up to two per CU (recompute | sweep), one beyond (each wave
-    // recomputes and sweeps in turn, the least SIMD time once the launch fills
-    // the GPU); block_size 64, 128 or 256 forces one, two or four.  1000 steps
-    // (sweep, ms; one / two / four waves), flat depth and gridded depth:
-    //   16,384 rays  3.88 / 2.49 / 1.48    4.83 / 3.56 / 2.10
-    //   24,576       4.05 / 2.97 / 2.95
-    //   32,768       4.05 / 3.09 / 3.18    5.04 / 3.85 / 4.17
-    //   49,152       4.07 / 5.73 / 4.52
-    //   65,536       4.14 / 6.13 / 6.12    5.89 / 7.71 / 8.25
+    // workgroup (latency-bound: recompute | two linearise | chain) up to two
+    // per CU, which its LDS lets run one after the other; over a constant
+    // current, whose evaluations are short, up to one, and two waves
+    // (recompute | sweep) from there to two; one beyond (each wave recomputes
+    // and sweeps in turn, the least SIMD time once the launch fills the GPU).
+    // block_size 64, 128 or 256 forces one, two or four.  1000 steps (one /
+    // two / four waves, ms), current alone, both gridded on shared axes, on
+    // axes of their own, depth alone:
+    //   16,384 rays  3.94/2.50/1.45  4.81/3.60/1.88  6.08/4.36/2.10  3.18/2.22/1.43
+    //   24,576       4.10/2.98/2.83  4.99/3.80/3.62  6.31/4.57/4.17  3.30/2.64/2.88
+    //   32,768       4.11/3.07/2.99  5.03/3.89/3.66  6.36/4.63/4.16  3.34/2.71/2.94
+    //   36,864                       5.04/7.44/5.47  6.34/8.99/6.32  3.33/4.94/4.33
+    //   65,536       4.15/6.16/5.86  6.01/7.76/7.22
     const int cus = cu_count();
     const int64_t groups = (n_rays + 63) / 64;
-    int waves = groups <= cus ? 4 : groups <= 2 * (int64_t)cus ? 2 : 1;
+    const int64_t four = current->kind == MR_CURRENT_GRID ? 2 * (int64_t)cus : cus;
+    int waves = groups <= four ? 4 : groups <= 2 * (int64_t)cus ? 2 : 1;
     if (o.block_size == 64 || o.block_size == 128 || o.block_size == 256)
         waves = o.block_size / 64;
     else if (o.block_size != 0)

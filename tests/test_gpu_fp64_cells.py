@@ -102,3 +102,34 @@ def test_gradients(block, n_rays, stride, rows):
         grads.append({k: t.cpu().numpy()[: 14 * 23 if k in "uv" else None] for k, t in r.items()})
     for k, want in grads[1].items():
         assert np.abs(grads[0][k] - want).max() <= 1e-11 * np.abs(want).max(), k
+
+
+@pytest.mark.parametrize("n_rays", [16_384, 16_385, 32_768, 32_769])
+@pytest.mark.parametrize("fields", ["current", "depth"])
+def test_sweep_chosen_by_size(fields, n_rays):
+    """On both sides of the launch sizes (64 and 128 rays for each of 256 CUs)
+    at which the default sweep changes, it gives the gradients of the one-wave
+    sweep: sums of the same terms."""
+    import torch
+
+    import mantaray_amd as mr
+    from mantaray_amd import adjoint
+    x, y, d, cx, cy, u, v = _fields(23, 14, "jittered", False)
+    rng = np.random.default_rng(n_rays)
+    s = [torch.tensor(a, device="cuda:0") for a in
+         (rng.uniform(x[2], x[-3], n_rays), rng.uniform(y[1], y[-2], n_rays),
+          rng.uniform(-0.2, 0.2, n_rays), rng.uniform(-0.2, 0.2, n_rays))]
+    if fields == "depth":
+        b = mr.Bathymetry.from_arrays(x.astype(np.float32), y.astype(np.float32), d)
+        c = mr.Current.constant(0.2, -0.1)
+    else:
+        b, c = mr.Bathymetry.constant(30.0), mr.Current.from_arrays(cx, cy, u, v)
+    f = adjoint.trace_fp64(b, c, *s, 0.0, 6.5, 0.7, stride=4)
+    g_end = torch.tensor(rng.normal(size=(n_rays, 4)), device="cuda:0")
+    got, want = (adjoint.adjoint(b, c, f, 0.0, 6.5, 0.7, 4, g_end=g_end, block_size=block)
+                 for block in (0, 64))
+    for k, w in want.items():
+        if w is None:                                    # a field without a grid
+            assert got[k] is None, k
+            continue
+        assert (got[k] - w).abs().max().item() <= 1e-11 * w.abs().max().item(), k
