@@ -21,7 +21,8 @@
 // recomputes the segment's states and stage states from the checkpoint
 // with the forward's own step code (bitwise the forward's values) into a
 // per-lane column of the work buffer, then runs the step adjoints in reverse
-// order over them.
+// order over them (adjoint_flat_kernel keeps the states alone and forms the
+// stage states again, by the same arithmetic).
 #include <mutex>
 
 // The fp64 mode owes the reference its algorithm, not its roundings: products
@@ -578,9 +579,8 @@ __global__ void __launch_bounds__(64) adjoint_seq_kernel(AdjointArgs a)
 // the queued sums, on a 2048 x 2048 current, forward and sweep 89.6 -> 64.7
 // ms (the forward is 13.5 of them); the queue alone, before its pairs shared
 // requests and with the stored stage points, cost 2 ms.  What is left is the
-// issue of about 1350 vector instructions a step (63 to 64 ms with the
-// later changes to every fp64 evaluation: zero terms left out, slow paths
-// out of line).
+// issue of about 1380 vector instructions a step (66.2 ms with the stage
+// derivatives bitwise the forward's, rhs64_with_lin).
 template <int BK, int CK, int MATH>
 __global__ void __launch_bounds__(64) adjoint_flat_kernel(AdjointArgs a)
 {
@@ -659,8 +659,8 @@ __global__ void __launch_bounds__(64) adjoint_flat_kernel(AdjointArgs a)
                 for (int q = 0; q < 4; ++q) Y[q] = s[q];
 #pragma unroll
                 for (int st = 0; st < 4; ++st) {
-                    rhs64_with_lin<BK, CK>(B, a.bp, C, a.cp, a.f, (st == 0 || st == 3) ? sa : sb,
-                                           K, Y, R, d);
+                    rhs64_with_lin<BK, CK, MATH>(B, a.bp, C, a.cp, a.f,
+                                                 (st == 0 || st == 3) ? sa : sb, K, Y, R, d);
                     if (st == 0) {
                         vm_wait_upto<2>();
                         prefetch64<BK, CK, false>(B, a.bp, C, a.cp, a.f, sa, sa,
