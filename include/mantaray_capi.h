@@ -148,9 +148,16 @@ int mr_field_grid_shape(const mr_field *f, int64_t *nx, int64_t *ny, int64_t *le
 /* Copies the axes widened to f64 and the value arrays (depth, or u then v). */
 int mr_field_copy_grid(const mr_field *f, double *x, double *y, double *a, double *b);
 
-/* Builds the field's device tables (8 x 8 record tiles) on `device` (-1 =
- * current) now instead of on first use.  No reference counterpart (the reference has no device);
- * lets callers keep table construction out of a timed region. */
+/* Builds the field's device tables (8 x 8 record tiles) and a gridded field's
+ * own cell records on `device` (-1 = current) now instead of on first use.
+ * No reference counterpart (the reference has no device); lets callers keep
+ * table construction out of a timed region: a device-memory trace of two
+ * uploaded fields neither allocates nor synchronises and may be the first
+ * under stream capture.  Two exceptions build on their pair's first trace: a
+ * gridded depth and current on the same cells run on records of both, and
+ * MR_PREC_FP64_INTERP has tables of its own.  Where the device has no memory
+ * for the cell records, traces run on the plain ones (the same results,
+ * slower) until a later upload finds room. */
 int mr_field_upload(const mr_field *f, int32_t device);
 
 /* ---- integration ----------------------------------------------------- */

@@ -98,9 +98,10 @@ def trace_many_device(bathymetry: Bathymetry, current: Current, x0, y0, kx0, ky0
 
     Outputs are torch tensors on the same device (or the preallocated ones in
     `out`), written by kernels enqueued on `stream` (default: torch's current
-    stream); the call does not synchronise.  record_tile: log2 of the edge of
-    the square tiles the gridded fields' cell records are stored in (-1 = 8 x
-    8; results do not depend on it).
+    stream); the call does not synchronise once its fields' tables are on the
+    device (their upload()).  record_tile: log2 of the edge of the square tiles
+    of the gridded fields' plain records (-1 = 8 x 8), which full queries read
+    and fields without cell records run on; results do not depend on it.
     """
     import torch
 

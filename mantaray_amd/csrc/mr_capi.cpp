@@ -57,7 +57,7 @@ struct DevTables {
     const double *va = nullptr;    // the field's own values: depth, or u
     const double *vb = nullptr;    // v
     const SCell *scells = nullptr; // combined records with a current on shared cells
-    // a gridded field's own cell records, built on first use without shared cells
+    // a gridded field's own cell records, for pairs that do not share cells
     const DCell *dcells = nullptr;
     const UCell *ucells = nullptr;
     ~DevTables()
@@ -148,6 +148,9 @@ struct mr_field {
     // a bathymetry's combined records with a current on shared cells, per
     // (device, current uid)
     std::map<std::pair<int, uint64_t>, std::unique_ptr<DevTables>> shared;
+    // a gridded field's own cell records, per device; null where the device
+    // had no memory for them (own_records)
+    std::map<int, std::unique_ptr<DevTables>> own;
 
     mr_field() { ++live; }
     ~mr_field()
@@ -923,16 +926,22 @@ int shared_tables(const mr_field *cb, const mr_field *cc, int tl, const SCell **
     return MR_OK;
 }
 
-// A gridded field's own cell records (DCell, UCell) on the current device,
-// built on first use and kept with its tables t.
-int own_records(const mr_field *cf, int tl, const DevTables *ct)
+// Whether the kernels can index a gridded field's own cell records with 32-bit
+// byte offsets (an analytic field has none).
+bool records_fit(const mr_field *f, size_t rec)
 {
-    mr_field *f = const_cast<mr_field *>(cf);
-    DevTables &t = *const_cast<DevTables *>(ct);
-    const bool bathy = f->kind == MR_BATHY_GRID;
-    if (!bathy && f->kind != MR_CURRENT_GRID) return MR_OK;
-    std::lock_guard<std::mutex> lk(f->mu);
-    if (t.dcells || t.ucells) return MR_OK;
+    return (f->nx - 1) * (f->ny - 1) * (int64_t)rec < (int64_t(1) << 32);
+}
+bool own_records_fit(const mr_field *f)
+{
+    if (f->kind == MR_BATHY_GRID) return records_fit(f, sizeof(DCell));
+    return f->kind != MR_CURRENT_GRID || records_fit(f, sizeof(UCell));
+}
+
+// the own records of f from its plain tables pt (tile tl)
+int build_own_records(const mr_field &f, int tl, const DevTables &pt, DevTables &t)
+{
+    const bool bathy = f.kind == MR_BATHY_GRID;
     auto axis32 = [](const std::vector<double> &a) {
         std::vector<float> r(a.size());
         for (size_t i = 0; i < a.size(); i++) r[i] = (float)a[i];    // cartesian_current.rs:375-378
@@ -945,9 +954,9 @@ int own_records(const mr_field *cf, int tl, const DevTables *ct)
         else t64 = thresholds64(a64);
         return fast_bounds(a32, bathy ? &t32 : nullptr, bathy ? nullptr : &t64);
     };
-    const std::vector<float> x = bathy ? f->xf : axis32(f->xd), y = bathy ? f->yf : axis32(f->yd);
+    const std::vector<float> x = bathy ? f.xf : axis32(f.xd), y = bathy ? f.yf : axis32(f.yd);
     const std::vector<float2> xp = axis_pairs(x), yp = axis_pairs(y);
-    const std::vector<float2> fx = bounds(x, f->xd), fy = bounds(y, f->yd);
+    const std::vector<float2> fx = bounds(x, f.xd), fy = bounds(y, f.yd);
     // the axis arrays in one upload, for the build alone
     std::vector<float2> axes(xp);
     for (const std::vector<float2> *v : {&yp, &fx, &fy}) axes.insert(axes.end(), v->begin(), v->end());
@@ -956,25 +965,57 @@ int own_records(const mr_field *cf, int tl, const DevTables *ct)
     int rc = dev_upload(tmp, axes.data(), axes.size(), &dxp);
     if (rc) return rc;
     const float2 *dyp = dxp + xp.size(), *dfx = dyp + yp.size(), *dfy = dfx + fx.size();
-    const size_t n = (size_t)((f->nx - 1) * (f->ny - 1));
+    const size_t n = (size_t)((f.nx - 1) * (f.ny - 1));
     RecBuildArgs a;
-    a.nx = f->nx; a.ny = f->ny;
+    a.nx = f.nx; a.ny = f.ny;
     a.xp = dxp; a.yp = dyp; a.fx = dfx; a.fy = dfy;
-    a.oob_from = first_oob_cell(f->nx, f->ny, (int64_t)f->a.size());
-    if (!bathy) a.oob_from = std::min(a.oob_from, first_oob_cell(f->nx, f->ny, (int64_t)f->b.size()));
-    a.ntx = (int)(tiles_along(f->nx, tl) << 4 | tl);
+    a.oob_from = first_oob_cell(f.nx, f.ny, (int64_t)f.a.size());
+    if (!bathy) a.oob_from = std::min(a.oob_from, first_oob_cell(f.nx, f.ny, (int64_t)f.b.size()));
+    a.ntx = (int)(tiles_along(f.nx, tl) << 4 | tl);
     DCell *dc = nullptr;
     UCell *uc = nullptr;
     if (bathy) {
         if ((rc = dev_alloc(t, n, &dc))) return rc;
-        MR_HIP_TRY(launch_build_depth_rec(a, t.bp.cells, dc, 0));
+        MR_HIP_TRY(launch_build_depth_rec(a, pt.bp.cells, dc, 0));
     } else {
         if ((rc = dev_alloc(t, n, &uc))) return rc;
-        MR_HIP_TRY(launch_build_current_rec(a, t.cp.cells, t.cp.mtab, uc, 0));
+        MR_HIP_TRY(launch_build_current_rec(a, pt.cp.cells, pt.cp.mtab, uc, 0));
     }
     MR_HIP_TRY(hipDeviceSynchronize());
     t.dcells = dc;
     t.ucells = uc;
+    return MR_OK;
+}
+
+// A gridded field's own cell records (DCell, UCell) on the current device,
+// built by mr_field_upload or on first use: *out, or null where the device
+// has no memory for them, which leaves the field to its plain records (they
+// are 1.8 and 2 times those records' size).  Traces after such a refusal do
+// not ask again (asking allocates); an upload does.  pt: the field's plain
+// tables (tile tl).
+int own_records(const mr_field *cf, int tl, const DevTables *pt, bool again,
+                const DevTables **out)
+{
+    *out = nullptr;
+    mr_field *f = const_cast<mr_field *>(cf);
+    int dev = 0;
+    MR_HIP_TRY(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lk(f->mu);
+    auto it = f->own.find(dev);
+    if (it != f->own.end() && (it->second || !again)) {
+        *out = it->second.get();
+        return MR_OK;
+    }
+    std::unique_ptr<DevTables> t(new DevTables);
+    const int rc = build_own_records(*f, tl, *pt, *t);
+    if (rc == MR_ERR_OUT_OF_MEMORY) {
+        (void)hipGetLastError();       // the launches that follow would return it
+        t.reset();
+    } else if (rc) {
+        return rc;
+    }
+    *out = t.get();
+    f->own[dev] = std::move(t);
     return MR_OK;
 }
 
@@ -987,27 +1028,31 @@ int own_records(const mr_field *cf, int tl, const DevTables *ct)
 // records (REC_NONE) instead.
 int record_mode(const mr_field *b, const mr_field *c)
 {
-    auto fits = [](const mr_field *f, size_t rec) {
-        return (f->nx - 1) * (f->ny - 1) * (int64_t)rec < (int64_t(1) << 32);
-    };
-    if (shared_cells(b, c) && fits(b, sizeof(SCell))) return REC_SHARED;
-    if (b->kind == MR_BATHY_GRID && !fits(b, sizeof(DCell))) return REC_NONE;
-    if (c->kind == MR_CURRENT_GRID && !fits(c, sizeof(UCell))) return REC_NONE;
-    return REC_OWN;
+    if (shared_cells(b, c) && records_fit(b, sizeof(SCell))) return REC_SHARED;
+    return own_records_fit(b) && own_records_fit(c) ? REC_OWN : REC_NONE;
 }
 
-// the records of a mode, built on first use (bt, ct: the fields' tables)
-int record_tables(const mr_field *b, const mr_field *c, int tl, int mode, const DevTables *bt,
+// The records of a mode, built on first use (bt, ct: the fields' plain
+// tables).  *mode becomes REC_NONE where a field has no room for its own.
+int record_tables(const mr_field *b, const mr_field *c, int tl, int *mode, const DevTables *bt,
                   const DevTables *ct, RecPtrs *out)
 {
     *out = RecPtrs{nullptr, nullptr, nullptr};
-    if (mode == REC_NONE) return MR_OK;
-    if (mode == REC_SHARED) return shared_tables(b, c, tl, &out->scells);
-    int rc = own_records(b, tl, bt);
-    if (!rc) rc = own_records(c, tl, ct);
-    out->dcells = bt->dcells;
-    out->ucells = ct->ucells;
-    return rc;
+    if (*mode == REC_NONE) return MR_OK;
+    if (*mode == REC_SHARED) return shared_tables(b, c, tl, &out->scells);
+    const DevTables *own;
+    int rc;
+    if (b->kind == MR_BATHY_GRID) {
+        if ((rc = own_records(b, tl, bt, false, &own))) return rc;
+        if (own) out->dcells = own->dcells;
+        else *mode = REC_NONE;
+    }
+    if (c->kind == MR_CURRENT_GRID && *mode != REC_NONE) {
+        if ((rc = own_records(c, tl, ct, false, &own))) return rc;
+        if (own) out->ucells = own->ucells;
+        else *mode = REC_NONE;
+    }
+    return MR_OK;
 }
 
 // the trace itself, all pointers device pointers, enqueued on stream
@@ -1044,7 +1089,7 @@ int trace_device(const mr_field *bathy, const mr_field *current, int64_t n_rays,
     a.end_out = end_out;
     a.solout = o.solout;
     a.records = record_mode(bathy, current);
-    if ((rc = record_tables(bathy, current, o.record_tile, a.records, bt, ct, &a.rec))) return rc;
+    if ((rc = record_tables(bathy, current, o.record_tile, &a.records, bt, ct, &a.rec))) return rc;
     // more waves than SIMDs: the form that lets two share one (mr_device.h,
     // FullInPlace)
     if (a.records == REC_OWN && a.rec.dcells && a.rec.ucells &&
@@ -1438,8 +1483,11 @@ int mr_field_upload(const mr_field *f, int32_t device)
     if (!f) return fail(MR_ERR_INVALID_ARGUMENT, "null field");
     DeviceGuard g(device);
     if (!g.ok) return fail(MR_ERR_DEVICE, "cannot select device");
-    const DevTables *t;
-    return field_tables(f, kDefaultTile, &t);
+    const DevTables *t, *own;
+    const int rc = field_tables(f, kDefaultTile, &t);
+    const bool gridded = f->kind == MR_BATHY_GRID || f->kind == MR_CURRENT_GRID;
+    if (rc || !gridded || !own_records_fit(f)) return rc;
+    return own_records(f, kDefaultTile, t, true, &own);
     MR_GUARD_END
 }
 
@@ -1632,13 +1680,14 @@ int mr_batch_create(int32_t n_scenes, const mr_scene *scenes, const mr_options *
         ray_scene.insert(ray_scene.end(), (size_t)sc.n_rays, i);
     }
     if (b->n_rays >= (int64_t(1) << 31)) return fail(MR_ERR_UNSUPPORTED, "too many rays");
-    for (int32_t i = 0; i < n_scenes; i++) {
+    for (int32_t i = 0, mode = b->records; i < n_scenes; i++) {
         const mr_field *sb = scenes[i].bathy, *sc = scenes[i].current;
         const DevTables *bt, *ct;
         if ((rc = field_tables(sb, o.record_tile, &bt)) ||
             (rc = field_tables(sc, o.record_tile, &ct)) ||
-            (rc = record_tables(sb, sc, o.record_tile, b->records, bt, ct, &desc[(size_t)i].rec)))
+            (rc = record_tables(sb, sc, o.record_tile, &mode, bt, ct, &desc[(size_t)i].rec)))
             return rc;
+        b->records = mode;             // (REC_NONE reads none of those found before)
     }
     if ((rc = dev_upload(*b->mem, desc.data(), desc.size(), &b->scenes)) ||
         (rc = dev_upload(*b->mem, ray_scene.data(), ray_scene.size(), &b->ray_scene)) ||

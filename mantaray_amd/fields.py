@@ -54,7 +54,8 @@ class _Field:
         return (x, y, a) if self.role == "bathymetry" else (x, y, a, b)
 
     def upload(self, device: int = -1) -> None:
-        """Build the device tables now (otherwise built on first use)."""
+        """Build the device tables and a gridded field's cell records now
+        (otherwise on first use)."""
         C.check(C.lib().mr_field_upload(self._h, device))
 
     def close(self) -> None:
