@@ -783,10 +783,10 @@ hipError_t launch_trace(const TraceArgs &a, int bk, int ck, int math, int block,
         using K = decltype(k);
         constexpr int REC = decltype(rc)::value;
         constexpr bool DY = decltype(dy)::value;
-        if (REC != REC_NONE && nout == 0)
+        if (nout == 0)
             hipLaunchKernelGGL((trace_kernel<K::bk, K::ck, K::math, 0, REC, DY>), grid,
                                dim3(block), 0, stream, a);
-        else if (REC != REC_NONE && nout == 4)
+        else if (nout == 4)
             hipLaunchKernelGGL((trace_kernel<K::bk, K::ck, K::math, 1, REC, DY>), grid,
                                dim3(block), 0, stream, a);
         else
