@@ -277,7 +277,8 @@ __device__ __forceinline__ float index32(float t, double inv_sp)
 // f64 fractional index RN64(t / sp) (cartesian_current.rs:244), reduced to
 // what the cell choice needs: the bound checks and floor.  The product with
 // the rounded reciprocal is within 2^-50 (relative) of the quotient; only
-// when it lies that close to an integer is the exact division taken.  ok is
+// when it lies that close to an integer is the exact division taken, or where
+// a negative quotient may underflow to zero, which is on the grid.  ok is
 // cleared where the reference returns Err (a NaN index errs later, in
 // bilinear, because all four corners collapse onto (0, 0)).  The returned
 // floor is meaningful only when ok is set.
@@ -287,11 +288,12 @@ __device__ __forceinline__ double index64(double p, double a0, double sp, double
     const double t = p - a0;
     double q = t * inv_sp;
     double fl = __builtin_floor(q);
-    if (__builtin_fabs((q - fl) - 0.5) > 0.5 - q * 0x1p-50) {   // near an integer
+    if ((__builtin_fabs((q - fl) - 0.5) > 0.5 - q * 0x1p-50) |  // near an integer
+        ((t < 0.0) & (q > -0x1p-1000))) {
         q = t / sp;
         fl = __builtin_floor(q);
     }
-    ok = ok & (t >= 0.0) & (q <= nm1);
+    ok = ok & (q >= 0.0) & (q <= nm1);
     return fl;
 }
 
