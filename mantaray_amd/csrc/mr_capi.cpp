@@ -18,6 +18,7 @@
 #include <string>
 #include <vector>
 
+#include "mr_axes.h"
 #include "mr_hostio.h"
 #include "mr_kernels.h"
 #include "mr_netcdf3.h"
@@ -60,6 +61,7 @@ struct DevTables {
     // a gridded field's own cell records, for pairs that do not share cells
     const DCell *dcells = nullptr;
     const UCell *ucells = nullptr;
+    double outside = 0.0;          // OwnAxes::outside
     ~DevTables()
     {
         for (void *p : allocs) (void)hipFree(p);
@@ -148,8 +150,8 @@ struct mr_field {
     // a bathymetry's combined records with a current on shared cells, per
     // (device, current uid)
     std::map<std::pair<int, uint64_t>, std::unique_ptr<DevTables>> shared;
-    // a gridded field's own cell records, per device; null where the device
-    // had no memory for them (own_records)
+    // a gridded field's own cell records, per device; null where it runs on
+    // its plain records (own_records)
     std::map<int, std::unique_ptr<DevTables>> own;
 
     mr_field() { ++live; }
@@ -217,125 +219,6 @@ int validate_grid(int64_t nx, int64_t ny, int64_t rec_bytes, int tl)
         (tiles_along(nx, tl) * tiles_along(ny, tl) << (2 * tl)) * rec_bytes >= (int64_t(1) << 32))
         return fail(MR_ERR_UNSUPPORTED, "grid too large for 32-bit cell offsets");
     return MR_OK;
-}
-
-// ---- cell thresholds -------------------------------------------------------
-// The reference's cell along an axis is a monotone step function of the
-// coordinate: the fractional index RN(RN(p - a0) / sp) is non-decreasing in
-// p (each rounding is monotone), and the cell is its floor, clamped to n-2 on
-// the last node.  T[i] = min{p : index(p) >= i} for i < n-1 and T[n-1] =
-// min{p : index(p) > n-1} make cell i exactly [T[i], T[i+1]) and the valid
-// range [T[0], T[n-1]).  Each T is found by bisection over the totally
-// ordered floating-point values, evaluating the index with the reference's
-// own operations (cartesian_netcdf3.rs:285, cartesian_current.rs:244).
-// T[i] is within a few roundings of a0 + i sp, so the search widens from there
-// (first_true) before it bisects: from the whole range an axis of 1500 nodes
-// takes 0.54 ms (f64) or 0.31 ms (f32) of the first trace of its field, from
-// the guess 0.012 and 0.008 ms.
-
-uint32_t key32(float f)
-{
-    uint32_t b;
-    std::memcpy(&b, &f, 4);
-    return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
-}
-float unkey32(uint32_t k)
-{
-    uint32_t b = (k & 0x80000000u) ? (k & 0x7fffffffu) : ~k;
-    float f;
-    std::memcpy(&f, &b, 4);
-    return f;
-}
-uint64_t key64(double f)
-{
-    uint64_t b;
-    std::memcpy(&b, &f, 8);
-    return (b >> 63) ? ~b : (b | (uint64_t(1) << 63));
-}
-double unkey64(uint64_t k)
-{
-    uint64_t b = (k >> 63) ? (k & ~(uint64_t(1) << 63)) : ~k;
-    double f;
-    std::memcpy(&f, &b, 8);
-    return f;
-}
-
-// The first key of (lo, hi] whose pred is true; pred does not decrease, is
-// taken as false at lo and as true at hi, and is evaluated at neither.
-template <class Key, class Pred>
-Key first_true(Key lo, Key hi, Key guess, Pred pred)
-{
-    if (guess > lo && guess < hi) {
-        // (hi - lo bounds the step, so doubling it cannot wrap)
-        if (pred(guess)) {
-            hi = guess;
-            for (Key step = 1; hi - lo > step; step *= 2) {
-                if (!pred(hi - step)) {
-                    lo = hi - step;
-                    break;
-                }
-                hi -= step;
-            }
-        } else {
-            lo = guess;
-            for (Key step = 1; hi - lo > step; step *= 2) {
-                if (pred(lo + step)) {
-                    hi = lo + step;
-                    break;
-                }
-                lo += step;
-            }
-        }
-    }
-    while (hi - lo > 1) {
-        const Key mid = lo + (hi - lo) / 2;
-        if (pred(mid)) hi = mid; else lo = mid;
-    }
-    return hi;
-}
-
-// f32 axis (bathymetry): thresholds T[0..n-1]
-std::vector<float> thresholds32(const std::vector<float> &a)
-{
-    const size_t n = a.size();
-    const float a0 = a[0], sp = std::fabs(a[1] - a[0]);
-    auto index = [&](float p) { return (p - a0) / sp; };        // :285
-    std::vector<float> t(n);
-    for (size_t i = 0; i < n; i++) {
-        const float lim = (float)i;
-        const bool upper = i == n - 1;                         // index > n-1 errs
-        auto pred = [&](uint32_t k) {
-            const float x = index(unkey32(k));
-            return upper ? x > lim : x >= lim;
-        };
-        const uint32_t lo = key32(-INFINITY), hi = key32(INFINITY);
-        // (a spacing that overflows leaves no order to widen in: lo, no guess)
-        const uint32_t guess =
-            std::isfinite(sp) ? key32((float)((double)a0 + (double)i * (double)sp)) : lo;
-        t[i] = unkey32(first_true(lo, hi, guess, pred));
-    }
-    return t;
-}
-
-// f64 axis (current): thresholds T[0..n-1]
-std::vector<double> thresholds64(const std::vector<double> &a)
-{
-    const size_t n = a.size();
-    const double a0 = a[0], sp = std::fabs(a[1] - a[0]);
-    auto index = [&](double p) { return (p - a0) / sp; };       // :244
-    std::vector<double> t(n);
-    for (size_t i = 0; i < n; i++) {
-        const double lim = (double)i;
-        const bool upper = i == n - 1;
-        auto pred = [&](uint64_t k) {
-            const double x = index(unkey64(k));
-            return upper ? x > lim : x >= lim;
-        };
-        const uint64_t lo = key64(-INFINITY), hi = key64(INFINITY);
-        const uint64_t guess = std::isfinite(sp) ? key64(a0 + (double)i * sp) : lo;
-        t[i] = unkey64(first_true(lo, hi, guess, pred));
-    }
-    return t;
 }
 
 // per-cell axis data of the bathymetry: (a[i], a[i+1], T[i], T[i+1])
@@ -827,47 +710,6 @@ bool shared_cells(const mr_field *b, const mr_field *c)
     return true;
 }
 
-// The fast region of each cell along one axis (SCell, DCell, UCell): the f32
-// targets p in [lo, hi] lie in cell i for the depth's f32 index rule (T32[i]
-// <= p < T32[i+1]; t32 null: no depth on this axis), for every f64 coordinate
-// that rounds to p lie in cell i for the current's f64 index rule (T64[i] <=
-// x < T64[i+1]; t64 null: no current), and are strictly between the cell's
-// node coordinates a[i] and a[i+1] (no corner).  If RN32(x) >= lo >
-// ceil32(T64[i]) then x > T64[i]; if RN32(x) <= hi < floor32(T64[i+1]) then
-// x < T64[i+1] (rounding is monotone).  The intervals need not meet (on axes
-// whose spacing varies, the index rules, which use the first spacing, can map
-// a cell's targets outside its nodes): an empty interval is stored as
-// (-inf, -inf), the one form of an empty region that the device's region
-// test (med3(p, lo, hi) - p) reads as empty; lo > hi would read as [hi, lo].
-std::vector<float2> fast_bounds(const std::vector<float> &a, const std::vector<float> *t32,
-                                const std::vector<double> *t64)
-{
-    auto up = [](float f) { return std::nextafter(f, INFINITY); };
-    auto down = [](float f) { return std::nextafter(f, -INFINITY); };
-    auto ceil32 = [&](double d) {
-        float f = (float)d;
-        return (double)f < d ? up(f) : f;
-    };
-    auto floor32 = [&](double d) {
-        float f = (float)d;
-        return (double)f > d ? down(f) : f;
-    };
-    std::vector<float2> b(a.size() - 1);
-    for (size_t i = 0; i + 1 < a.size(); i++) {
-        float lo = up(a[i]), hi = down(a[i + 1]);
-        if (t32) {
-            lo = std::max(lo, (*t32)[i]);
-            hi = std::min(hi, down((*t32)[i + 1]));
-        }
-        if (t64) {
-            lo = std::max(lo, up(ceil32((*t64)[i])));
-            hi = std::min(hi, down(floor32((*t64)[i + 1])));
-        }
-        b[i] = lo <= hi ? make_float2(lo, hi) : make_float2(-INFINITY, -INFINITY);
-    }
-    return b;
-}
-
 // the combined records of a depth and a current on shared cells (SCell) on
 // the current device, built on first use and kept with the bathymetry
 int shared_tables(const mr_field *cb, const mr_field *cc, int tl, const SCell **out)
@@ -890,7 +732,7 @@ int shared_tables(const mr_field *cb, const mr_field *cc, int tl, const SCell **
     auto bounds = [](const std::vector<float> &a32, const std::vector<double> &a64) {
         const std::vector<float> t32 = thresholds32(a32);
         const std::vector<double> t64 = thresholds64(a64);
-        return fast_bounds(a32, &t32, &t64);
+        return fast_bounds<float2>(a32, &t32, &t64);
     };
     std::vector<float2> fx = bounds(b->xf, cc->xd), fy = bounds(b->yf, cc->yd);
     float2 *dfx, *dfy;
@@ -938,33 +780,49 @@ bool own_records_fit(const mr_field *f)
     return f->kind != MR_CURRENT_GRID || records_fit(f, sizeof(UCell));
 }
 
+// a gridded field's f32 axes as the records hold them, with the fast regions
+// of its own index rule and the share of targets outside them
+struct OwnAxes {
+    std::vector<float> x, y;
+    std::vector<float2> fx, fy;
+    double outside;                    // the axes' worst cells' shares, added
+};
+
+OwnAxes own_axes(const mr_field &f)
+{
+    OwnAxes o;
+    if (f.kind == MR_BATHY_GRID) {
+        const std::vector<float> tx = thresholds32(f.xf), ty = thresholds32(f.yf);
+        o.x = f.xf; o.y = f.yf;
+        o.fx = fast_bounds<float2>(o.x, &tx, nullptr);
+        o.fy = fast_bounds<float2>(o.y, &ty, nullptr);
+        o.outside = worst_outside(o.fx, tx) + worst_outside(o.fy, ty);
+    } else {
+        const std::vector<double> tx = thresholds64(f.xd), ty = thresholds64(f.yd);
+        o.x.assign(f.xd.begin(), f.xd.end());              // (f32) casts,
+        o.y.assign(f.yd.begin(), f.yd.end());              // cartesian_current.rs:375-378
+        o.fx = fast_bounds<float2>(o.x, nullptr, &tx);
+        o.fy = fast_bounds<float2>(o.y, nullptr, &ty);
+        o.outside = worst_outside(o.fx, tx) + worst_outside(o.fy, ty);
+    }
+    return o;
+}
+
 // the own records of f from its plain tables pt (tile tl)
-int build_own_records(const mr_field &f, int tl, const DevTables &pt, DevTables &t)
+int build_own_records(const mr_field &f, const OwnAxes &o, int tl, const DevTables &pt,
+                      DevTables &t)
 {
     const bool bathy = f.kind == MR_BATHY_GRID;
-    auto axis32 = [](const std::vector<double> &a) {
-        std::vector<float> r(a.size());
-        for (size_t i = 0; i < a.size(); i++) r[i] = (float)a[i];    // cartesian_current.rs:375-378
-        return r;
-    };
-    auto bounds = [&](const std::vector<float> &a32, const std::vector<double> &a64) {
-        std::vector<float> t32;
-        std::vector<double> t64;
-        if (bathy) t32 = thresholds32(a32);
-        else t64 = thresholds64(a64);
-        return fast_bounds(a32, bathy ? &t32 : nullptr, bathy ? nullptr : &t64);
-    };
-    const std::vector<float> x = bathy ? f.xf : axis32(f.xd), y = bathy ? f.yf : axis32(f.yd);
-    const std::vector<float2> xp = axis_pairs(x), yp = axis_pairs(y);
-    const std::vector<float2> fx = bounds(x, f.xd), fy = bounds(y, f.yd);
+    const std::vector<float2> xp = axis_pairs(o.x), yp = axis_pairs(o.y);
     // the axis arrays in one upload, for the build alone
     std::vector<float2> axes(xp);
-    for (const std::vector<float2> *v : {&yp, &fx, &fy}) axes.insert(axes.end(), v->begin(), v->end());
+    for (const std::vector<float2> *v : {&yp, &o.fx, &o.fy})
+        axes.insert(axes.end(), v->begin(), v->end());
     DevTables tmp;
     float2 *dxp;
     int rc = dev_upload(tmp, axes.data(), axes.size(), &dxp);
     if (rc) return rc;
-    const float2 *dyp = dxp + xp.size(), *dfx = dyp + yp.size(), *dfy = dfx + fx.size();
+    const float2 *dyp = dxp + xp.size(), *dfx = dyp + yp.size(), *dfy = dfx + o.fx.size();
     const size_t n = (size_t)((f.nx - 1) * (f.ny - 1));
     RecBuildArgs a;
     a.nx = f.nx; a.ny = f.ny;
@@ -984,15 +842,38 @@ int build_own_records(const mr_field &f, int tl, const DevTables &pt, DevTables 
     MR_HIP_TRY(hipDeviceSynchronize());
     t.dcells = dc;
     t.ucells = uc;
+    t.outside = o.outside;
     return MR_OK;
 }
 
 // A gridded field's own cell records (DCell, UCell) on the current device,
-// built by mr_field_upload or on first use: *out, or null where the device
-// has no memory for them, which leaves the field to its plain records (they
-// are 1.8 and 2 times those records' size).  Traces after such a refusal do
-// not ask again (asking allocates); an upload does.  pt: the field's plain
-// tables (tile tl).
+// built by mr_field_upload or on first use: *out, or null, which leaves the
+// field to its plain records,
+//   - where the device has no memory for them (they take 64 and 128 bytes a
+//     cell beside the plain records' 32 and 72).  Traces after such a refusal
+//     do not ask again (asking allocates); an upload does;
+//   - where more than kOutside of a cell's targets lie outside its fast
+//     region: one lane there takes the wave through the full queries, which
+//     the plain records' own cell test needs only on a change of cells.  A
+//     region leaves out the f32 value of its nodes (of the current also its
+//     neighbours'), which is one of few where the axis lies far from zero;
+//     and an axis whose first spacing is off, by its f32 rounding or because
+//     its spacing varies, has cells of the index rule that miss their nodes.
+//     500 steps of 20,000 rays on 700 x 700 cells of 128 m at growing
+//     distances, on own and on plain records (ms):
+//       f32 spacing / cell     0      0.0005  0.001  0.002  0.004  0.008
+//       depth alone, own       0.49   0.60    0.63   0.74   1.02   1.17
+//                    plain     0.66   0.66    0.66   0.66   0.66   0.66
+//       current alone, own     0.57   0.70    0.76   0.90   1.12   1.41
+//                      plain   0.78   0.81    0.83   0.88   0.96   1.11
+//       both, own              0.66   1.07    1.19   1.56   2.06   2.50
+//             plain            1.00   1.05    1.07   1.13   1.26   1.42
+//     The line is on the sum over a pair's axes, each by its worst cell
+//     (record_tables): of the depth alone the spacing counts twice, of both
+//     about five times.
+// pt: the field's plain tables (tile tl).
+constexpr double kOutside = 1.0 / 512;
+
 int own_records(const mr_field *cf, int tl, const DevTables *pt, bool again,
                 const DevTables **out)
 {
@@ -1006,13 +887,17 @@ int own_records(const mr_field *cf, int tl, const DevTables *pt, bool again,
         *out = it->second.get();
         return MR_OK;
     }
-    std::unique_ptr<DevTables> t(new DevTables);
-    const int rc = build_own_records(*f, tl, *pt, *t);
-    if (rc == MR_ERR_OUT_OF_MEMORY) {
-        (void)hipGetLastError();       // the launches that follow would return it
-        t.reset();
-    } else if (rc) {
-        return rc;
+    std::unique_ptr<DevTables> t;
+    const OwnAxes axes = own_axes(*f);
+    if (axes.outside <= kOutside) {
+        t.reset(new DevTables);
+        const int rc = build_own_records(*f, axes, tl, *pt, *t);
+        if (rc == MR_ERR_OUT_OF_MEMORY) {
+            (void)hipGetLastError();   // the launches that follow would return it
+            t.reset();
+        } else if (rc) {
+            return rc;
+        }
     }
     *out = t.get();
     f->own[dev] = std::move(t);
@@ -1033,25 +918,27 @@ int record_mode(const mr_field *b, const mr_field *c)
 }
 
 // The records of a mode, built on first use (bt, ct: the fields' plain
-// tables).  *mode becomes REC_NONE where a field has no room for its own.
+// tables).  *mode becomes REC_NONE where a field runs on its plain records
+// (own_records), or the two together have too many targets outside their
+// fast regions.
 int record_tables(const mr_field *b, const mr_field *c, int tl, int *mode, const DevTables *bt,
                   const DevTables *ct, RecPtrs *out)
 {
     *out = RecPtrs{nullptr, nullptr, nullptr};
     if (*mode == REC_NONE) return MR_OK;
     if (*mode == REC_SHARED) return shared_tables(b, c, tl, &out->scells);
-    const DevTables *own;
+    const bool bg = b->kind == MR_BATHY_GRID, cg = c->kind == MR_CURRENT_GRID;
+    const DevTables *bo = nullptr, *co = nullptr;
     int rc;
-    if (b->kind == MR_BATHY_GRID) {
-        if ((rc = own_records(b, tl, bt, false, &own))) return rc;
-        if (own) out->dcells = own->dcells;
-        else *mode = REC_NONE;
+    if (bg && (rc = own_records(b, tl, bt, false, &bo))) return rc;
+    if (cg && (!bg || bo) && (rc = own_records(c, tl, ct, false, &co))) return rc;
+    if ((bg && !bo) || (cg && !co) ||
+        (bo ? bo->outside : 0.0) + (co ? co->outside : 0.0) > kOutside) {
+        *mode = REC_NONE;
+        return MR_OK;
     }
-    if (c->kind == MR_CURRENT_GRID && *mode != REC_NONE) {
-        if ((rc = own_records(c, tl, ct, false, &own))) return rc;
-        if (own) out->ucells = own->ucells;
-        else *mode = REC_NONE;
-    }
+    if (bo) out->dcells = bo->dcells;
+    if (co) out->ucells = co->ucells;
     return MR_OK;
 }
 
