@@ -160,6 +160,11 @@ int mr_field_copy_grid(const mr_field *f, double *x, double *y, double *a, doubl
  * slower) until a later upload finds room. */
 int mr_field_upload(const mr_field *f, int32_t device);
 
+/* Frees what host-memory traces keep for the next one and no call is using:
+ * at most two sets of 12 streams, 48 MiB of pinned memory and 512 MiB of
+ * device memory (16 MiB once no field handle lives). */
+int mr_release_host_buffers(void);
+
 /* ---- integration ----------------------------------------------------- */
 
 /* ode_solvers 0.4.0 Rk4::integrate step count: n = ceil((t_end - t0)/dt).

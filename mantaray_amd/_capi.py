@@ -36,7 +36,8 @@ EXPORTS = (
     "mr_bathy_open_nc3", "mr_current_open_nc3", "mr_bathy_from_arrays",
     "mr_current_from_arrays", "mr_bathy_constant", "mr_bathy_slope", "mr_bathy_array",
     "mr_current_constant", "mr_field_free", "mr_field_kind", "mr_field_grid_shape",
-    "mr_field_copy_grid", "mr_field_upload", "mr_num_steps", "mr_trace_many",
+    "mr_field_copy_grid", "mr_field_upload", "mr_release_host_buffers", "mr_num_steps",
+    "mr_trace_many",
     "mr_single_ray", "mr_time_rows", "mr_rhs_many", "mr_checkpoint_count", "mr_adjoint_workspace_size",
     "mr_trace_fp64", "mr_adjoint_many", "mr_adjoint_many_noalloc", "mr_ray_result_json",
     "mr_ray_result_append_tsv",
@@ -108,6 +109,7 @@ _SIGS = {
     "mr_field_grid_shape": (ctypes.c_int, [_fieldp, _i64p, _i64p, _i64p, _i64p]),
     "mr_field_copy_grid": (ctypes.c_int, [_fieldp, _vp, _vp, _vp, _vp]),
     "mr_field_upload": (ctypes.c_int, [_fieldp, ctypes.c_int32]),
+    "mr_release_host_buffers": (ctypes.c_int, []),
     "mr_num_steps": (ctypes.c_int, [_f64, _f64, _f64, _i64p]),
     "mr_trace_many": (ctypes.c_int, [_fieldp, _fieldp, _i64, _vp, _vp, _vp, _vp, _f64, _f64,
                                      _f64, ctypes.POINTER(Options), _vp, _vp, _vp, _vp, _vp,

@@ -83,13 +83,25 @@ struct DeviceGuard {
     }
 };
 
+// hipMalloc, with the host calls' idle buffers given back if it finds no memory
+hipError_t dev_malloc(void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        drop_idle_stages();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
 template <class T>
 int dev_upload(DevTables &t, const T *host, size_t n, T **out)
 {
     *out = nullptr;
     if (n == 0) return MR_OK;
     void *p = nullptr;
-    MR_HIP_TRY(hipMalloc(&p, n * sizeof(T)));
+    MR_HIP_TRY(dev_malloc(&p, n * sizeof(T)));
     t.allocs.push_back(p);
     MR_HIP_TRY(hipMemcpy(p, host, n * sizeof(T), hipMemcpyHostToDevice));
     *out = static_cast<T *>(p);
@@ -102,7 +114,7 @@ int dev_alloc(DevTables &t, size_t n, T **out)
     *out = nullptr;
     if (n == 0) return MR_OK;
     void *p = nullptr;
-    MR_HIP_TRY(hipMalloc(&p, n * sizeof(T)));
+    MR_HIP_TRY(dev_malloc(&p, n * sizeof(T)));
     t.allocs.push_back(p);
     *out = static_cast<T *>(p);
     return MR_OK;
@@ -157,7 +169,7 @@ struct mr_field {
     mr_field() { ++live; }
     ~mr_field()
     {
-        if (--live == 0) drop_idle_stages();
+        if (--live == 0) trim_idle_stages();
     }
     static std::atomic<int64_t> live;   // handles of the process
 };
@@ -1026,7 +1038,11 @@ int trace_host(const mr_field *bathy, const mr_field *current, int64_t n_rays, c
     hipError_t e = hipSuccess;
     const StagePtr st = acquire_stage(used, &e);
     MR_HIP_TRY(e);
-    MR_HIP_TRY(copy_in(*st, in));
+    if ((e = copy_in(*st, in)) != hipSuccess) {
+        // (the stage goes back to the pool with nothing in flight)
+        (void)hipStreamSynchronize(stage_stream(*st));
+        MR_HIP_TRY(e);
+    }
     char *dev = stage_device(*st);
     auto at = [&](const void *host, size_t off) {
         return host ? reinterpret_cast<double *>(dev + off) : nullptr;
@@ -1375,6 +1391,14 @@ int mr_field_upload(const mr_field *f, int32_t device)
     const bool gridded = f->kind == MR_BATHY_GRID || f->kind == MR_CURRENT_GRID;
     if (rc || !gridded || !own_records_fit(f)) return rc;
     return own_records(f, kDefaultTile, t, true, &own);
+    MR_GUARD_END
+}
+
+int mr_release_host_buffers(void)
+{
+    MR_GUARD_BEGIN
+    drop_idle_stages();
+    return MR_OK;
     MR_GUARD_END
 }
 

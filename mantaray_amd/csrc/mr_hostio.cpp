@@ -10,11 +10,15 @@
 // 60 ms before and takes 8.3 ms.  Memory belonging to the caller is not
 // pinned in place (hipHostRegister), and no result lives in the pool.
 //
-// The chunks, the stream and the device buffer are kept between calls (small
+// The chunks, the streams and the device buffer are kept between calls (small
 // calls spent more on allocations and on one copy per array than on their
 // copies).  The pool is bounded: at most kIdleStages idle stages a process,
 // each with kChunk x kWorkers pinned bytes and at most kKeepDevice of device
-// memory; it is freed when the last field handle is.
+// memory.  When the last field handle dies, the device memory beyond
+// kKeepIdle goes; the rest stays, as a call on file paths opens and frees its
+// fields each time and would otherwise make and free its chunks and streams as
+// well.  All of it is given back by drop_idle_stages (mr_release_host_buffers),
+// and by an allocation that fails.
 #include "mr_hostio.h"
 
 #include <algorithm>
@@ -30,12 +34,16 @@ namespace {
 
 // A pinned chunk: 75 us on the bus, long against a wait's overhead.  A thread
 // is worth starting for each megabyte (about 100 us of copying into fresh
-// pages, against 15 us to start it).
+// pages, against 15 us to start it), a worker's stream and chunk worth making
+// for each kPerNewWorker.
 constexpr size_t kChunk = size_t(4) << 20;
+constexpr size_t kLeastChunk = size_t(64) << 10;
 constexpr size_t kPerThread = size_t(1) << 20;
+constexpr size_t kPerNewWorker = size_t(4) << 20;
 constexpr int kWorkers = 12;
 constexpr size_t kIdleStages = 2;
 constexpr size_t kKeepDevice = size_t(512) << 20;
+constexpr size_t kKeepIdle = size_t(16) << 20;
 
 }  // namespace
 
@@ -43,17 +51,32 @@ struct HostStage {
     int device = 0;
     hipStream_t stream[kWorkers] = {};
     char *pin[kWorkers] = {};
+    size_t pin_bytes[kWorkers] = {};
     char *dev = nullptr;
     size_t dev_bytes = 0;
 
-    // the pinned chunk and stream of worker w, made on first use
-    hipError_t need(int w)
+    // the stream of worker w and a pinned chunk of at least `bytes` (up to
+    // kChunk), made on first use; worker w's chunk is not in use
+    hipError_t need(int w, size_t bytes)
     {
         hipError_t e = hipSuccess;
         if (!stream[w]) e = hipStreamCreateWithFlags(&stream[w], hipStreamNonBlocking);
-        if (e == hipSuccess && !pin[w])
-            e = hipHostMalloc(reinterpret_cast<void **>(&pin[w]), kChunk, hipHostMallocDefault);
+        if (e != hipSuccess || pin_bytes[w] >= bytes) return e;
+        size_t n = kLeastChunk;
+        while (n < bytes) n *= 2;
+        if (pin[w]) (void)hipHostFree(pin[w]);
+        pin_bytes[w] = 0;
+        e = hipHostMalloc(reinterpret_cast<void **>(&pin[w]), n, hipHostMallocDefault);
+        if (e != hipSuccess) pin[w] = nullptr;
+        else pin_bytes[w] = n;
         return e;
+    }
+    // workers whose stream and chunk are there
+    int made() const
+    {
+        int w = 0;
+        while (w < kWorkers && pin_bytes[w]) w++;
+        return w;
     }
     hipError_t grow(size_t bytes)
     {
@@ -133,12 +156,26 @@ StagePtr acquire_stage(size_t bytes, hipError_t *err)
         s.reset(new HostStage);
         s->device = device;
     }
-    if ((*err = s->need(0)) != hipSuccess || (*err = s->grow(bytes)) != hipSuccess) return nullptr;
-    return s;
+    *err = s->grow(bytes);
+    if (*err == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        drop_idle_stages();
+        *err = s->grow(bytes);
+    }
+    if (*err == hipSuccess) *err = s->need(0, std::min(kChunk, std::max(bytes, kLeastChunk)));
+    return *err == hipSuccess ? std::move(s) : nullptr;
 }
 
 hipStream_t stage_stream(const HostStage &s) { return s.stream[0]; }
 char *stage_device(const HostStage &s) { return s.dev; }
+
+void trim_idle_stages()
+{
+    Pool &p = pool();
+    std::lock_guard<std::mutex> lk(p.mu);
+    for (HostStage *s : p.idle)
+        if (s && s->dev_bytes > kKeepIdle) s->drop_device();
+}
 
 void drop_idle_stages()
 {
@@ -199,9 +236,9 @@ void move_range(const std::vector<HostPiece> &pieces, size_t lo, size_t hi, char
 hipError_t copy_in(HostStage &s, const std::vector<HostPiece> &pieces)
 {
     if (pieces.empty()) return hipSuccess;
-    const size_t end = pieces.back().offset + pieces.back().bytes;
-    for (size_t lo = pieces.front().offset; lo < end; lo += kChunk) {
-        const size_t hi = std::min(end, lo + kChunk);
+    const size_t end = pieces.back().offset + pieces.back().bytes, chunk = s.pin_bytes[0];
+    for (size_t lo = pieces.front().offset; lo < end; lo += chunk) {
+        const size_t hi = std::min(end, lo + chunk);
         move_range<true>(pieces, lo, hi, s.pin[0]);
         hipError_t e = hipMemcpyAsync(s.dev + lo, s.pin[0], hi - lo, hipMemcpyHostToDevice,
                                       s.stream[0]);
@@ -217,9 +254,19 @@ hipError_t copy_out(HostStage &s, const std::vector<HostPiece> &pieces)
     if (pieces.empty()) return hipStreamSynchronize(s.stream[0]);
     const size_t begin = pieces.front().offset;
     const size_t bytes = pieces.back().offset + pieces.back().bytes - begin;
-    const int threads = copy_threads(bytes);
+    // as many workers as the bytes are worth, of new ones fewer
+    int threads = copy_threads(bytes);
+    threads = std::min(threads, std::max(s.made(), 1 + (int)std::min<size_t>(
+                                                           kWorkers, bytes / kPerNewWorker)));
     // few bytes: one chunk for each thread
-    const size_t step = std::min(kChunk, (bytes / (size_t)threads + 4096) & ~size_t(4095));
+    const size_t step =
+        std::min({kChunk, s.pin_bytes[0], (bytes / (size_t)threads + 4096) & ~size_t(4095)});
+    // (without memory for a worker, those there do the work)
+    for (int w = 1; w < threads; w++)
+        if (s.need(w, step) != hipSuccess) {
+            (void)hipGetLastError();
+            threads = w;
+        }
     auto chunk = [&](int64_t c, int w) {
         const size_t lo = begin + (size_t)c * step, hi = std::min(begin + bytes, lo + step);
         hipError_t e = hipMemcpyAsync(s.pin[w], s.dev + lo, hi - lo, hipMemcpyDeviceToHost,
@@ -235,10 +282,6 @@ hipError_t copy_out(HostStage &s, const std::vector<HostPiece> &pieces)
             if (e != hipSuccess) return e;
         }
         return hipSuccess;
-    }
-    for (int w = 1; w < threads; w++) {
-        const hipError_t e = s.need(w);
-        if (e != hipSuccess) return e;
     }
     hipError_t e0 = hipStreamSynchronize(s.stream[0]);
     if (e0 != hipSuccess) return e0;

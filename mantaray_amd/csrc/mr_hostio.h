@@ -48,7 +48,11 @@ struct HostPiece {
 hipError_t copy_in(HostStage &s, const std::vector<HostPiece> &pieces);
 hipError_t copy_out(HostStage &s, const std::vector<HostPiece> &pieces);
 
-// Frees every stage not in use (the last field handle of the process died).
+// Frees the larger device buffers of the stages not in use (the last field
+// handle of the process died).
+void trim_idle_stages();
+
+// Frees every stage not in use.
 void drop_idle_stages();
 
 }  // namespace mr

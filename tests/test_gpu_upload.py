@@ -140,13 +140,15 @@ for pair in PAIRS:
     assert refused.value == 0
     limit.value = own - 1000
     b, c = _fields(pair, N)
+    before = 0
     for step in ("trace", "again", "uploaded"):
         got = mr.trace_many(b, c, *rays, 0.0, 14.0, 0.7)
         for k, v in want.items():
             assert np.array_equal(got[k], v, equal_nan=True), (pair, step, k)
-        # one refusal a trace on new fields, none on the same ones again, one
-        # an upload
-        assert refused.value == (1 if step == "trace" else 1 if step == "again" else 2), step
+        # asked for by a trace on new fields, not by one on the same fields
+        # again, and by an upload
+        asked, before = refused.value > before, refused.value
+        assert asked == (step != "again"), step
         if step == "again":
             b.upload()
             c.upload()
@@ -155,7 +157,7 @@ for pair in PAIRS:
     c.upload()
     limit.value = own - 1000
     got = mr.trace_many(b, c, *rays, 0.0, 14.0, 0.7)
-    assert refused.value == 2
+    assert refused.value == before
     assert np.array_equal(got["x"], want["x"], equal_nan=True)
     limit.value = 0
     refused.value = 0
