@@ -34,13 +34,23 @@ namespace {
 
 // A pinned chunk: 75 us on the bus, long against a wait's overhead.  A thread
 // is worth starting for each megabyte (about 100 us of copying into fresh
-// pages, against 15 us to start it), a worker's stream and chunk worth making
-// for each kPerNewWorker.
+// pages, against 15 us to start it).  A chunk takes 50 us to make, but each of
+// a process's first four streams 3 ms.  So a stage has one stream, which all
+// workers share, until a later call copies kManyStreams or more; then kStreams,
+// with which 8191 rays (262 MB) below take 9.9 ms, with one 10.9 (of 64 MB 6.2 and 6.3).  First
+// and later calls of ray_tracing on NetCDF paths in a process, 1000 steps:
+//                      500 rays       2000 rays      8191 rays
+//   plain copies       20 / 11.5      30 / 20.8      77 / 61   ms
+//   a stream a worker  31 /  4.8      34 /  6.2      41 / 10.0
+//   one stream first   16 /  4.9      20 /  6.6      24 / 10.4
+// (A process's very first call still waits for that one stream: one ray 13.0
+// ms against 11.9.)
 constexpr size_t kChunk = size_t(4) << 20;
 constexpr size_t kLeastChunk = size_t(64) << 10;
 constexpr size_t kPerThread = size_t(1) << 20;
-constexpr size_t kPerNewWorker = size_t(4) << 20;
+constexpr size_t kManyStreams = size_t(128) << 20;
 constexpr int kWorkers = 12;
+constexpr int kStreams = 4;
 constexpr size_t kIdleStages = 2;
 constexpr size_t kKeepDevice = size_t(512) << 20;
 constexpr size_t kKeepIdle = size_t(16) << 20;
@@ -49,34 +59,35 @@ constexpr size_t kKeepIdle = size_t(16) << 20;
 
 struct HostStage {
     int device = 0;
-    hipStream_t stream[kWorkers] = {};
+    hipStream_t stream[kStreams] = {};
+    int streams = 0;                   // those made
+    bool used = false;                 // by a call before this one
     char *pin[kWorkers] = {};
     size_t pin_bytes[kWorkers] = {};
     char *dev = nullptr;
     size_t dev_bytes = 0;
 
-    // the stream of worker w and a pinned chunk of at least `bytes` (up to
-    // kChunk), made on first use; worker w's chunk is not in use
-    hipError_t need(int w, size_t bytes)
+    hipError_t need_streams(int n)
     {
         hipError_t e = hipSuccess;
-        if (!stream[w]) e = hipStreamCreateWithFlags(&stream[w], hipStreamNonBlocking);
-        if (e != hipSuccess || pin_bytes[w] >= bytes) return e;
+        for (; e == hipSuccess && streams < n; streams += e == hipSuccess)
+            e = hipStreamCreateWithFlags(&stream[streams], hipStreamNonBlocking);
+        return e;
+    }
+    // a pinned chunk of at least `bytes` (up to kChunk) for worker w, whose
+    // chunk is not in use
+    hipError_t need_chunk(int w, size_t bytes)
+    {
+        if (pin_bytes[w] >= bytes) return hipSuccess;
         size_t n = kLeastChunk;
         while (n < bytes) n *= 2;
         if (pin[w]) (void)hipHostFree(pin[w]);
         pin_bytes[w] = 0;
-        e = hipHostMalloc(reinterpret_cast<void **>(&pin[w]), n, hipHostMallocDefault);
+        const hipError_t e =
+            hipHostMalloc(reinterpret_cast<void **>(&pin[w]), n, hipHostMallocDefault);
         if (e != hipSuccess) pin[w] = nullptr;
         else pin_bytes[w] = n;
         return e;
-    }
-    // workers whose stream and chunk are there
-    int made() const
-    {
-        int w = 0;
-        while (w < kWorkers && pin_bytes[w]) w++;
-        return w;
     }
     hipError_t grow(size_t bytes)
     {
@@ -99,10 +110,9 @@ struct HostStage {
         const bool sw = hipGetDevice(&prev) == hipSuccess && prev != device &&
                         hipSetDevice(device) == hipSuccess;
         drop_device();
-        for (int w = 0; w < kWorkers; w++) {
-            if (stream[w]) (void)hipStreamDestroy(stream[w]);
-            if (pin[w]) (void)hipHostFree(pin[w]);
-        }
+        for (int k = 0; k < streams; k++) (void)hipStreamDestroy(stream[k]);
+        for (char *p : pin)
+            if (p) (void)hipHostFree(p);
         if (sw) (void)hipSetDevice(prev);
     }
 };
@@ -126,6 +136,7 @@ void StageReturn::operator()(HostStage *s) const
 {
     if (!s) return;
     if (s->dev_bytes > kKeepDevice) s->drop_device();
+    s->used = true;
     {
         Pool &p = pool();
         std::lock_guard<std::mutex> lk(p.mu);
@@ -162,7 +173,8 @@ StagePtr acquire_stage(size_t bytes, hipError_t *err)
         drop_idle_stages();
         *err = s->grow(bytes);
     }
-    if (*err == hipSuccess) *err = s->need(0, std::min(kChunk, std::max(bytes, kLeastChunk)));
+    if (*err == hipSuccess) *err = s->need_streams(1);
+    if (*err == hipSuccess) *err = s->need_chunk(0, std::min(kChunk, std::max(bytes, kLeastChunk)));
     return *err == hipSuccess ? std::move(s) : nullptr;
 }
 
@@ -254,24 +266,24 @@ hipError_t copy_out(HostStage &s, const std::vector<HostPiece> &pieces)
     if (pieces.empty()) return hipStreamSynchronize(s.stream[0]);
     const size_t begin = pieces.front().offset;
     const size_t bytes = pieces.back().offset + pieces.back().bytes - begin;
-    // as many workers as the bytes are worth, of new ones fewer
     int threads = copy_threads(bytes);
-    threads = std::min(threads, std::max(s.made(), 1 + (int)std::min<size_t>(
-                                                           kWorkers, bytes / kPerNewWorker)));
     // few bytes: one chunk for each thread
     const size_t step =
         std::min({kChunk, s.pin_bytes[0], (bytes / (size_t)threads + 4096) & ~size_t(4095)});
-    // (without memory for a worker, those there do the work)
+    // (without memory for a worker's chunk, or streams for them, the copy does
+    // with what is there)
     for (int w = 1; w < threads; w++)
-        if (s.need(w, step) != hipSuccess) {
+        if (s.need_chunk(w, step) != hipSuccess) {
             (void)hipGetLastError();
             threads = w;
         }
+    if (s.used && bytes >= kManyStreams && s.need_streams(std::min(threads, kStreams)) != hipSuccess)
+        (void)hipGetLastError();
     auto chunk = [&](int64_t c, int w) {
         const size_t lo = begin + (size_t)c * step, hi = std::min(begin + bytes, lo + step);
-        hipError_t e = hipMemcpyAsync(s.pin[w], s.dev + lo, hi - lo, hipMemcpyDeviceToHost,
-                                      s.stream[w]);
-        if (e == hipSuccess) e = hipStreamSynchronize(s.stream[w]);
+        const hipStream_t stream = s.stream[w % s.streams];
+        hipError_t e = hipMemcpyAsync(s.pin[w], s.dev + lo, hi - lo, hipMemcpyDeviceToHost, stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(stream);
         if (e == hipSuccess) move_range<false>(pieces, lo, hi, s.pin[w]);
         return e;
     };
