@@ -277,24 +277,23 @@ __device__ __forceinline__ float index32(float t, double inv_sp)
 // f64 fractional index RN64(t / sp) (cartesian_current.rs:244), reduced to
 // what the cell choice needs: the bound checks and floor.  The product with
 // the rounded reciprocal is within 2^-50 (relative) of the quotient; only
-// when it lies that close to an integer is the exact division taken.  A
-// negative quotient of up to 2^-1075, half the least number, rounds to -0 and
-// is on the grid (both sides of that test are scaled by 2^600, to compare
-// without subnormal numbers).  ok is cleared where the reference returns Err
-// (a NaN index errs later, in bilinear, because all four corners collapse
-// onto (0, 0)).  The returned floor is meaningful only when ok is set.
+// when it lies that close to an integer is the exact division taken, zero
+// among them: a negative quotient may underflow to -0, which is on the grid.
+// ok is cleared where the reference returns Err (a NaN index errs later, in
+// bilinear, because all four corners collapse onto (0, 0)).  The returned
+// floor is meaningful only when ok is set.
 __device__ __forceinline__ double index64(double p, double a0, double sp, double inv_sp,
                                           double nm1, bool &ok)
 {
     const double t = p - a0;
     double q = t * inv_sp;
     double fl = __builtin_floor(q);
-    if (__builtin_fabs((q - fl) - 0.5) > 0.5 - q * 0x1p-50) {   // near an integer
+    if (__builtin_fabs((q - fl) - 0.5) >= 0.5 - q * 0x1p-50) {  // near an integer
         q = t / sp;
         fl = __builtin_floor(q);
     }
-    ok = ok & (t * 0x1p600 >= sp * -0x1p-475) & (q <= nm1);
-    return __builtin_fmax(fl, 0.0);
+    ok = ok & (q >= 0.0) & (q <= nm1);
+    return fl;
 }
 
 // Wait for every outstanding vector memory operation (s_waitcnt vmcnt(0),
