@@ -727,40 +727,34 @@ __global__ void __launch_bounds__(64) adjoint_flat_kernel(AdjointArgs a)
 // The reverse sweep with the linearisations on waves of their own.  A
 // step's four stage linearisations (field queries, dispersion terms, the
 // matrix of rhs64_lin) do not depend on the cotangent chain, only their
-// application does.  A workgroup is 2 + NL waves over the same 64 rays, in
+// application does.  A workgroup is four waves over the same 64 rays, in
 // rounds separated by a barrier:
 //   wave 0          recomputes one step of segment c-1 (as in adjoint_kernel);
-//   waves 1 .. NL   linearise one step of segment c, 4/NL stages each
+//   waves 1, 2      linearise one step of segment c, two stages each
 //                   (latest first), in reverse step order, into a
 //                   double-buffered LDS ring; each loads the next round's
 //                   step from the work buffer while it works on this one;
-//   wave NL + 1     applies the records of the step linearised the round
+//   wave 3          applies the records of the step linearised the round
 //                   before (the chain of rk4_step_adjoint), adds the row
 //                   cotangents and sums the grid cotangents.
 // Segment c's K steps take K rounds; segment cmax is recomputed alone first
 // and the chain trails by one round: (cmax + 2) K + 1 rounds in all.  A
-// round costs about 4/NL stage linearisations, against eight in the
+// round costs about two stage linearisations, against eight in the
 // two-wave sweep.  Meant for launches of a workgroup or two per CU, where
-// the sweep is latency-bound (the LDS ring holds one workgroup per CU).  NL
-// = 2 is the one launched: with NL = 4 the six waves share SIMDs and the
-// 256 registers a wave then gets spill.
-// Whether linearising wave W (NL = 2: 1 or 2; 0: every wave otherwise)
-// uses field f of a step's data in the work buffer: f in [0, 4) is the
-// state y, [4, 8), [8, 12) and [12, 16) the stage states of stages 1, 2, 3
-// (wave 1 evaluates stages 2 and 1 and guesses its next cell from y's
-// position; wave 2 evaluates stages 3 and 0).
+// the sweep is latency-bound (the LDS ring holds one workgroup per CU).
+// Whether linearising wave W (1 or 2) uses field f of a step's data in the
+// work buffer: f in [0, 4) is the state y, [4, 8), [8, 12) and [12, 16) the
+// stage states of stages 1, 2, 3 (wave 1 evaluates stages 2 and 1 and guesses
+// its next cell from y's position; wave 2 evaluates stages 3 and 0).
 template <int W>
 __device__ constexpr bool lin_uses(int f)
 {
-    if (W == 1) return f < 2 || (f >= 4 && f < 12);
-    if (W == 2) return f < 4 || f >= 12;
-    return true;
+    return W == 1 ? f < 2 || (f >= 4 && f < 12) : f < 4 || f >= 12;
 }
 
-template <int BK, int CK, bool SH, int MATH, int NL>
-__global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs a)
+template <int BK, int CK, bool SH, int MATH>
+__global__ void __launch_bounds__(4 * 64) adjoint_lin_kernel(AdjointArgs a)
 {
-    constexpr int SPW = 4 / NL;                        // stages per linearising wave
     __shared__ double ring[2][4][LIN_N][64];
     const int64_t nr = a.n_rays;
     const int wave = (int)(threadIdx.x >> 6);
@@ -781,7 +775,6 @@ __global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs 
     const int cmax_r = (active && m >= 1) ? (int)((m - 1) / stride) : -1;
     const int cmax = wave_max(cmax_r);
     const int rounds = cmax >= 0 ? (cmax + 2) * stride + 1 : 0;
-    const int chain = NL + 1;
     // Each role runs a loop of its own, with the same rounds and one barrier
     // per round: the state of one role is then not live across another's
     // code, and registers go to the largest role, not to all of them.
@@ -809,10 +802,9 @@ __global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs 
             }
             __syncthreads();
         }
-    } else if (wave < chain) {
-        // W: the linearising wave with NL = 2 (1 or 2), as a compile-time
-        // value, so that each loads and keeps only the step data its stages
-        // use; 0 for the general case
+    } else if (wave < 3) {
+        // W: the linearising wave, as a compile-time value, so that each loads
+        // and keeps only the step data its stages use
         auto lin_role = [&](auto wc) {
             constexpr int W = decltype(wc)::value;
             Slots64<BK, CK, SH> sn;
@@ -856,90 +848,48 @@ __global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs 
                     const double bx = W == 2 ? 0.0 : 2.0 * (d[0] - P[1][0]);
                     const double by = W == 2 ? 0.0 : 2.0 * (d[1] - P[1][1]);
                     Slots64<BK, CK, SH> sq = sn;
-                    if (NL == 2) {
-                        // the cells of this wave's next point, into sn (see below)
-                        if constexpr (W == 1)
-                            prefetch64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, sn, P[1][0] + bx,
+                    // the cells of this wave's next point, into sn (see below)
+                    if constexpr (W == 1)
+                        prefetch64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, sn, P[1][0] + bx,
                                                P[1][1] + by);
-                        else
-                            prefetch64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, sn, P[0][0], P[0][1]);
-                    }
+                    else
+                        prefetch64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, sn, P[0][0], P[0][1]);
                     // start loading the next round's step (same segment)
                     pre = j >= 1;
                     if (pre) {
                         work_get(wb, ld, r, j - 1, nxt, [](int f) { return lin_uses<W>(f); });
                     }
-                    if (NL == 2) {
-                        // The stage points pair up: stages 2 and 1 lie together near
-                        // y + k dt/2, and stage 0 here lies with stage 3 of the next
-                        // round (one step earlier).  Wave 1 takes stages 2 and 1,
-                        // wave 2 stages 3 and 0, so each needs one prefetch per
-                        // round: wave 1 for the next round's midpoint (guessed one
-                        // step back along k1), wave 2 for stage 0 (known), which
-                        // it evaluates in the prefetched slot (the lanes that did
-                        // not prefetch hold the same cells in both).
-                        double R[LIN_N];
-                        if constexpr (W == 1) {
-                            rhs64_lin<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, K, P[2][0], P[2][1],
-                                              P[2][2], P[2][3], R);
+                    // The stage points pair up: stages 2 and 1 lie together near
+                    // y + k dt/2, and stage 0 here lies with stage 3 of the next
+                    // round (one step earlier).  Wave 1 takes stages 2 and 1,
+                    // wave 2 stages 3 and 0, so each needs one prefetch per
+                    // round: wave 1 for the next round's midpoint (guessed one
+                    // step back along k1), wave 2 for stage 0 (known), which
+                    // it evaluates in the prefetched slot (the lanes that did
+                    // not prefetch hold the same cells in both).
+                    double R[LIN_N];
+                    if constexpr (W == 1) {
+                        rhs64_lin<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, K, P[2][0], P[2][1],
+                                          P[2][2], P[2][3], R);
 #pragma unroll
-                            for (int f = 0; f < LIN_N; ++f)
-                                if (lin_field_used<BK, CK, SH>(f)) ring[rho & 1][2][f][lane] = R[f];
-                            rhs64_lin<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, K, P[1][0], P[1][1],
-                                              P[1][2], P[1][3], R);
+                        for (int f = 0; f < LIN_N; ++f)
+                            if (lin_field_used<BK, CK, SH>(f)) ring[rho & 1][2][f][lane] = R[f];
+                        rhs64_lin<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, K, P[1][0], P[1][1],
+                                          P[1][2], P[1][3], R);
 #pragma unroll
-                            for (int f = 0; f < LIN_N; ++f)
-                                if (lin_field_used<BK, CK, SH>(f)) ring[rho & 1][1][f][lane] = R[f];
-                        } else {
-                            rhs64_lin<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, K, P[3][0], P[3][1],
-                                              P[3][2], P[3][3], R);
-#pragma unroll
-                            for (int f = 0; f < LIN_N; ++f)
-                                if (lin_field_used<BK, CK, SH>(f)) ring[rho & 1][3][f][lane] = R[f];
-                            rhs64_lin<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sn, K, P[0][0], P[0][1],
-                                              P[0][2], P[0][3], R);
-#pragma unroll
-                            for (int f = 0; f < LIN_N; ++f)
-                                if (lin_field_used<BK, CK, SH>(f)) ring[rho & 1][0][f][lane] = R[f];
-                        }
+                        for (int f = 0; f < LIN_N; ++f)
+                            if (lin_field_used<BK, CK, SH>(f)) ring[rho & 1][1][f][lane] = R[f];
                     } else {
-                        // this wave's stages, latest first (the wave selects values,
-                        // the indices stay compile-time)
-                        const int first = 3 - (wave - 1) * SPW;
+                        rhs64_lin<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, K, P[3][0], P[3][1],
+                                          P[3][2], P[3][3], R);
 #pragma unroll
-                        for (int h = 0; h < SPW; ++h) {
-                            const int st = first - h;
-                            double Y[4];
+                        for (int f = 0; f < LIN_N; ++f)
+                            if (lin_field_used<BK, CK, SH>(f)) ring[rho & 1][3][f][lane] = R[f];
+                        rhs64_lin<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sn, K, P[0][0], P[0][1],
+                                          P[0][2], P[0][3], R);
 #pragma unroll
-                            for (int q = 0; q < 4; ++q)
-                                Y[q] = st == 3   ? P[3][q]
-                                       : st == 2 ? P[2][q]
-                                       : st == 1 ? P[1][q]
-                                                 : P[0][q];
-                            Slots64<BK, CK, SH> sq = sn;
-                            // the next point: this wave's next stage, or, after its
-                            // last, its first stage one step earlier (guessed one
-                            // step back along k1)
-                            double gx, gy;
-                            if (h + 1 < SPW) {
-                                const int sx_ = st - 1;
-                                gx = sx_ == 2 ? P[2][0] : sx_ == 1 ? P[1][0] : P[0][0];
-                                gy = sx_ == 2 ? P[2][1] : sx_ == 1 ? P[1][1] : P[0][1];
-                            } else {
-                                const double fx = first == 3 ? P[3][0] : first == 2 ? P[2][0]
-                                                : first == 1 ? P[1][0] : P[0][0];
-                                const double fy = first == 3 ? P[3][1] : first == 2 ? P[2][1]
-                                                : first == 1 ? P[1][1] : P[0][1];
-                                gx = fx + bx;
-                                gy = fy + by;
-                            }
-                            prefetch64<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, sn, gx, gy);
-                            double R[LIN_N];
-                            rhs64_lin<BK, CK, SH>(B, a.bp, C, a.cp, a.f, sq, K, Y[0], Y[1], Y[2], Y[3], R);
-#pragma unroll
-                            for (int f = 0; f < LIN_N; ++f)
-                                if (lin_field_used<BK, CK, SH>(f)) ring[rho & 1][st][f][lane] = R[f];
-                        }
+                        for (int f = 0; f < LIN_N; ++f)
+                            if (lin_field_used<BK, CK, SH>(f)) ring[rho & 1][0][f][lane] = R[f];
                     }
                 } else {
                     pre = false;
@@ -947,9 +897,8 @@ __global__ void __launch_bounds__(64 * (NL + 2)) adjoint_lin_kernel(AdjointArgs 
                 __syncthreads();
             }
         };
-        if (NL == 2 && wave == 1) lin_role(std::integral_constant<int, 1>{});
-        else if (NL == 2) lin_role(std::integral_constant<int, 2>{});
-        else lin_role(std::integral_constant<int, 0>{});
+        if (wave == 1) lin_role(std::integral_constant<int, 1>{});
+        else lin_role(std::integral_constant<int, 2>{});
     } else {
         double lam[4] = {0.0, 0.0, 0.0, 0.0};          // the cotangent
         Sums64<BK, CK, SH, NoQueue> sums(nullptr);
@@ -1096,7 +1045,7 @@ hipError_t launch_adjoint(const AdjointArgs &a, int bk, int ck, int math, int wa
         using KK = decltype(k);
         constexpr bool SH = decltype(sh)::value;
         if (waves == 4)
-            hipLaunchKernelGGL((adjoint_lin_kernel<KK::bk, KK::ck, SH, KK::math, 2>), grid,
+            hipLaunchKernelGGL((adjoint_lin_kernel<KK::bk, KK::ck, SH, KK::math>), grid,
                                dim3(4 * 64), 0, stream, a);
         else if (waves == 2)
             hipLaunchKernelGGL((adjoint_kernel<KK::bk, KK::ck, SH, KK::math>), grid,

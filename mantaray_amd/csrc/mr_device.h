@@ -33,8 +33,6 @@ namespace mr {
 
 #define MR_NANF_INIT __builtin_nanf("")
 #define MR_NAN_INIT __builtin_nan("")
-// a double whose two f32 halves are both -inf
-#define MR_EMPTY_REGION __builtin_bit_cast(double, 0xFF800000FF800000ull)
 
 constexpr double G = 9.8;                        // src/wave_ray_path.rs:23
 
@@ -505,15 +503,6 @@ __device__ __forceinline__ bool current_query(const CurrentView &C, const Curren
 
 // ---------------------------------------------------------------------------
 // f64 helpers for the fast dispersion evaluation
-
-// 1/x: hardware reciprocal estimate (about 5e-8 relative) refined by one
-// Newton step (about 2e-15).
-__device__ __forceinline__ double rcp_nr(double x)
-{
-    const double r = __builtin_amdgcn_rcp(x);
-    const double e = __builtin_fma(-x, r, 1.0);
-    return __builtin_fma(r, e, r);
-}
 
 // 1/sqrt(x): hardware estimate (about 5e-8 relative) refined by one Newton
 // step (about 4e-15).
