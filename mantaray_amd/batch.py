@@ -5,8 +5,10 @@
     b.run()                      # enqueued on torch's current stream
     res = b.results()            # per scene: {"len": (n,), "end": (n, 4)}
 
-record_tile (keyword of Batch) sets the record tile shape of the gridded
-fields; autotune() picks the launch shape and then the tile shape.  Each
+record_tile (keyword of Batch) sets the tile shape of the gridded fields'
+plain records, which matters only to a batch that runs on them (a field
+without cell records of its own); autotune() picks the launch shape and then
+the tile shape.  Each
 scene has its own fields, step, step count and rays; every ray's row
 count and last row are what trace_many gives for its scene.  The launch takes
 rays from one queue, so lanes freed by rays that end early (edge exits,
@@ -59,7 +61,7 @@ class Batch:
         return self.device.index if self.device.index is not None else -1
 
     def _create(self, record_tile: int):
-        """A batch handle over the same scenes with cell records in tiles of
+        """A batch handle over the same scenes with plain records in tiles of
         2^record_tile cells a side (-1 = 8 x 8)."""
         o = C.options(math=self._math, solout=self._solout, memory=C.MR_MEM_DEVICE,
                       device=self._dev_index(), record_tile=record_tile)
@@ -90,9 +92,11 @@ class Batch:
     def autotune(self, key: str, force: bool = False, tuner=None, tiles=(2, 3, 4, 5)):
         """Pick block size and workgroups per CU for this batch by timing the
         candidates (mantaray_amd.autotune), then, with that launch shape, the
-        record tile shape among `tiles` (log2 of the tile edge); later run()
-        calls use the choice.  Returns (launch shape, its search table, tile
-        search table)."""
+        record tile shape among `tiles` (log2 of the tile edge; tiles=() leaves
+        that search out: on cell records all shapes run alike, and the fields
+        keep the plain records of each shape until they are freed); later
+        run() calls use the choice.  Returns (launch shape, its search table,
+        tile search table)."""
         from .autotune import Autotuner
         tuner = tuner or Autotuner()
         cands = [{"block_size": b, "blocks_per_cu": p}
