@@ -1114,18 +1114,27 @@ int adjoint_run(const mr_field *bathy, const mr_field *current, const double *de
     // current, whose evaluations are short, up to one, and two waves
     // (recompute | sweep) from there to two; one beyond (each wave recomputes
     // and sweeps in turn, the least SIMD time once the launch fills the GPU).
+    // Over a flat depth two waves also serve from one to 4/3 per CU, where few
+    // workgroups would wait for a pass of four of their own.
     // block_size 64, 128 or 256 forces one, two or four.  1000 steps (one /
     // two / four waves, ms), current alone, both gridded on shared axes, on
     // axes of their own, depth alone:
-    //   16,384 rays  3.94/2.50/1.45  4.81/3.60/1.88  6.08/4.36/2.10  3.18/2.22/1.43
-    //   24,576       4.10/2.98/2.83  4.99/3.80/3.62  6.31/4.57/4.17  3.30/2.64/2.88
-    //   32,768       4.11/3.07/2.99  5.03/3.89/3.66  6.36/4.63/4.16  3.34/2.71/2.94
-    //   36,864                       5.04/7.44/5.47  6.34/8.99/6.32  3.33/4.94/4.33
-    //   65,536       4.15/6.16/5.86  6.01/7.76/7.22
+    //   16,384 rays  3.95/2.49/1.48  4.78/3.59/1.86  6.08/4.36/2.10  3.18/2.22/1.43
+    //   16,448       4.09/2.55/2.76  4.94/3.60/3.60
+    //   20,480       4.11/2.66/2.80  4.98/3.69/3.65
+    //   22,528         - /2.88/2.84
+    //   24,576       4.11/2.96/2.84  4.99/3.79/3.64  6.31/4.57/4.17  3.30/2.64/2.88
+    //   32,768       4.12/3.04/2.95  5.02/3.88/3.66  6.36/4.63/4.16  3.34/2.71/2.94
+    //   36,864       4.14/5.61/4.26  5.03/7.48/5.46  6.34/8.99/6.32  3.33/4.94/4.33
+    //   65,536       4.19/6.18/5.80  5.98/7.75/7.31
+    // (axes of their own, 600 x 500 cells: 16,448 rays two 4.84, four 4.58)
     const int cus = cu_count();
     const int64_t groups = (n_rays + 63) / 64;
-    const int64_t four = current->kind == MR_CURRENT_GRID ? 2 * (int64_t)cus : cus;
-    int waves = groups <= four ? 4 : groups <= 2 * (int64_t)cus ? 2 : 1;
+    const bool grid_c = current->kind == MR_CURRENT_GRID;
+    const bool flat = bathy->kind == MR_BATHY_CONSTANT || bathy->kind == MR_BATHY_ARRAY;
+    const int64_t four = grid_c ? 2 * (int64_t)cus : cus;
+    const bool few_over = flat && groups > cus && groups <= cus + cus / 3;
+    int waves = groups <= four && !few_over ? 4 : groups <= 2 * (int64_t)cus ? 2 : 1;
     if (o.block_size == 64 || o.block_size == 128 || o.block_size == 256)
         waves = o.block_size / 64;
     else if (o.block_size != 0)

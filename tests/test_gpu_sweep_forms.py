@@ -54,6 +54,17 @@ def test_one_wave_default(pair, n_rays):
     _agree(sweep(0), sweep(128))
 
 
+@pytest.mark.parametrize("pair", ["current", "both"])
+@pytest.mark.parametrize("n_rays", [16_385, 21_824, 21_825])
+def test_between_one_and_two_workgroups_a_cu(pair, n_rays):
+    """4/3 workgroups for each of 256 CUs are 341: 21,824 rays."""
+    sweep = _case(pair, n_rays, False)
+    got = sweep(0)
+    _agree(got, sweep(64))
+    _agree(got, sweep(128))
+    _agree(got, sweep(256))
+
+
 @pytest.mark.parametrize("n_rays", [1, 63, 65, 500])
 def test_flat_depth_literal_forward(n_rays):
     sweep = _case("current", n_rays, False, "literal")
