@@ -579,8 +579,9 @@ __global__ void __launch_bounds__(64) adjoint_seq_kernel(AdjointArgs a)
 // the queued sums, on a 2048 x 2048 current, forward and sweep 89.6 -> 64.7
 // ms (the forward is 13.5 of them); the queue alone, before its pairs shared
 // requests and with the stored stage points, cost 2 ms.  What is left is the
-// issue of about 1380 vector instructions a step (66.2 ms with the stage
-// derivatives bitwise the forward's, rhs64_with_lin).
+// issue of 1,320 vector instructions a step by the counters, the
+// recomputation's among them (64.3 to 66.2 ms with the stage derivatives
+// bitwise the forward's, rhs64_with_lin, against 64.1 to 65.4).
 template <int BK, int CK, int MATH>
 __global__ void __launch_bounds__(64) adjoint_flat_kernel(AdjointArgs a)
 {

@@ -8,7 +8,8 @@ namespace mr {
 // Which cell records a trace or batch runs on: one combined record per cell
 // for a gridded depth and current on the same cells; each gridded field's
 // own (analytic fields have none); or none, for grids whose records the
-// kernels could not index with 32-bit byte offsets.  REC_OWN_MANY: the own
+// kernels could not index with 32-bit byte offsets and for fields that run on
+// their plain records (own_records in mr_capi.cpp).  REC_OWN_MANY: the own
 // records of two gridded fields in a launch with more waves than SIMDs.
 enum RecMode : int { REC_NONE = 0, REC_SHARED = 1, REC_OWN = 2, REC_OWN_MANY = 3 };
 

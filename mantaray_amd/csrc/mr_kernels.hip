@@ -25,7 +25,8 @@ namespace mr {
 // with the stop test of WaveRayPath::solout (wave_ray_path.rs:236-246).
 //
 // rk4_step runs on the plain records (BCell, CCell), for the grids whose
-// cell records rk4_step_rec cannot index (record_mode in mr_capi.cpp).
+// cell records rk4_step_rec cannot index and the fields it would serve worse
+// (record_mode and own_records in mr_capi.cpp).
 // Stages 1 and 3 start the loads of the plain records that the following
 // stages will most likely use (their points guessed from the latest
 // derivative) when those are not the cells already held, so a record is in
