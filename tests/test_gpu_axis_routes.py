@@ -173,3 +173,30 @@ def test_cell_lines(oracle_mod, a0, sp, n, grids, precision):
     assert np.isfinite(ref["kx"][1]).any()
     scale = np.nanmax(np.abs(ref["kx"])) + np.nanmax(np.abs(ref["ky"]))
     assert max(np.nanmax(np.abs(got[k] - ref[k])) for k in ("kx", "ky")) <= 1e-12 * scale
+
+
+@pytest.mark.parametrize("order", [("near", "1/160 of a cell"), ("1/160 of a cell", "near")])
+@pytest.mark.parametrize("pair", PAIRS)
+def test_batch_over_both_routes(pair, order):
+    """A batch runs on one kind of records: on the plain ones when any of its
+    scenes does, in whatever order they come.  The end states are those of a
+    trace of each scene, bitwise."""
+    import torch
+
+    import mantaray_amd as mr
+    from mantaray_amd.batch import Batch
+    scenes, want = [], []
+    for name in order:
+        off, sp, n, *_ = AXES[name]
+        b, c = _made(mr, mr, pair, off, sp, n)
+        s = _rays(off, sp, n, 150)
+        want.append(mr.trace_many(b, c, *s, 0.0, 11.0, 0.7, trajectories=False))
+        scenes.append({"bathymetry": b, "current": c, "t0": 0.0, "t_end": 11.0, "dt": 0.7,
+                       **dict(zip(("x0", "y0", "kx0", "ky0"), s))})
+    batch = Batch(scenes)
+    batch.run()
+    torch.cuda.synchronize()
+    for got, w in zip(batch.results(), want):
+        assert np.array_equal(got["len"].cpu().numpy(), w["len"])
+        assert np.array_equal(got["end"].cpu().numpy(), w["end"], equal_nan=True)
+    batch.close()
