@@ -161,7 +161,7 @@ int mr_field_copy_grid(const mr_field *f, double *x, double *y, double *a, doubl
 int mr_field_upload(const mr_field *f, int32_t device);
 
 /* Frees what host-memory traces keep for the next one and no call is using:
- * at most two sets of 4 streams, 48 MiB of pinned memory and 512 MiB of
+ * at most two sets of 12 streams, 48 MiB of pinned memory and 512 MiB of
  * device memory (16 MiB once no field handle lives). */
 int mr_release_host_buffers(void);
 

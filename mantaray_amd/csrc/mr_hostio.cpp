@@ -35,22 +35,21 @@ namespace {
 // A pinned chunk: 75 us on the bus, long against a wait's overhead.  A thread
 // is worth starting for each megabyte (about 100 us of copying into fresh
 // pages, against 15 us to start it).  A chunk takes 50 us to make, but each of
-// a process's first four streams 3 ms.  So a stage has one stream, which all
-// workers share, until a later call copies kManyStreams or more; then kStreams,
-// with which 8191 rays (262 MB) below take 9.9 ms, with one 10.9 (of 64 MB 6.2 and 6.3).  First
-// and later calls of ray_tracing on NetCDF paths in a process, 1000 steps:
-//                      500 rays       2000 rays      8191 rays
-//   plain copies       20 / 11.5      30 / 20.8      77 / 61   ms
-//   a stream a worker  31 /  4.8      34 /  6.2      41 / 10.0
-//   one stream first   16 /  4.9      20 /  6.6      24 / 10.4
-// (A process's very first call still waits for that one stream: one ray 13.0
-// ms against 11.9.)
+// a process's first four streams 3 ms.  So a stage has one stream, which its
+// workers share, and each later call that could use another makes one, up to a
+// stream a worker, with which copies of 6 to 130 MB take 5 to 9 % less of a
+// call than with one.  First and later calls of ray_tracing on NetCDF paths in
+// a process, 1000 steps:
+//                        500 rays     2000 rays    8191 rays
+//   plain copies         20 / 11.5    30 / 20.8    77 / 61   ms
+//   every stream at once 31 /  4.8    34 /  6.2    41 / 10.0
+//   a stream a call      17 /  4.9    23 /  7.2    25 / 11.2
+// (A process's very first call still waits for that one stream, one ray 13 to
+// 14 ms against 11.9, and the three after it for one each.)
 constexpr size_t kChunk = size_t(4) << 20;
 constexpr size_t kLeastChunk = size_t(64) << 10;
 constexpr size_t kPerThread = size_t(1) << 20;
-constexpr size_t kManyStreams = size_t(128) << 20;
 constexpr int kWorkers = 12;
-constexpr int kStreams = 4;
 constexpr size_t kIdleStages = 2;
 constexpr size_t kKeepDevice = size_t(512) << 20;
 constexpr size_t kKeepIdle = size_t(16) << 20;
@@ -59,7 +58,7 @@ constexpr size_t kKeepIdle = size_t(16) << 20;
 
 struct HostStage {
     int device = 0;
-    hipStream_t stream[kStreams] = {};
+    hipStream_t stream[kWorkers] = {};
     int streams = 0;                   // those made
     bool used = false;                 // by a call before this one
     char *pin[kWorkers] = {};
@@ -277,7 +276,7 @@ hipError_t copy_out(HostStage &s, const std::vector<HostPiece> &pieces)
             (void)hipGetLastError();
             threads = w;
         }
-    if (s.used && bytes >= kManyStreams && s.need_streams(std::min(threads, kStreams)) != hipSuccess)
+    if (s.used && s.need_streams(std::min(threads, s.streams + 1)) != hipSuccess)
         (void)hipGetLastError();
     auto chunk = [&](int64_t c, int w) {
         const size_t lo = begin + (size_t)c * step, hi = std::min(begin + bytes, lo + step);

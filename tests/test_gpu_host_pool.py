@@ -86,16 +86,22 @@ calls = [fan(100, 300), fan(700, 900), fan(3000, 1000)]
 first = [mr.core.ray_tracing(*c) for c in calls]
 made = n()
 assert var("largest", ctypes.c_size_t).value <= 4 << 20
-# (a process's first streams take 3 ms each: one is enough for these)
-assert made[0] == 1 and var("destroyed").value == 0
+# (a process's first streams take 3 ms each: no call makes more than one)
+assert 1 <= made[0] <= 4 and var("destroyed").value == 0
 again = [mr.core.ray_tracing(*c) for c in calls] + [mr.core.single_ray(*one)]
-assert n()[0] == 1 and var("destroyed").value == 0
+assert made[0] <= n()[0] <= made[0] + 4 and var("destroyed").value == 0
 for p, q in zip(first + [a], again):
     for k in ("time", "x", "y", "kx", "ky"):
         assert np.array_equal(p[k].values, q[k].values, equal_nan=True), k
+for _ in range(8):                     # up to a stream and a chunk a worker
+    again = [mr.core.ray_tracing(*c) for c in calls] + [mr.core.single_ray(*one)]
 made = n()
+assert made[0] <= 12
 for _ in range(3):
     again = [mr.core.ray_tracing(*c) for c in calls] + [mr.core.single_ray(*one)]
+    for p, q in zip(first + [a], again):
+        for k in ("time", "x", "y", "kx", "ky"):
+            assert np.array_equal(p[k].values, q[k].values, equal_nan=True), k
 assert n() == made, (n(), made)
 print("kept ok", flush=True)
 # all of it released
