@@ -35,17 +35,18 @@ namespace {
 // A pinned chunk: 75 us on the bus, long against a wait's overhead.  A thread
 // is worth starting for each megabyte (about 100 us of copying into fresh
 // pages, against 15 us to start it).  A chunk takes 50 us to make, but each of
-// a process's first four streams 3 ms.  So a stage has one stream, which its
-// workers share, and each later call that could use another makes one, up to a
-// stream a worker, with which copies of 6 to 130 MB take 5 to 9 % less of a
-// call than with one.  First and later calls of ray_tracing on NetCDF paths in
-// a process, 1000 steps:
-//                        500 rays     2000 rays    8191 rays
-//   plain copies         20 / 11.5    30 / 20.8    77 / 61   ms
-//   every stream at once 31 /  4.8    34 /  6.2    41 / 10.0
-//   a stream a call      17 /  4.9    23 /  7.2    25 / 11.2
+// a process's first four streams 3 ms.  So a stage's first call copies on one
+// stream, which its workers share, and the next one that has use for them makes
+// a stream for each worker: with one stream repeated calls of 6 to 130 MB took 5
+// to 9 % longer, with four those of 16 to 40 MB 5 %; made one a call, each
+// cost its call 2 to 9 ms.  Calls of ray_tracing on NetCDF paths in a process,
+// 1000 steps, the first / second / later ones (ms):
+//                        500 rays          2000 rays         8191 rays
+//   plain copies         20 / 11 / 11.5    30 / 22 / 20.8    77 / 64 / 61
+//   all streams at first 31 / -  /  4.8    34 / -  /  6.2    41 / -  / 10.0
+//   on the second call   17 / 19 /  4.6    20 / 19 /  6.3    23 / 25 /  9.8
 // (A process's very first call still waits for that one stream, one ray 13 to
-// 14 ms against 11.9, and the three after it for one each.)
+// 14 ms against 11.9.)
 constexpr size_t kChunk = size_t(4) << 20;
 constexpr size_t kLeastChunk = size_t(64) << 10;
 constexpr size_t kPerThread = size_t(1) << 20;
@@ -276,8 +277,7 @@ hipError_t copy_out(HostStage &s, const std::vector<HostPiece> &pieces)
             (void)hipGetLastError();
             threads = w;
         }
-    if (s.used && s.need_streams(std::min(threads, s.streams + 1)) != hipSuccess)
-        (void)hipGetLastError();
+    if (s.used && s.need_streams(threads) != hipSuccess) (void)hipGetLastError();
     auto chunk = [&](int64_t c, int w) {
         const size_t lo = begin + (size_t)c * step, hi = std::min(begin + bytes, lo + step);
         const hipStream_t stream = s.stream[w % s.streams];
